@@ -69,4 +69,30 @@ emfa_status gemm_launch_f32(hipStream_t s, const GemmArgs &g, int tag = 0);  // 
 emfa_status gemm_launch_f64(hipStream_t s, const GemmArgs &g, int tag = 0);  // TA=double, TC=double
 emfa_status gemm_launch_f32_f64(hipStream_t s, const GemmArgs &g);   // TA=float,  TC=double
 
+// Products with few columns (skinny.hip): C = beta C + sign A X, complex,
+// A M x K (row stride lda), X K x m (ldx), C M x m (ldc).
+template <typename TA, typename TC>
+struct SkinnyJob {
+    const cx<TA> *A = nullptr;
+    long long lda = 0;
+    const cx<TC> *X = nullptr;
+    long long ldx = 0;
+    cx<TC> *C = nullptr;
+    long long ldc = 0;
+    int M = 0, K = 0;
+    TC sign = 1;
+    int beta = 0;
+};
+// one product, or two of the same m in one launch
+emfa_status skinny_mm(hipStream_t s, const SkinnyJob<float, float> &j, int m,
+                      const SkinnyJob<float, float> *second = nullptr);
+emfa_status skinny_mm(hipStream_t s, const SkinnyJob<double, double> &j, int m,
+                      const SkinnyJob<double, double> *second = nullptr);
+// K in slices of kc: with P, plane z of P (M x m each) is A X over slice z
+// (C, sign and beta unused); without P one slice
+emfa_status skinny_mm_slices(hipStream_t s, const SkinnyJob<float, double> &j, int m, int slices, int kc,
+                             cx<double> *P);
+emfa_status skinny_mm_slices(hipStream_t s, const SkinnyJob<double, double> &j, int m, int slices, int kc,
+                             cx<double> *P);
+
 }  // namespace emfa

@@ -1510,188 +1510,13 @@ __global__ __launch_bounds__(256) void k_dinv_apply(const cx<R> *__restrict__ Di
     }
 }
 
-constexpr int kSkinnyMaxCols = 64;
-
-// Small products with at most 64 columns, the form every few-RHS solve step
-// and the refinement residual take:
-//   C (M x m) = beta C + sign A (M x K) X (K x m)      (P == null)
-//   plane z of P = A X over K slice [z kc, (z + 1) kc)  (P given)
-// The column tile MC (8, 16, 32, 64) follows m, so no lane works on padding
-// columns: lane tx owns column tx, rows ty + h RG (h < RPT) of the
-// workgroup's RPT RG rows (RG = 256 / MC).  Two rows per lane: more rows per
-// workgroup cut the re-reads of X but cost more in parallelism (measured:
-// eight rows per lane on tall 32 / 64-column products made a 7680-row solve
-// 2.5 -> 4.2 ms and the served stream 223 -> 187 solves/s).
-// K goes through LDS in chunks of 64 with the next chunk's operands loaded
-// into registers while the current chunk is multiplied.
-template <int MC>
-constexpr int smallmm_rpt() {
-    return 2;
-}
-
-template <int MC, int RPT = smallmm_rpt<MC>()>
-constexpr int smallmm_rb() {
-    return RPT * (256 / MC);
-}
-
-// row block bx, K slice z of C (+)= sign A X (see k_smallmm); LDS from the caller
-template <typename TA, typename TC, int MC, int RPT = smallmm_rpt<MC>()>
-__device__ __forceinline__ void smallmm_body(const cx<TA> *__restrict__ A, long long lda,
-                                             const cx<TC> *__restrict__ X, long long ldx, cx<TC> *C, long long ldc,
-                                             int M, int K, int m, int kc, TC sign, int beta, cx<TC> *__restrict__ P,
-                                             int bx, int z, cx<TA> (*As)[65], cx<TC> (*Xs)[MC]) {
-    constexpr int RG = 256 / MC, RB = RPT * RG, KC = 64;
-    constexpr int AL = RB * KC / 256, XL = KC * MC / 256;  // chunk elements per thread
-    const int tid = threadIdx.x, tx = tid % MC, ty = tid / MC;
-    const int rb = bx * RB;
-    const int kb = z * kc, ke = min(K, kb + kc);
-    cx<TA> ra[AL];
-    cx<TC> rx[XL];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < AL; ++i) {
-            const int e = tid + 256 * i, r = e / KC, k = e % KC;
-            ra[i] = (rb + r < M && k0 + k < ke) ? A[(size_t)(rb + r) * lda + k0 + k] : cx<TA>{TA(0), TA(0)};
-        }
-#pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int e = tid + 256 * i, k = e / MC, c = e % MC;
-            rx[i] = (k0 + k < ke && c < m) ? X[(size_t)(k0 + k) * ldx + c] : cx<TC>{TC(0), TC(0)};
-        }
-    };
-    cx<TC> acc[RPT];
-#pragma unroll
-    for (int h = 0; h < RPT; ++h) acc[h] = {TC(0), TC(0)};
-    if (kb < ke) gload(kb);
-    for (int k0 = kb; k0 < ke; k0 += KC) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < AL; ++i) {
-            const int e = tid + 256 * i;
-            As[e / KC][e % KC] = ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < XL; ++i) {
-            const int e = tid + 256 * i;
-            Xs[e / MC][e % MC] = rx[i];
-        }
-        __syncthreads();
-        if (k0 + KC < ke) gload(k0 + KC);
-#pragma unroll 8
-        for (int k = 0; k < KC; ++k) {
-            const cx<TC> x = Xs[k][tx];
-#pragma unroll
-            for (int h = 0; h < RPT; ++h) {
-                const cx<TA> a = As[ty + h * RG][k];
-                acc[h].re += (TC)a.re * x.re - (TC)a.im * x.im;
-                acc[h].im += (TC)a.re * x.im + (TC)a.im * x.re;
-            }
-        }
-    }
-    if (tx >= m) return;
-#pragma unroll
-    for (int h = 0; h < RPT; ++h) {
-        const int r = rb + ty + h * RG;
-        if (r >= M) continue;
-        const cx<TC> v = acc[h];
-        if (P) {
-            P[(size_t)z * M * m + (size_t)r * m + tx] = v;
-        } else {
-            cx<TC> c = beta ? C[(size_t)r * ldc + tx] : cx<TC>{TC(0), TC(0)};
-            c.re += sign * v.re;
-            c.im += sign * v.im;
-            C[(size_t)r * ldc + tx] = c;
-        }
-    }
-}
-
-template <typename TA, typename TC, int MC, int RPT>
-__global__ __launch_bounds__(256) void k_smallmm(const cx<TA> *__restrict__ A, long long lda,
-                                                 const cx<TC> *__restrict__ X, long long ldx, cx<TC> *C,
-                                                 long long ldc, int M, int K, int m, int kc, TC sign, int beta,
-                                                 cx<TC> *__restrict__ P) {
-    __shared__ cx<TA> As[smallmm_rb<MC, RPT>()][65];
-    __shared__ cx<TC> Xs[64][MC];
-    smallmm_body<TA, TC, MC, RPT>(A, lda, X, ldx, C, ldc, M, K, m, kc, sign, beta, P, blockIdx.x, blockIdx.y, As,
-                                  Xs);
-}
-
-// One step of a triangular solve through the diagonal-block inverses, in one
-// launch: workgroups [0, n0) form Y_b = D_b W_b on the block's rows (C0 =
-// D W, K = wb), the rest update the other rows with the same W_b through the
-// inverse-scaled off-diagonal block (C1 -= G W, G = L21 D_L^-1 or U12 D_U^-1
-// stored with the factor).  Both only read W_b and write disjoint rows.
-template <typename R, int MC>
-__global__ __launch_bounds__(256) void k_solve_step(const cx<R> *__restrict__ D, const cx<R> *__restrict__ G,
-                                                    long long ldg, const cx<R> *__restrict__ Wb, int m,
-                                                    cx<R> *__restrict__ Yb, cx<R> *__restrict__ C1, int wb, int M1,
-                                                    int n0) {
-    __shared__ cx<R> As[smallmm_rb<MC>()][65];
-    __shared__ cx<R> Xs[64][MC];
-    if ((int)blockIdx.x < n0)
-        smallmm_body<R, R, MC>(D, kDinvB, Wb, m, Yb, m, wb, wb, m, wb, R(1), 0, nullptr, blockIdx.x, 0, As, Xs);
-    else
-        smallmm_body<R, R, MC>(G, ldg, Wb, m, C1, m, M1, wb, m, wb, R(-1), 1, nullptr, blockIdx.x - n0, 0, As, Xs);
-}
-
-// launch k_smallmm with the column tile for m (<= 64); slices on gridDim.y.
-// rpt: rows per lane, 2 (short products: the most workgroups) or 8 (long-K
-// products such as the refinement residual: every workgroup reads its slice
-// of X, so fewer, taller workgroups read it fewer times; 32 / 64-column tiles)
-template <typename TA, typename TC>
-static emfa_status smallmm(hipStream_t s, const cx<TA> *A, long long lda, const cx<TC> *X, long long ldx, cx<TC> *C,
-                           long long ldc, int M, int K, int m, int slices, int kc, TC sign, int beta, cx<TC> *P,
-                           int rpt = 2) {
-    if (M <= 0 || m <= 0) return EMFA_OK;
-    EMFA_REQUIRE(m <= kSkinnyMaxCols && slices >= 1 && kc > 0, EMFA_E_INVALID, "smallmm: bad shape m=%d", m);
-    auto go = [&](auto mc) {
-        constexpr int MC = decltype(mc)::value;
-        if constexpr (MC >= 32) {
-            if (rpt == 8) {
-                constexpr int RB = smallmm_rb<MC, 8>();
-                const dim3 grid((M + RB - 1) / RB, slices);
-                k_smallmm<TA, TC, MC, 8><<<grid, 256, 0, s>>>(A, lda, X, ldx, C, ldc, M, K, m, kc, sign, beta, P);
-                return;
-            }
-        }
-        constexpr int RB = smallmm_rb<MC, 2>();
-        const dim3 grid((M + RB - 1) / RB, slices);
-        k_smallmm<TA, TC, MC, 2><<<grid, 256, 0, s>>>(A, lda, X, ldx, C, ldc, M, K, m, kc, sign, beta, P);
-    };
-    if (m <= 8)
-        go(std::integral_constant<int, 8>{});
-    else if (m <= 16)
-        go(std::integral_constant<int, 16>{});
-    else if (m <= 32)
-        go(std::integral_constant<int, 32>{});
-    else
-        go(std::integral_constant<int, 64>{});
-    EMFA_HIP_CHECK(hipGetLastError());
-    return EMFA_OK;
-}
-
-// one solve step (k_solve_step) with the column tile for m (<= 64)
-template <typename R>
-static emfa_status solve_step(hipStream_t s, const cx<R> *D, const cx<R> *G, long long ldg, const cx<R> *Wb, int m,
-                              cx<R> *Yb, cx<R> *C1, int wb, int M1) {
-    EMFA_REQUIRE(m >= 1 && m <= kSkinnyMaxCols && wb >= 1 && wb <= kDinvB && M1 >= 0, EMFA_E_INVALID,
-                 "solve step: bad shape m=%d wb=%d", m, wb);
-    auto go = [&](auto mc) {
-        constexpr int MC = decltype(mc)::value, RB = smallmm_rb<MC>();
-        const int n0 = (wb + RB - 1) / RB, n1 = (M1 + RB - 1) / RB;
-        k_solve_step<R, MC><<<n0 + n1, 256, 0, s>>>(D, G, ldg, Wb, m, Yb, C1, wb, M1, n0);
-    };
-    if (m <= 8)
-        go(std::integral_constant<int, 8>{});
-    else if (m <= 16)
-        go(std::integral_constant<int, 16>{});
-    else if (m <= 32)
-        go(std::integral_constant<int, 32>{});
-    else
-        go(std::integral_constant<int, 64>{});
-    EMFA_HIP_CHECK(hipGetLastError());
-    return EMFA_OK;
-}
+// Few right-hand sides: the steps of a solve and the refinement residual are
+// skinny products (skinny.hip) up to kSkinnyCols columns, on matrices of up to
+// kSkinnyMaxN unknowns also wider ones; else the expanded-operand MFMA GEMM.
+// Refined FP32 factorisations, ms with the GEMM / with the skinny products
+// above 64 columns: 1920 unknowns, 181 columns 4.99 / 4.28; 8321, 181 columns
+// 36.6 / 34.8; 14981, 100 columns 88.3 / 89.4; 30720, 181 columns 436 / 462.
+constexpr int kSkinnyCols = 64, kSkinnyMaxCols = 256, kSkinnyMaxN = 12288, kResidSkinnyCols = 128;
 
 // W = P B: row i of W is row perm[i] of B
 template <typename R>
@@ -2355,33 +2180,22 @@ static emfa_status solve_impl(emfa_ctx *ctx, const emfa_mat *LUm, const int *ipi
             EMFA_HIP_CHECK(hipGetLastError());
         }
         const dim3 g_apply(kDinvB / 32, (m + 31) / 32);
-        // k_smallmm up to 64 columns; above that the expanded-operand MFMA
-        // GEMM.  Contexts that share the device take the GEMM from 32
-        // columns: k_smallmm is VALU-bound there and the MFMA product needs
-        // about half the CU time (served 64-request stream: 193 -> 201
-        // solves/s, median of 14 passes), while a lone solve finishes sooner
-        // on k_smallmm's many small workgroups.
-        int skinny_max = ctx->cu_share > 0 ? 31 : kSkinnyMaxCols;
+        int skinny_max = N <= kSkinnyMaxN ? kSkinnyMaxCols : kSkinnyCols;
         if (const char *e = getenv("EMFA_SKINNY_MAX")) skinny_max = std::min(kSkinnyMaxCols, atoi(e));
         const bool skinny = m <= skinny_max;
         const char *apply_env = getenv("EMFA_APPLY_MFMA");  // 0: k_dinv_apply for every width
         const bool apply_mfma = !(apply_env && atoi(apply_env) == 0);
-        // fewest columns for the MFMA applies: above 64 only (from 32 columns in
-        // server contexts the served 64-request stream measured 187-192
-        // against 195-196 solves/s: three launches instead of one per block)
-        int apply_min = kSkinnyMaxCols + 1;
-        if (const char *e = getenv("EMFA_APPLY_MFMA_MIN")) apply_min = std::max(1, atoi(e));
         // rows [c_r0, c_r0 + M) of C -= F[rows, cols r0 .. r0 + wb) X_b
         auto update = [&](int M, const cx<R> *Fa, const cx<R> *Xb, cx<R> *C, int wb) -> emfa_status {
             if (M <= 0) return EMFA_OK;
             if (!skinny) return gemm_update<R>(ctx, "solve_gemm", M, m, wb, Fa, ldf, Bt, 2LL * wb, C, m);
             ProfScope ps2(ctx, "solve_gemm", 8.0 * (double)M * m * wb);
-            return smallmm<R, R>(ctx->stream, Fa, ldf, Xb, m, C, m, M, wb, m, 1, wb, R(-1), 1, nullptr);
+            return skinny_mm(ctx->stream, SkinnyJob<R, R>{Fa, ldf, Xb, m, C, m, M, wb, R(-1), 1}, m);
         };
         // Y_b = D_b^-1 W_b
         auto apply = [&](const cx<R> *D, int wb, const cx<R> *Wb, cx<R> *Yb) -> emfa_status {
-            if (skinny) return smallmm<R, R>(ctx->stream, D, kDinvB, Wb, m, Yb, m, wb, wb, m, 1, wb, R(1), 0, nullptr);
-            if (sizeof(R) == 4 && m >= apply_min && apply_mfma) {
+            if (skinny) return skinny_mm(ctx->stream, SkinnyJob<R, R>{D, kDinvB, Wb, m, Yb, m, wb, wb, R(1), 0}, m);
+            if (sizeof(R) == 4 && m > kSkinnyCols && apply_mfma) {
                 // many FP32 right-hand sides: Y_b = D_b W_b on the MFMA GEMM
                 // (W_b expanded first), then Y_b expanded for the update.
                 // k_dinv_apply ran 48 VALU workgroups at ~2 TFLOP/s here
@@ -2403,12 +2217,15 @@ static emfa_status solve_impl(emfa_ctx *ctx, const emfa_mat *LUm, const int *ipi
         // with the inverse-scaled blocks GH a step is one launch: the apply and
         // the other rows' update both read the step's input block
         const cx<R> *GH = skinny ? (const cx<R> *)gh : nullptr;
+        auto step = [&](const cx<R> *D, const cx<R> *G, const cx<R> *Wb, cx<R> *Yb, cx<R> *C, int wb, int M) {
+            const SkinnyJob<R, R> other{G, ldf, Wb, m, C, m, M, wb, R(-1), 1};
+            return skinny_mm(ctx->stream, SkinnyJob<R, R>{D, kDinvB, Wb, m, Yb, m, wb, wb, R(1), 0}, m, &other);
+        };
         for (int b = 0; b < nblk; ++b) {
             const int r0 = b * kDinvB, wb = std::min(kDinvB, N - r0);
             if (GH) {
-                st = solve_step<R>(ctx->stream, DL + (size_t)b * kDinvB * kDinvB, GH + (size_t)(r0 + wb) * ldf + r0,
-                                   ldf, W + (size_t)r0 * m, m, Y + (size_t)r0 * m, W + (size_t)(r0 + wb) * m, wb,
-                                   N - r0 - wb);
+                st = step(DL + (size_t)b * kDinvB * kDinvB, GH + (size_t)(r0 + wb) * ldf + r0, W + (size_t)r0 * m,
+                          Y + (size_t)r0 * m, W + (size_t)(r0 + wb) * m, wb, N - r0 - wb);
                 if (st) return st;
                 continue;
             }
@@ -2421,8 +2238,8 @@ static emfa_status solve_impl(emfa_ctx *ctx, const emfa_mat *LUm, const int *ipi
         for (int b = nblk - 1; b >= 0; --b) {
             const int r0 = b * kDinvB, wb = std::min(kDinvB, N - r0);
             if (GH) {
-                st = solve_step<R>(ctx->stream, DU + (size_t)b * kDinvB * kDinvB, GH + r0, ldf, Y + (size_t)r0 * m, m,
-                                   B + (size_t)r0 * m, Y, wb, r0);
+                st = step(DU + (size_t)b * kDinvB * kDinvB, GH + r0, Y + (size_t)r0 * m, B + (size_t)r0 * m, Y, wb,
+                          r0);
                 if (st) return st;
                 continue;
             }
@@ -2567,28 +2384,22 @@ emfa_status gemm_residual(emfa_ctx *ctx, const emfa_mat *A, const emfa_mat *X, e
     const int N = A->rows, K = A->cols, m = X->cols;
     EMFA_REQUIRE(X->rows == K && C->rows == N && C->cols == m && X->prec == EMFA_F64 && C->prec == EMFA_F64,
                  EMFA_E_INVALID, "gemm_residual: shape/precision mismatch");
-    // k_smallmm on the VALU up to 64 columns, the FP64 MFMA GEMM above.
-    // Contexts that share the device take the GEMM from 17 columns: the
-    // served 64-request stream (1045-14981 unknowns, 1-64 excitations per
-    // request) measured 116.3 against 107.2 solves/s (median of 3 passes),
-    // the VALU residual having held 18 % of the CUs' time.
+    // skinny FP64 MFMA products for few columns, the expanded-operand FP64
+    // MFMA GEMM for many (the rule at kSkinnyCols)
     static const char *resid_env = [] {
         const char *e = getenv("EMFA_RESID_SKINNY_MAX");
         return e ? e : getenv("EMFA_SKINNY_MAX");
     }();
-    const int resid_skinny_max =
-        resid_env ? std::min(kSkinnyMaxCols, atoi(resid_env)) : ctx->cu_share > 0 ? 16 : kSkinnyMaxCols;
+    const int resid_skinny_max = resid_env           ? std::min(kSkinnyMaxCols, atoi(resid_env))
+                                 : N <= kSkinnyMaxN ? kResidSkinnyCols
+                                                    : kSkinnyCols;
     if (m <= resid_skinny_max) {
-        // row blocks x K slices (summed in slice order) on the VALU
-        const int mc = m <= 8 ? 8 : m <= 16 ? 16 : m <= 32 ? 32 : 64;
-        // tall residuals with wide column tiles: 8 rows per lane (X re-read 4x less)
-        int rpt = N >= 2048 && mc >= 32 ? 8 : 2;
-        if (const char *e = getenv("EMFA_RESID_RPT")) rpt = atoi(e) == 8 && mc >= 32 ? 8 : 2;
-        const int rbk = rpt * (256 / mc);  // rows per workgroup of k_smallmm
-        const long long wgs = (N + rbk - 1) / rbk;
+        // 16-row tiles x 64-column groups x K slices (summed in slice order);
+        // the slices give every CU four workgroups
+        const long long wgs = (long long)((N + 15) / 16) * ((m + 63) / 64);
         int S = (int)std::min<long long>(32, std::max<long long>(1, (4LL * ctx->num_cu + wgs - 1) / wgs));
         if (const char *e = getenv("EMFA_RESID_SPLIT")) S = std::max(1, std::min(64, atoi(e)));
-        const int kc = (int)(((long long)K + S - 1) / S + 63) / 64 * 64;
+        const int kc = (int)(((long long)K + S - 1) / S + 127) / 128 * 128;
         S = (K + kc - 1) / kc;
         const size_t p_b = S > 1 ? (size_t)S * N * m * sizeof(cx<double>) : 0;
         void *scr = nullptr;
@@ -2601,10 +2412,14 @@ emfa_status gemm_residual(emfa_ctx *ctx, const emfa_mat *A, const emfa_mat *X, e
         const double sign = negate ? -1.0 : 1.0;
         emfa_status s2 =
             A->prec == EMFA_F32
-                ? smallmm<float, double>(ctx->stream, (const cx<float> *)A->d, K, (const cx<double> *)X->d, m,
-                                         (cx<double> *)C->d, m, N, K, m, S, kc, sign, accumulate, P, rpt)
-                : smallmm<double, double>(ctx->stream, (const cx<double> *)A->d, K, (const cx<double> *)X->d, m,
-                                          (cx<double> *)C->d, m, N, K, m, S, kc, sign, accumulate, P, rpt);
+                ? skinny_mm_slices(ctx->stream,
+                                   SkinnyJob<float, double>{(const cx<float> *)A->d, K, (const cx<double> *)X->d, m,
+                                                            (cx<double> *)C->d, m, N, K, sign, accumulate},
+                                   m, S, kc, P)
+                : skinny_mm_slices(ctx->stream,
+                                   SkinnyJob<double, double>{(const cx<double> *)A->d, K, (const cx<double> *)X->d, m,
+                                                             (cx<double> *)C->d, m, N, K, sign, accumulate},
+                                   m, S, kc, P);
         if (s2) return s2;
         if (S > 1) {
             const long long tot2 = (long long)N * 2 * m;
