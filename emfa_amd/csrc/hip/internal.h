@@ -59,10 +59,14 @@ struct Batch {
     int count = 1;
 };
 
+// The base comes out of memory, so the compiler cannot see that it is global
+// and would reach the matrix with flat instructions (which wait with LDS
+// operations); the cast says so.
 template <typename T>
 __device__ __forceinline__ T *batch_mat(const Batch &b, T *p, int z) {
     if (!b.mat) return p;
-    return (T *)(b.mat[z] + ((const char *)p - b.mat0));
+    using Global = const __attribute__((address_space(1))) char;
+    return (T *)(const char *)((Global *)b.mat[z] + ((const char *)p - b.mat0));
 }
 
 template <typename T>

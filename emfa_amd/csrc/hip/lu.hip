@@ -24,6 +24,7 @@
 
 #include "gemm.h"
 #include "internal.h"
+#include "nopiv.h"
 
 namespace emfa {
 
@@ -1547,218 +1548,6 @@ struct PermWs {
     }
 };
 
-// ---------------------------------------------------------------------------
-// Panel without row interchanges (FP32 factorisations that are refined in
-// FP64): the w x w diagonal block is factored in one workgroup, then every
-// row below solves x U11 = a on its own (L21 = A21 U11^-1), so a panel needs
-// no cross-workgroup exchange at all.  Both kernels raise flags[2] when a
-// pivot is zero or a multiplier exceeds sqrt(tau2) in modulus (partial
-// pivoting keeps them <= 1); the factorisation is then redone with
-// interchanges.
-// ---------------------------------------------------------------------------
-constexpr int kNoPivW = 64;  // widest pivot-free panel
-
-// Diagonal block (w <= 64): lane i of every wave holds row i, wave v holds
-// columns 4 v .. 4 v + 3 in registers (16 waves).  LU by 4-column blocks:
-// the owning wave factors its four columns (pivots read with v_readlane) and
-// publishes the four multiplier columns through LDS; after one barrier every
-// wave to the right forms the four pivot-row entries of its columns (a 4 x 4
-// unit-lower solve on wave-uniform values) and applies the rank-4 update.
-// Then U11^-1 from a copy of U in LDS by recursive doubling on all 16 waves
-// (tile_inv64), written to uinv (64 x 64, row-major).  Rows and columns past
-// w act as identity; the LU's LDS buffers alternate by block parity.
-// reciprocal for the pivot-free FP32 factor (refined in FP64 afterwards):
-// the hardware estimate (1 ulp) instead of a correctly rounded division
-template <typename R>
-__device__ __forceinline__ R fast_recip(R x) {
-    if constexpr (sizeof(R) == 4)
-        return __builtin_amdgcn_rcpf(x);
-    else
-        return R(1) / x;
-}
-
-template <typename R>
-__device__ __forceinline__ R lane_read(R v, int l) {
-    if constexpr (sizeof(R) == 4) {
-        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-    } else {
-        const long long b = __double_as_longlong(v);
-        const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
-        const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-        return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-    }
-}
-
-constexpr int kDiagCpw = 4, kDiagWaves = kNoPivW / kDiagCpw;  // columns per wave, waves
-
-template <typename R>
-__device__ __forceinline__ void cfms(cx<R> &acc, const cx<R> &a, const cx<R> &b) {  // acc -= a b
-    acc.re -= a.re * b.re - a.im * b.im;
-    acc.im -= a.re * b.im + a.im * b.re;
-}
-
-template <typename R>
-__global__ __launch_bounds__(kDiagWaves * 64) void k_diag_lu(cx<R> *__restrict__ A, long long lda, int js, int w,
-                                                            int *__restrict__ ipiv, int *flags, R tau2,
-                                                            cx<R> *__restrict__ uinv, Batch bt) {
-    // the matrix, its (scratch) pivots, flags and U11^-1 for the batch's matrix z
-    A = batch_mat(bt, A);
-    ipiv = batch_scr(bt, ipiv);
-    flags = batch_scr(bt, flags);
-    uinv = batch_scr(bt, uinv);
-    static_assert(sizeof(R) == 4, "the pivot-free diagonal block is an FP32 kernel");
-    __shared__ cx<R> buf[2][kDiagCpw][kNoPivW];
-    __shared__ cx<float> Tu[kNoPivW][kNoPivW + 1], Tx[kNoPivW][kNoPivW + 1], Tc[kNoPivW][kNoPivW + 1];
-    __shared__ int bad;
-    // wave index as a scalar: block tests below are uniform per wave
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    cx<R> a[kDiagCpw];
-#pragma unroll
-    for (int q = 0; q < kDiagCpw; ++q) {
-        const int j = kDiagCpw * wv + q;
-        a[q] = (lane < w && j < w) ? A[(size_t)(js + lane) * lda + js + j] : cx<R>{lane == j ? R(1) : R(0), R(0)};
-    }
-    if (threadIdx.x == 0) bad = 0;
-    bool mybad = false;
-    const int nbk = (w + kDiagCpw - 1) / kDiagCpw;
-    __syncthreads();
-    for (int b = 0; b < nbk; ++b) {
-        const int p = b & 1, c0 = kDiagCpw * b;
-        if (wv == b) {
-#pragma unroll
-            for (int cc = 0; cc < kDiagCpw; ++cc) {
-                const int c = c0 + cc;
-                cx<R> l = {R(0), R(0)};
-                if (c < w) {
-                    const R pr = lane_read(a[cc].re, c), pi = lane_read(a[cc].im, c);
-                    const R den = pr * pr + pi * pi;
-                    const R rd = den > R(0) ? fast_recip(den) : R(0);
-                    if (!(den > R(0))) mybad = true;
-                    const bool below = lane > c;
-                    l = cmul(a[cc], cx<R>{pr * rd, -pi * rd});
-                    if (!below) l = {R(0), R(0)};
-                    if (l.re * l.re + l.im * l.im > tau2) mybad = true;
-                    if (below) a[cc] = l;
-#pragma unroll
-                    for (int q = cc + 1; q < kDiagCpw; ++q) {
-                        const cx<R> u = {lane_read(a[q].re, c), lane_read(a[q].im, c)};
-                        cfms(a[q], l, u);
-                    }
-                }
-                buf[p][cc][lane] = l;
-            }
-        }
-        __syncthreads();
-        if (wv > b) {
-            cx<R> l[kDiagCpw];
-#pragma unroll
-            for (int m = 0; m < kDiagCpw; ++m) l[m] = buf[p][m][lane];
-#pragma unroll
-            for (int q = 0; q < kDiagCpw; ++q) {
-                cx<R> u[kDiagCpw];
-#pragma unroll
-                for (int k = 0; k < kDiagCpw; ++k) {
-                    u[k] = {lane_read(a[q].re, c0 + k), lane_read(a[q].im, c0 + k)};
-#pragma unroll
-                    for (int m = 0; m < k; ++m) cfms(u[k], buf[p][m][c0 + k], u[m]);
-                }
-#pragma unroll
-                for (int m = 0; m < kDiagCpw; ++m) cfms(a[q], l[m], u[m]);
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < kDiagCpw; ++q) {
-        const int j = kDiagCpw * wv + q;
-        if (lane < w && j < w) A[(size_t)(js + lane) * lda + js + j] = a[q];
-    }
-    // U11^-1 by recursive doubling on all waves, from a copy of U in LDS
-    // (the strictly lower part of the copy is never read)
-#pragma unroll
-    for (int q = 0; q < kDiagCpw; ++q) Tu[lane][kDiagCpw * wv + q] = a[q];
-    __syncthreads();
-    tile_inv64<true>(Tu, Tx, Tc, threadIdx.x, kDiagWaves * 64);
-    for (int e = threadIdx.x; e < kNoPivW * kNoPivW; e += kDiagWaves * 64) uinv[e] = Tx[e >> 6][e & 63];
-    if (threadIdx.x < w) ipiv[js + threadIdx.x] = js + threadIdx.x;
-    if (mybad) bad = 1;
-    __syncthreads();
-    if (threadIdx.x == 0 && bad) flags[2] = 1;
-}
-
-// Rows r0..r1-1 of the panel: L21 = A21 U11^-1 with the inverse from
-// k_diag_lu.  32 rows x w columns per workgroup (lane tx: column, rows
-// ty * 8 + a), in place: a workgroup reads all of its rows before writing.
-template <typename R>
-__device__ __forceinline__ void l21_body(cx<R> *__restrict__ A, long long lda, int js, int w, int r0, int r1,
-                                         const cx<R> *__restrict__ uinv, int *flags, R tau2, int bx,
-                                         cx<R> (*Us)[kNoPivW + 1], cx<R> (*As)[kNoPivW + 1]) {
-    const int tid = threadIdx.x, tx = tid & 63, ty = tid >> 6;
-    const int base = r0 + bx * 32, nrow = min(32, r1 - base);
-    for (int e = tid; e < kNoPivW * kNoPivW; e += 256) {
-        const int k = e >> 6, c = e & 63;
-        Us[k][c] = (k < w && c < w) ? uinv[k * kNoPivW + c] : cx<R>{R(0), R(0)};
-    }
-    for (int e = tid; e < 32 * kNoPivW; e += 256) {
-        const int r = e >> 6, c = e & 63;
-        As[r][c] = (r < nrow && c < w) ? A[(size_t)(base + r) * lda + js + c] : cx<R>{R(0), R(0)};
-    }
-    __syncthreads();
-    cx<R> acc[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) acc[q] = {R(0), R(0)};
-    for (int k = 0; k < w; ++k) {
-        const cx<R> u = Us[k][tx];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const cx<R> v = As[ty * 8 + q][k];
-            acc[q].re += v.re * u.re - v.im * u.im;
-            acc[q].im += v.re * u.im + v.im * u.re;
-        }
-    }
-    bool bad = false;
-    if (tx < w) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const int r = ty * 8 + q;
-            if (r < nrow) {
-                A[(size_t)(base + r) * lda + js + tx] = acc[q];
-                if (acc[q].re * acc[q].re + acc[q].im * acc[q].im > tau2) bad = true;
-            }
-        }
-    }
-    if (bad) flags[2] = 1;
-}
-
-template <typename R>
-__global__ __launch_bounds__(256) void k_l21(cx<R> *__restrict__ A, long long lda, int js, int w, int r0, int r1,
-                                            const cx<R> *__restrict__ uinv, int *flags, R tau2, Batch bt) {
-    __shared__ cx<R> Us[kNoPivW][kNoPivW + 1], As[32][kNoPivW + 1];
-    l21_body<R>(batch_mat(bt, A), lda, js, w, r0, r1, batch_scr(bt, uinv), batch_scr(bt, flags), tau2, blockIdx.x,
-                Us, As);
-}
-
-// The two products that follow a pivot-free diagonal block, in one launch:
-// workgroups [0, nl21) form L21 rows r0..r1-1 (as k_l21), the rest solve the
-// block's U rows for panel columns c0..c1-1 (as k_trsm64 with a unit-lower
-// 64-row block, writing Bt for the in-panel update).  The two touch disjoint
-// parts of A and only read the diagonal block, so they run side by side.
-template <typename R>
-__global__ __launch_bounds__(256) void k_l21_u12(cx<R> *__restrict__ A, long long lda, int js, int w, int r0,
-                                                int r1, const cx<R> *__restrict__ uinv, int *flags, R tau2,
-                                                int nl21, int c0, int c1, R *__restrict__ Bt, long long ldbt,
-                                                int passes, Batch bt) {
-    __shared__ cx<R> smem[(kNoPivW + 32) * (kNoPivW + 1)];
-    A = batch_mat(bt, A);
-    uinv = batch_scr(bt, uinv);
-    flags = batch_scr(bt, flags);
-    Bt = batch_scr(bt, Bt);
-    auto *T0 = (cx<R>(*)[kNoPivW + 1])smem;
-    if ((int)blockIdx.x < nl21)
-        l21_body<R>(A, lda, js, w, r0, r1, uinv, flags, tau2, blockIdx.x, T0, T0 + kNoPivW);
-    else
-        trsm64_body<R>(A, lda, A, lda, js, w, c0, c1, 0, Bt, ldbt, 0, passes, blockIdx.x - nl21, T0);
-}
-
 // Apply the interchanges k0..k1-1 to columns [c0,c1) and [c2,c3).
 template <typename R>
 static emfa_status laswp_launch(emfa_ctx *ctx, cx<R> *A, long long lda, const int *ipiv, int k0, int k1, int c0,
@@ -1888,7 +1677,7 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
         if (const char *e = getenv("EMFA_LU_BF16X3")) split_update = atoi(e) != 0;
     }
     size_t planes_b = split_update ? UpdatePlanes::bytes(N, nb) : 0;
-    const size_t uinv_b = (size_t)kNoPivW * kNoPivW * sizeof(cx<R>);
+    const size_t uinv_b = 2 * (size_t)kNoPivW * kNoPivW * sizeof(cx<R>);
     size_t total = slot_rows_b + slot_val_b + slot_idx_b + rowc_b + bar_b + 2 * bt_b + perm_b + x_pk_b + x_rw_b +
                    x_cw_b + x_val_b + planes_b + uinv_b + 8192;
     // a batch: one slab of this layout per matrix (plus its flags and pivots)
@@ -1921,7 +1710,8 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     R *x_val = (R *)take(x_val_b);
     UpdatePlanes planes;
     if (split_update) planes.carve(take(planes_b), N, nb);
-    cx<R> *uinv = (cx<R> *)take(uinv_b);  // U11^-1 of the current pivot-free panel
+    cx<R> *uinv = (cx<R> *)take(uinv_b);  // U11^-1 and L11^-1 of the current pivot-free panel
+    cx<R> *linv = uinv + kNoPivW * kNoPivW;
     // growth flags and pivots: the context's for one matrix, each slab's for a batch
     int *flagsp = batched ? (int *)take(256) : ctx->flags;
     int *ipivp = batched ? (int *)take((size_t)N * sizeof(int)) : ipiv;
@@ -1967,23 +1757,12 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
             const bool right = js + w < j0 + jb;  // panel columns right of the block
             if constexpr (sizeof(R) == 4) {
                 ProfScope ps(ctx, "lu_panel", 0);
-                const dim3 g1(1, 1, ctx->batch.count);
-                k_diag_lu<R><<<g1, kDiagWaves * 64, 0, ctx->stream>>>(A, lda, js, w, ipivp, flagsp, tau2, uinv,
-                                                                      ctx->batch);
-                const int nl21 = (N - js - w + 31) / 32;
-                if (right) {
-                    // L21 and the block's U rows (one 64-row step of trsm_blocked) in one launch
-                    const int c0 = js + w, c1 = j0 + jb, ncols = c1 - c0;
-                    const int passes = std::max(1, std::min(8, ncols / (kTrsmColsPerPass * 1024)));
-                    const int cpw = kTrsmColsPerPass * passes, nt = (ncols + cpw - 1) / cpw;
-                    k_l21_u12<R><<<dim3(nl21 + nt, 1, ctx->batch.count), 256, 0, ctx->stream>>>(
-                        A, lda, js, w, js + w, N, uinv, flagsp, tau2, nl21, c0, c1, Bt_in, 2LL * w, passes,
-                        ctx->batch);
-                } else if (nl21 > 0) {
-                    k_l21<R><<<dim3(nl21, 1, ctx->batch.count), 256, 0, ctx->stream>>>(A, lda, js, w, js + w, N, uinv,
-                                                                                        flagsp, tau2, ctx->batch);
-                }
-                EMFA_HIP_CHECK(hipGetLastError());
+                st = nopiv_diag_launch(ctx->stream, A, lda, js, w, ipivp, flagsp, tau2, uinv, linv, kNoPivW,
+                                       ctx->batch);
+                if (!st)
+                    st = nopiv_rows_launch(ctx->stream, A, lda, js, w, N, uinv, linv, kNoPivW, flagsp, tau2, js + w,
+                                           right ? j0 + jb : 0, Bt_in, 2LL * w, ctx->batch);
+                if (st) return st;
             }
             if (right) {
                 emfa_status s2 = gemm_update<R>(ctx, "lu_gemm", N - js - w, j0 + jb - js - w, w,
