@@ -1126,78 +1126,6 @@ __device__ __forceinline__ void tile_mac(TileAcc<R> &acc, const cx<R> (*Ta)[65],
     }
 }
 
-// Inverse of a triangular 64 x 64 FP32 tile held in LDS, by recursive
-// doubling: inverses of the 1 x 1 diagonal blocks, then for b = 1, 2, .., 32
-// each pair of b-blocks is joined (L: X21 = -X22 L21 X11; U: X12 = -X11 U12
-// X22), the product's middle factor staged in C.  T is read in its triangle
-// only (unit diagonal taken for L); X receives the inverse, zero in the other
-// triangle.  All `nthr` threads of the workgroup call it (it synchronises).
-template <bool UPPER>
-__device__ void tile_inv64(const cx<float> (*T)[65], cx<float> (*X)[65], cx<float> (*C)[65], int tid, int nthr) {
-    using R = float;
-    for (int e = tid; e < 64 * 64; e += nthr) {
-        const int rr = e >> 6, cc = e & 63;
-        cx<R> v = {R(0), R(0)};
-        if (rr == cc) {
-            if (UPPER) {
-                const cx<R> d = T[rr][rr];
-                const R den = d.re * d.re + d.im * d.im;
-                v = den > R(0) ? cx<R>{d.re / den, -d.im / den} : cx<R>{R(0), R(0)};
-            } else {
-                v = {R(1), R(0)};
-            }
-        }
-        X[rr][cc] = v;
-    }
-    __syncthreads();
-    for (int b = 1; b < 64; b *= 2) {
-        // pairs p: block start s = 2 b p; off-diagonal block rows/cols
-        // L: C = L21 X11 (rows s+b.., cols s..), then X21 = -X22 C
-        // U: C = U12 X22 (rows s.., cols s+b..), then X12 = -X11 C
-        const int per = b * b, tot = (64 / (2 * b)) * per;
-        for (int e = tid; e < tot; e += nthr) {
-            const int pr = e / per, q = e % per, rr = q / b, cc = q % b, s0 = 2 * b * pr;
-            cx<R> acc = {R(0), R(0)};
-            if (!UPPER) {
-                for (int k = 0; k < b; ++k) {
-                    const cx<R> a = T[s0 + b + rr][s0 + k], x = X[s0 + k][s0 + cc];
-                    acc.re += a.re * x.re - a.im * x.im;
-                    acc.im += a.re * x.im + a.im * x.re;
-                }
-                C[s0 + b + rr][s0 + cc] = acc;
-            } else {
-                for (int k = 0; k < b; ++k) {
-                    const cx<R> a = T[s0 + rr][s0 + b + k], x = X[s0 + b + k][s0 + b + cc];
-                    acc.re += a.re * x.re - a.im * x.im;
-                    acc.im += a.re * x.im + a.im * x.re;
-                }
-                C[s0 + rr][s0 + b + cc] = acc;
-            }
-        }
-        __syncthreads();
-        for (int e = tid; e < tot; e += nthr) {
-            const int pr = e / per, q = e % per, rr = q / b, cc = q % b, s0 = 2 * b * pr;
-            cx<R> acc = {R(0), R(0)};
-            if (!UPPER) {
-                for (int k = 0; k < b; ++k) {
-                    const cx<R> a = X[s0 + b + rr][s0 + b + k], x = C[s0 + b + k][s0 + cc];
-                    acc.re -= a.re * x.re - a.im * x.im;
-                    acc.im -= a.re * x.im + a.im * x.re;
-                }
-                X[s0 + b + rr][s0 + cc] = acc;
-            } else {
-                for (int k = 0; k < b; ++k) {
-                    const cx<R> a = X[s0 + rr][s0 + k], x = C[s0 + k][s0 + b + cc];
-                    acc.re -= a.re * x.re - a.im * x.im;
-                    acc.im -= a.re * x.im + a.im * x.re;
-                }
-                X[s0 + rr][s0 + b + cc] = acc;
-            }
-        }
-        __syncthreads();
-    }
-}
-
 template <typename R, bool UPPER>
 __device__ void tri_inv_block(const cx<R> *__restrict__ F, long long ldf, int N, cx<R> *__restrict__ Dinv,
                               cx<R> (*Ta)[65], cx<R> (*Tb)[65]) {
@@ -1314,101 +1242,6 @@ __global__ __launch_bounds__(256) void k_tri_inv(const cx<R> *__restrict__ F, lo
         tri_inv_block<R, false>(F, ldf, N, Dinv, Ta, Tb);
     else
         tri_inv_block<R, true>(F, ldf, N, Dinv + (size_t)gridDim.x * kDinvB * kDinvB, Ta, Tb);
-}
-
-// FP32 diagonal-block inverses spread over the chip.  k_dinv_diag inverts
-// every 64 x 64 diagonal tile (one workgroup per tile and triangle, grid
-// (blocks * 4, 2), blockIdx.y 0: unit lower, 1: upper) and zeroes the other
-// triangle of the tile's row; k_dinv_off(d), d = 1, 2, 3, forms the tiles on
-// the d-th sub-diagonal (L) or super-diagonal (U) of every 256-block, one
-// workgroup per tile (grid (blocks * (4 - d), 2)):
-//   L: X_{i,i-d} = -X_ii sum_{k=i-d}^{i-1} L_ik X_{k,i-d}
-//   U: X_{i,i+d} = -X_ii sum_{k=i+1}^{i+d} U_ik X_{k,i+d}
-// so each launch reads only tiles written by the earlier ones.  Layout as
-// k_tri_inv: L inverses at Dinv, U inverses at Dinv + blocks * 256 * 256,
-// row-major 256 x 256 per block; rows and columns past N act as identity.
-__device__ __forceinline__ void dinv_load_F(cx<float> (*T)[65], const cx<float> *__restrict__ F, long long ldf,
-                                            int N, int gr0, int gc0, int tid) {
-    for (int e = tid; e < 64 * 64; e += 256) {
-        const int rr = e >> 6, cc = e & 63, gr = gr0 + rr, gc = gc0 + cc;
-        cx<float> v = {0.f, 0.f};
-        if (gr < N && gc < N)
-            v = F[(size_t)gr * ldf + gc];
-        else if (gr == gc)
-            v = {1.f, 0.f};
-        T[rr][cc] = v;
-    }
-}
-
-__device__ __forceinline__ void dinv_load_X(cx<float> (*T)[65], const cx<float> *__restrict__ X, int i, int j,
-                                            int tid) {
-    for (int e = tid; e < 64 * 64; e += 256) T[e >> 6][e & 63] = X[(size_t)(64 * i + (e >> 6)) * kDinvB + 64 * j + (e & 63)];
-}
-
-__global__ __launch_bounds__(256) void k_dinv_diag(const cx<float> *__restrict__ F, long long ldf, int N,
-                                                   cx<float> *__restrict__ Dinv, int nblk, Batch bf, Batch bd) {
-    __shared__ cx<float> Ta[64][65], Tb[64][65], Tc[64][65];
-    F = batch_mat(bf, F);  // a batch: factor z and its inverses on blockIdx.z
-    Dinv = batch_mat(bd, Dinv);
-    const int blk = blockIdx.x >> 2, i = blockIdx.x & 3, tid = threadIdx.x;
-    const bool upper = blockIdx.y != 0;
-    cx<float> *X = Dinv + (upper ? (size_t)nblk * kDinvB * kDinvB : 0) + (size_t)blk * kDinvB * kDinvB;
-    const int r0 = blk * kDinvB + 64 * i;
-    dinv_load_F(Ta, F, ldf, N, r0, r0, tid);
-    __syncthreads();
-    if (upper)
-        tile_inv64<true>(Ta, Tb, Tc, tid, 256);
-    else
-        tile_inv64<false>(Ta, Tb, Tc, tid, 256);
-    for (int e = tid; e < 64 * 64; e += 256) X[(size_t)(64 * i + (e >> 6)) * kDinvB + 64 * i + (e & 63)] = Tb[e >> 6][e & 63];
-    for (int j = 0; j < 4; ++j)
-        if (upper ? j < i : j > i)
-            for (int e = tid; e < 64 * 64; e += 256)
-                X[(size_t)(64 * i + (e >> 6)) * kDinvB + 64 * j + (e & 63)] = {0.f, 0.f};
-}
-
-__global__ __launch_bounds__(256) void k_dinv_off(const cx<float> *__restrict__ F, long long ldf, int N,
-                                                  cx<float> *__restrict__ Dinv, int nblk, int d, Batch bf, Batch bd) {
-    __shared__ cx<float> Ta[64][65], Tb[64][65];
-    F = batch_mat(bf, F);
-    Dinv = batch_mat(bd, Dinv);
-    const int per = 4 - d, blk = blockIdx.x / per, t = blockIdx.x % per, tid = threadIdx.x;
-    const int ty = tid >> 4, tx = tid & 15;
-    const bool upper = blockIdx.y != 0;
-    cx<float> *X = Dinv + (upper ? (size_t)nblk * kDinvB * kDinvB : 0) + (size_t)blk * kDinvB * kDinvB;
-    const int r0 = blk * kDinvB;
-    const int i = upper ? t : d + t, j = upper ? i + d : i - d;
-    const int kb = upper ? i + 1 : j, ke = upper ? j : i - 1;  // inclusive
-    TileAcc<float> acc;
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc.v[a][b] = {0.f, 0.f};
-    for (int k = kb; k <= ke; ++k) {
-        if (k != kb) __syncthreads();
-        dinv_load_F(Ta, F, ldf, N, r0 + 64 * i, r0 + 64 * k, tid);
-        dinv_load_X(Tb, X, k, j, tid);
-        __syncthreads();
-        tile_mac(acc, Ta, Tb, ty, tx);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) Tb[ty * 4 + a][tx + 16 * b] = acc.v[a][b];
-    dinv_load_X(Ta, X, i, i, tid);
-    __syncthreads();
-    TileAcc<float> out;
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) out.v[a][b] = {0.f, 0.f};
-    tile_mac(out, Ta, Tb, ty, tx);
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-            X[(size_t)(64 * i + ty * 4 + a) * kDinvB + 64 * j + tx + 16 * b] = {-out.v[a][b].re, -out.v[a][b].im};
 }
 
 // Inverse-scaled off-diagonal blocks of an FP32 factor, for one-launch solve
@@ -1677,7 +1510,9 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
         if (const char *e = getenv("EMFA_LU_BF16X3")) split_update = atoi(e) != 0;
     }
     size_t planes_b = split_update ? UpdatePlanes::bytes(N, nb) : 0;
-    const size_t uinv_b = 2 * (size_t)kNoPivW * kNoPivW * sizeof(cx<R>);
+    // pivot-free panels: U11^-1 of the current one, L^-1 of the outer block's 256-blocks
+    const int nli = (nb + kInvB - 1) / kInvB;
+    const size_t uinv_b = ((size_t)kNoPivW * kNoPivW + (size_t)nli * kInvB * kInvB) * sizeof(cx<R>);
     size_t total = slot_rows_b + slot_val_b + slot_idx_b + rowc_b + bar_b + 2 * bt_b + perm_b + x_pk_b + x_rw_b +
                    x_cw_b + x_val_b + planes_b + uinv_b + 8192;
     // a batch: one slab of this layout per matrix (plus its flags and pivots)
@@ -1710,7 +1545,7 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     R *x_val = (R *)take(x_val_b);
     UpdatePlanes planes;
     if (split_update) planes.carve(take(planes_b), N, nb);
-    cx<R> *uinv = (cx<R> *)take(uinv_b);  // U11^-1 and L11^-1 of the current pivot-free panel
+    cx<R> *uinv = (cx<R> *)take(uinv_b);
     cx<R> *linv = uinv + kNoPivW * kNoPivW;
     // growth flags and pivots: the context's for one matrix, each slab's for a batch
     int *flagsp = batched ? (int *)take(256) : ctx->flags;
@@ -1757,10 +1592,11 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
             const bool right = js + w < j0 + jb;  // panel columns right of the block
             if constexpr (sizeof(R) == 4) {
                 ProfScope ps(ctx, "lu_panel", 0);
-                st = nopiv_diag_launch(ctx->stream, A, lda, js, w, ipivp, flagsp, tau2, uinv, linv, kNoPivW,
-                                       ctx->batch);
+                const int o = js - j0, t = o % kInvB;
+                cx<R> *li = linv + (size_t)(o / kInvB) * kInvB * kInvB + (size_t)t * kInvB + t;
+                st = nopiv_diag_launch(ctx->stream, A, lda, js, w, ipivp, flagsp, tau2, uinv, li, kInvB, ctx->batch);
                 if (!st)
-                    st = nopiv_rows_launch(ctx->stream, A, lda, js, w, N, uinv, linv, kNoPivW, flagsp, tau2, js + w,
+                    st = nopiv_rows_launch(ctx->stream, A, lda, js, w, N, uinv, li, kInvB, flagsp, tau2, js + w,
                                            right ? j0 + jb : 0, Bt_in, 2LL * w, ctx->batch);
                 if (st) return st;
             }
@@ -1772,6 +1608,11 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
             }
             js += w;
         }
+        if constexpr (sizeof(R) == 4)
+            if (nopiv && j0 + jb < N) {
+                ProfScope ps(ctx, "lu_panel", 0);
+                return nopiv_linv_launch(ctx->stream, A + (size_t)j0 * lda + j0, lda, jb, linv, ctx->batch);
+            }
         while (js < j0 + jb) {
             const int M = N - js;
             int w = std::min(plan.w, j0 + jb - js);
@@ -1827,6 +1668,22 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     auto outer_swap_trsm = [&](int j0, int jb) -> emfa_status {
         emfa_status s2 = nopiv ? EMFA_OK : laswp_launch<R>(ctx, A, lda, ipiv, j0, j0 + jb, 0, j0, j0 + jb, N, pws);
         if (s2) return s2;
+        if constexpr (sizeof(R) == 4) {
+            // U rows through the inverses of L's 256-blocks
+            for (int o = 0; nopiv && o < jb && j0 + jb < N; o += kInvB) {
+                const int wb = std::min(kInvB, jb - o), r0 = j0 + o;
+                for (int u = 0; u < o; u += kInvB) {
+                    s2 = gemm_update<R>(ctx, "trsm_gemm", wb, N - j0 - jb, kInvB, A + (size_t)r0 * lda + j0 + u, lda,
+                                        Bt_out + 2 * u, 2LL * jb, A + (size_t)r0 * lda + j0 + jb, lda);
+                    if (s2) return s2;
+                }
+                ProfScope ps(ctx, "lu_trsm", 0);
+                s2 = nopiv_urows_launch(ctx->stream, A, lda, r0, wb, j0 + jb, N,
+                                        linv + (size_t)(o / kInvB) * kInvB * kInvB, Bt_out, 2LL * jb, o, ctx->batch);
+                if (s2) return s2;
+            }
+            if (nopiv) return EMFA_OK;
+        }
         if (j0 + jb < N) return trsm_blocked<R>(ctx, A, lda, A, lda, j0, jb, j0 + jb, N, 0, Bt_out, "lu_trsm");
         return EMFA_OK;
     };
@@ -2090,14 +1947,6 @@ emfa_status lu_solve_inplace(emfa_ctx *ctx, const emfa_lu *lu, emfa_mat *B) {
     return solve_impl<double>(ctx, lu->a, lu->ipiv, lu->perm, B, lu->dinv, lu->interchanges);
 }
 
-// Inverses of the diagonal blocks of L (unit) and U, both [nblk][256][256]
-// FP32 diagonal-block inverses of one factor, or (bf, bd) of a batch of factors
-static void dinv_launch_f32(hipStream_t s, const cx<float> *F, int N, cx<float> *D, int nblk, const Batch &bf,
-                            const Batch &bd) {
-    k_dinv_diag<<<dim3(nblk * 4, 2, bf.count), 256, 0, s>>>(F, N, N, D, nblk, bf, bd);
-    for (int d = 1; d < 4; ++d) k_dinv_off<<<dim3(nblk * (4 - d), 2, bf.count), 256, 0, s>>>(F, N, N, D, nblk, d, bf, bd);
-}
-
 // the inverse-scaled off-diagonal blocks (GH) after the inverses
 static void gh_launch_f32(hipStream_t s, const cx<float> *F, int N, const cx<float> *D, int nblk, cx<float> *GH,
                           const Batch &bf, const Batch &bd, const Batch &bg) {
@@ -2128,7 +1977,8 @@ static emfa_status build_dinv(emfa_ctx *ctx, emfa_lu *lu) {
     if (lu->a->prec == EMFA_F32) {
         const cx<float> *F = (const cx<float> *)lu->a->d;
         cx<float> *D = (cx<float> *)lu->dinv;
-        dinv_launch_f32(ctx->stream, F, N, D, nblk, Batch(), Batch());
+        emfa_status st = dinv_f32_launch(ctx->stream, F, N, D, nblk, Batch(), Batch());
+        if (st) return st;
         if (gh_wanted()) {
             if (ctx_alloc(ctx, &lu->gh, (size_t)N * N * sizeof(cx<float>)) != hipSuccess) {
                 (void)hipGetLastError();
@@ -2496,8 +2346,9 @@ emfa_status emfa_lu_factor_batch(emfa_ctx *ctx, const emfa_mat *const *Z, int co
         bd.mat0 = hdinv[0];
         bd.count = count;
         ProfScope ps(ctx, "lu_dinv", 0);
-        dinv_launch_f32(ctx->stream, (const cx<float> *)lus[0]->a->d, n, (cx<float> *)lus[0]->dinv, nblk, bf, bd);
-        EMFA_HIP_CHECK(hipGetLastError());
+        if ((st = dinv_f32_launch(ctx->stream, (const cx<float> *)lus[0]->a->d, n, (cx<float> *)lus[0]->dinv, nblk,
+                                  bf, bd)))
+            return fail(st);
         if (gh_wanted()) {
             for (int z = 0; z < count; ++z) {
                 if (ctx_alloc(ctx, &lus[z]->gh, (size_t)n * n * sizeof(cx<float>)) != hipSuccess) {

@@ -23,4 +23,22 @@ emfa_status nopiv_rows_launch(hipStream_t s, cx<float> *A, long long lda, int js
                               const cx<float> *uinv, const cx<float> *linv, long long ldl, int *flags, float tau2,
                               int c0, int c1, float *Bt, long long ldbt, const Batch &bt);
 
+// L^-1 of the diagonal blocks of 256 of an outer block: F (n x n) factored, n <=
+// the outer block; Li holds ceil(n / 256) blocks of 256 x 256 in scratch whose
+// 64 x 64 diagonal tiles nopiv_diag_launch has written.
+emfa_status nopiv_linv_launch(hipStream_t s, const cx<float> *F, long long ldf, int n, cx<float> *Li,
+                              const Batch &bt);
+
+// U rows of one such block, in place: rows [r0, r0 + wb) of A, columns [c0, c1)
+// become L^-1 times themselves, also expanded into Bt at its complex K offset
+// kofs (row stride ldbt).
+emfa_status nopiv_urows_launch(hipStream_t s, cx<float> *A, long long lda, int r0, int wb, int c0, int c1,
+                               const cx<float> *Li, float *Bt, long long ldbt, int kofs, const Batch &bt);
+
+// Inverses of the 256 x 256 diagonal blocks of an FP32 factor F (N x N): Dinv
+// [2][nblk][256][256], L's (unit) then U's.  F in batch bf, Dinv in batch bd,
+// both as matrices.
+emfa_status dinv_f32_launch(hipStream_t s, const cx<float> *F, int N, cx<float> *Dinv, int nblk, const Batch &bf,
+                            const Batch &bd);
+
 }  // namespace emfa

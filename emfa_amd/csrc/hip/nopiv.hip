@@ -349,6 +349,167 @@ __global__ __launch_bounds__(256) void k_nopiv_rows(cf *__restrict__ A, long lon
     if (bad) flags[2] = 1;
 }
 
+// ---------------------------------------------------------------------------
+// Inverses of 256 x 256 diagonal blocks in three launches: every 64 x 64
+// diagonal tile (k_inv_diag), then pairs of 64, then pairs of 128 (k_inv_join,
+// one workgroup per 8 columns of a pair's off-diagonal block: the columns are
+// independent, so both products of X21 = -X22 (L21 X11) stay in it).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(kDiagThreads) void k_inv_diag(const cf *__restrict__ F, int N, cf *__restrict__ Dinv,
+                                                           int nblk, Batch bf, Batch bd) {
+    __shared__ __attribute__((aligned(16))) Tri64 T;
+    __shared__ cf dinv[64];
+    F = batch_mat(bf, F);
+    Dinv = batch_mat(bd, Dinv);
+    const int blk = blockIdx.x >> 2, i = blockIdx.x & 3, r0 = blk * kInvB + 64 * i;
+    const bool up = blockIdx.y != 0;
+    const int tid = threadIdx.x, lane = tid & 63, v = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (r0 >= N) return;
+    for (int r = v; r < 64; r += 16) {
+        // identity past the matrix
+        const cf d = (r0 + r < N && r0 + lane < N) ? F[(size_t)(r0 + r) * N + r0 + lane]
+                                                   : cf{r == lane ? 1.f : 0.f, 0.f};
+        T.m[0][r][lane] = d;
+        T.m[up ? 2 : 1][r][lane] = {0.f, 0.f};
+        if (r == lane) {
+            const float den = d.re * d.re + d.im * d.im;
+            dinv[r] = den > 0.f ? cf{d.re / den, -d.im / den} : cf{0.f, 0.f};
+        }
+    }
+    __syncthreads();
+    if (v == 0) {
+        if (up)
+            inv8<true>(T, dinv, lane);
+        else
+            inv8<false>(T, dinv, lane);
+    }
+    __syncthreads();
+    join64(T, up ? 2 : 1, v, lane);
+    cf *X = Dinv + (up ? (size_t)nblk * kInvB * kInvB : 0) + (size_t)blk * kInvB * kInvB + (size_t)64 * i * kInvB;
+    for (int r = v; r < 64; r += 16) {
+        X[(size_t)r * kInvB + 64 * i + lane] =
+            (up ? lane >= r : lane <= r) ? T.m[up ? 2 : 1][r][lane] : cf{0.f, 0.f};
+        for (int j = 0; j < 4; ++j)
+            if (up ? j < i : j > i) X[(size_t)r * kInvB + 64 * j + lane] = {0.f, 0.f};
+    }
+}
+
+template <int B>
+__global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long long ldf, int N,
+                                                  cf *__restrict__ Dinv, int nblk, int scr, Batch bf, Batch bd) {
+    constexpr int STRIPS = B / 8, PAIRS = kInvB / (2 * B), RT = B / 64;  // 16-row tiles per wave
+    __shared__ cf C[B][12];
+    F = batch_mat(bf, F);
+    Dinv = scr ? batch_scr(bd, Dinv) : batch_mat(bd, Dinv);
+    const int c = 8 * ((int)blockIdx.x % STRIPS), pr = (int)blockIdx.x / STRIPS, blk = pr / PAIRS;
+    const int s0 = 2 * B * (pr % PAIRS), s1 = s0 + B, r0 = blk * kInvB;
+    const bool up = blockIdx.y != 0;
+    if (r0 + s1 >= N) return;
+    cf *X = Dinv + (up ? (size_t)nblk * kInvB * kInvB : 0) + (size_t)blk * kInvB * kInvB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
+    const bool odd = l16 & 1;
+    // rows fr.. and columns fc.. of F times the strip of X that starts at row xk
+    const int fr = r0 + (up ? s0 : s1), fc = r0 + (up ? s1 : s0), xk = up ? s1 : s0;
+    const int k0 = up ? 0 : c, k1 = up ? c + 8 : B;  // X's strip is zero outside
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const int r = 16 * (RT * wave + t), row = fr + r + l16;
+        const cf *Ar = F + (size_t)min(row, N - 1) * ldf + fc;
+        const cf *Xs = X + (size_t)xk * kInvB + xk + c + (l16 >> 1);
+        f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int k = k0; k < k1; k += 8) {
+            const int ka = k + 2 * g;
+            f4 a = {0.f, 0.f, 0.f, 0.f};
+            if (row < N && fc + ka + 1 < N) {
+                a = *(const f4_a8 *)(Ar + ka);
+            } else if (row < N && fc + ka < N) {
+                a.x = Ar[ka].re;
+                a.y = Ar[ka].im;
+            }
+            acc = mac2(acc, a, Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB], odd);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ((float *)&C[r + 4 * g + i][0])[l16] = acc[i];
+    }
+    __syncthreads();
+    const int orow = up ? s0 : s1, ocol = (up ? s1 : s0) + c;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const int r = 16 * (RT * wave + t);
+        const cf *Ar = X + (size_t)(orow + r + l16) * kInvB + orow;
+        f4 acc = {0.f, 0.f, 0.f, 0.f};
+        const int j0 = up ? r : 0, j1 = up ? B : r + 16;
+#pragma unroll 4
+        for (int k = j0; k < j1; k += 8) {
+            const int ka = k + 2 * g;
+            acc = mac2(acc, *(const f4 *)(Ar + ka), C[ka][l16 >> 1], C[ka + 1][l16 >> 1], odd);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ((float *)(X + (size_t)(orow + r + 4 * g + i) * kInvB + ocol))[l16] = -acc[i];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// U rows of a 256-row block: U = L^-1 A on its rows, for 8 CT columns per
+// workgroup, in place (the columns go to LDS first).  Wave v takes 16-row
+// tiles v and 15 - v, so the triangle's work is even.  Against the blocked
+// substitution it replaces (per 64 rows one substitution and one update
+// launch, 15 launches per 512 rows) it is one launch per 256 rows.
+// ---------------------------------------------------------------------------
+template <int CT>
+__global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long long lda, int r0, int wb, int c0,
+                                                     int c1, const cf *__restrict__ Li, float *__restrict__ Bt,
+                                                     long long ldbt, int kofs, Batch bt) {
+    constexpr int S = 8 * CT;
+    __shared__ cf Xs[kInvB][S + 4];
+    A = batch_mat(bt, A);
+    Li = batch_scr(bt, Li);
+    Bt = batch_scr(bt, Bt);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
+    const bool odd = l16 & 1;
+    const int cb = c0 + S * (int)blockIdx.x;
+#pragma unroll 4
+    for (int e = tid; e < kInvB * S; e += 512) {
+        const int k = e / S, j = e % S;
+        Xs[k][j] = (k < wb && cb + j < c1) ? A[(size_t)(r0 + k) * lda + cb + j] : cf{0.f, 0.f};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const int r = 16 * (half ? 15 - wave : wave);
+        if (r >= wb) continue;
+        const cf *Ar = Li + (size_t)(r + l16) * kInvB + 2 * g;
+        f4 acc[CT];
+#pragma unroll
+        for (int t = 0; t < CT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int k = 0; k < r + 16; k += 8) {
+            const f4 a = *(const f4 *)(Ar + k);
+#pragma unroll
+            for (int t = 0; t < CT; ++t)
+                acc[t] = mac2(acc[t], a, Xs[k + 2 * g][8 * t + (l16 >> 1)], Xs[k + 2 * g + 1][8 * t + (l16 >> 1)],
+                              odd);
+        }
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+            const int j = cb + 8 * t + (l16 >> 1);
+            float o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = __shfl_xor(acc[t][i], 1) * (odd ? 1.f : -1.f);
+            if (j >= c1) continue;
+            // expanded operand: rows 2j {Re, -Im}, 2j + 1 {Im, Re}
+            float *b = Bt + (2LL * (j - c0) + odd) * ldbt + 2 * (kofs + r + 4 * g);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (r + 4 * g + i >= wb) continue;
+                ((float *)(A + (size_t)(r0 + r + 4 * g + i) * lda + j))[odd] = acc[t][i];
+                *(float2 *)(b + 2 * i) = make_float2(acc[t][i], o[i]);
+            }
+        }
+    }
+}
+
 }  // namespace
 
 emfa_status nopiv_diag_launch(hipStream_t s, cf *A, long long lda, int js, int w, int *ipiv, int *flags, float tau2,
@@ -366,6 +527,38 @@ emfa_status nopiv_rows_launch(hipStream_t s, cf *A, long long lda, int js, int w
     if (nl + nu <= 0) return EMFA_OK;
     k_nopiv_rows<<<dim3(nl + nu, 1, bt.count), 256, 0, s>>>(A, lda, js, w, N, uinv, linv, ldl, flags, tau2, nl, c0,
                                                             c1, Bt, ldbt, bt);
+    EMFA_HIP_CHECK(hipGetLastError());
+    return EMFA_OK;
+}
+
+emfa_status nopiv_linv_launch(hipStream_t s, const cf *F, long long ldf, int n, cf *Li, const Batch &bt) {
+    const int nblk = (n + kInvB - 1) / kInvB;
+    if (n > 64) k_inv_join<64><<<dim3(nblk * 16, 1, bt.count), 256, 0, s>>>(F, ldf, n, Li, nblk, 1, bt, bt);
+    if (n > 128) k_inv_join<128><<<dim3(nblk * 16, 1, bt.count), 256, 0, s>>>(F, ldf, n, Li, nblk, 1, bt, bt);
+    EMFA_HIP_CHECK(hipGetLastError());
+    return EMFA_OK;
+}
+
+emfa_status nopiv_urows_launch(hipStream_t s, cf *A, long long lda, int r0, int wb, int c0, int c1, const cf *Li,
+                               float *Bt, long long ldbt, int kofs, const Batch &bt) {
+    if (c1 <= c0 || wb <= 0) return EMFA_OK;
+    EMFA_REQUIRE(wb <= kInvB, EMFA_E_INVALID, "U rows of a block of %d", wb);
+    const int nc = c1 - c0;
+    // wider strips read L^-1 fewer times once they still fill the chip
+    if (nc * bt.count >= 32 * 1024)
+        k_nopiv_urows<4><<<dim3((nc + 31) / 32, 1, bt.count), 512, 0, s>>>(A, lda, r0, wb, c0, c1, Li, Bt, ldbt, kofs,
+                                                                          bt);
+    else
+        k_nopiv_urows<2><<<dim3((nc + 15) / 16, 1, bt.count), 512, 0, s>>>(A, lda, r0, wb, c0, c1, Li, Bt, ldbt, kofs,
+                                                                          bt);
+    EMFA_HIP_CHECK(hipGetLastError());
+    return EMFA_OK;
+}
+
+emfa_status dinv_f32_launch(hipStream_t s, const cf *F, int N, cf *Dinv, int nblk, const Batch &bf, const Batch &bd) {
+    k_inv_diag<<<dim3(nblk * 4, 2, bf.count), kDiagThreads, 0, s>>>(F, N, Dinv, nblk, bf, bd);
+    k_inv_join<64><<<dim3(nblk * 16, 2, bf.count), 256, 0, s>>>(F, N, N, Dinv, nblk, 0, bf, bd);
+    k_inv_join<128><<<dim3(nblk * 16, 2, bf.count), 256, 0, s>>>(F, N, N, Dinv, nblk, 0, bf, bd);
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
 }
