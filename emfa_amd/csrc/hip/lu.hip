@@ -2024,9 +2024,10 @@ emfa_status gemm_residual(emfa_ctx *ctx, const emfa_mat *A, const emfa_mat *X, e
                                                     : kSkinnyCols;
     if (m <= resid_skinny_max) {
         // 16-row tiles x 64-column groups x K slices (summed in slice order);
-        // the slices give every CU four workgroups
+        // enough slices that the last round of workgroups is a small part (8321
+        // unknowns, 49 columns: four workgroups per CU 20.2 ms, sixteen 19.9)
         const long long wgs = (long long)((N + 15) / 16) * ((m + 63) / 64);
-        int S = (int)std::min<long long>(32, std::max<long long>(1, (4LL * ctx->num_cu + wgs - 1) / wgs));
+        int S = (int)std::min<long long>(32, std::max<long long>(1, (16LL * ctx->num_cu + wgs - 1) / wgs));
         if (const char *e = getenv("EMFA_RESID_SPLIT")) S = std::max(1, std::min(64, atoi(e)));
         const int kc = (int)(((long long)K + S - 1) / S + 127) / 128 * 128;
         S = (K + kc - 1) / kc;

@@ -353,7 +353,9 @@ __global__ __launch_bounds__(256) void k_nopiv_rows(cf *__restrict__ A, long lon
 // Inverses of 256 x 256 diagonal blocks in three launches: every 64 x 64
 // diagonal tile (k_inv_diag), then pairs of 64, then pairs of 128 (k_inv_join,
 // one workgroup per 8 columns of a pair's off-diagonal block: the columns are
-// independent, so both products of X21 = -X22 (L21 X11) stay in it).
+// independent, so both products of X21 = -X22 (L21 X11) stay in it): 31 us per
+// factor whatever its size; 230 us with one VALU workgroup per 64 x 64 tile and
+// a launch per sub-diagonal.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kDiagThreads) void k_inv_diag(const cf *__restrict__ F, int N, cf *__restrict__ Dinv,
                                                            int nblk, Batch bf, Batch bd) {
@@ -417,17 +419,33 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
         const cf *Ar = F + (size_t)min(row, N - 1) * ldf + fc;
         const cf *Xs = X + (size_t)xk * kInvB + xk + c + (l16 >> 1);
         f4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int k = k0; k < k1; k += 8) {
-            const int ka = k + 2 * g;
-            f4 a = {0.f, 0.f, 0.f, 0.f};
-            if (row < N && fc + ka + 1 < N) {
-                a = *(const f4_a8 *)(Ar + ka);
-            } else if (row < N && fc + ka < N) {
-                a.x = Ar[ka].re;
-                a.y = Ar[ka].im;
+        if (fr + B <= N && fc + B <= N) {
+            // loads ahead of the products, 64 of K at a time; 64 x 64 tiles of X
+            // across the diagonal hold nothing
+#pragma unroll
+            for (int h = 0; h < B; h += 64) {
+                if (h >= k1 || h + 64 <= k0) continue;
+#pragma unroll
+                for (int k = h; k < h + 64; k += 8) {
+                    const int ka = k + 2 * g;
+                    acc = mac2(acc, *(const f4_a8 *)(Ar + ka), Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB],
+                               odd);
+                }
             }
-            acc = mac2(acc, a, Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB], odd);
+        } else {
+            for (int k = k0; k < k1; k += 8) {
+                const int ka = k + 2 * g;
+                f4 a = {0.f, 0.f, 0.f, 0.f};
+                if (row < N && fc + ka < N) {
+                    a.x = Ar[ka].re;
+                    a.y = Ar[ka].im;
+                }
+                if (row < N && fc + ka + 1 < N) {
+                    a.z = Ar[ka + 1].re;
+                    a.w = Ar[ka + 1].im;
+                }
+                acc = mac2(acc, a, Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB], odd);
+            }
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) ((float *)&C[r + 4 * g + i][0])[l16] = acc[i];
@@ -439,11 +457,14 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
         const int r = 16 * (RT * wave + t);
         const cf *Ar = X + (size_t)(orow + r + l16) * kInvB + orow;
         f4 acc = {0.f, 0.f, 0.f, 0.f};
-        const int j0 = up ? r : 0, j1 = up ? B : r + 16;
-#pragma unroll 4
-        for (int k = j0; k < j1; k += 8) {
-            const int ka = k + 2 * g;
-            acc = mac2(acc, *(const f4 *)(Ar + ka), C[ka][l16 >> 1], C[ka + 1][l16 >> 1], odd);
+#pragma unroll
+        for (int h = 0; h < B; h += 64) {
+            if (up ? h + 64 <= r : h > r) continue;
+#pragma unroll
+            for (int k = h; k < h + 64; k += 8) {
+                const int ka = k + 2 * g;
+                acc = mac2(acc, *(const f4 *)(Ar + ka), C[ka][l16 >> 1], C[ka + 1][l16 >> 1], odd);
+            }
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) ((float *)(X + (size_t)(orow + r + 4 * g + i) * kInvB + ocol))[l16] = -acc[i];
@@ -455,7 +476,8 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
 // workgroup, in place (the columns go to LDS first).  Wave v takes 16-row
 // tiles v and 15 - v, so the triangle's work is even.  Against the blocked
 // substitution it replaces (per 64 rows one substitution and one update
-// launch, 15 launches per 512 rows) it is one launch per 256 rows.
+// launch, 15 launches and 176 us per 512 rows at 1920 unknowns) it is one
+// launch per 256 rows: 50 us with the update between the two.
 // ---------------------------------------------------------------------------
 template <int CT>
 __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long long lda, int r0, int wb, int c0,
@@ -480,16 +502,26 @@ __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long lo
         const int r = 16 * (half ? 15 - wave : wave);
         if (r >= wb) continue;
         const cf *Ar = Li + (size_t)(r + l16) * kInvB + 2 * g;
-        f4 acc[CT];
+        f4 acc[CT], a[4];
 #pragma unroll
         for (int t = 0; t < CT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-        for (int k = 0; k < r + 16; k += 8) {
-            const f4 a = *(const f4 *)(Ar + k);
+        // steps of 32 of K, the next step's rows of L^-1 loaded ahead; the
+        // last step may reach past the tile's diagonal, where L^-1 is zero
 #pragma unroll
-            for (int t = 0; t < CT; ++t)
-                acc[t] = mac2(acc[t], a, Xs[k + 2 * g][8 * t + (l16 >> 1)], Xs[k + 2 * g + 1][8 * t + (l16 >> 1)],
-                              odd);
+        for (int q = 0; q < 4; ++q) a[q] = *(const f4 *)(Ar + 8 * q);
+        for (int k = 0; k < r + 16; k += 32) {
+            f4 nx[4];
+            const int kn = min(k + 32, kInvB - 32);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) nx[q] = *(const f4 *)(Ar + kn + 8 * q);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int t = 0; t < CT; ++t)
+                    acc[t] = mac2(acc[t], a[q], Xs[k + 8 * q + 2 * g][8 * t + (l16 >> 1)],
+                                  Xs[k + 8 * q + 2 * g + 1][8 * t + (l16 >> 1)], odd);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) a[q] = nx[q];
         }
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
@@ -544,13 +576,20 @@ emfa_status nopiv_urows_launch(hipStream_t s, cf *A, long long lda, int r0, int 
     if (c1 <= c0 || wb <= 0) return EMFA_OK;
     EMFA_REQUIRE(wb <= kInvB, EMFA_E_INVALID, "U rows of a block of %d", wb);
     const int nc = c1 - c0;
-    // wider strips read L^-1 fewer times once they still fill the chip
-    if (nc * bt.count >= 32 * 1024)
-        k_nopiv_urows<4><<<dim3((nc + 31) / 32, 1, bt.count), 512, 0, s>>>(A, lda, r0, wb, c0, c1, Li, Bt, ldbt, kofs,
+    // Wider strips read L^-1 fewer times, narrower ones have the shorter chain:
+    // 8 columns while they fill the chip at most twice over (1920 unknowns: 15.6
+    // us per launch, 16 columns 22.5)
+    const long long cols = (long long)nc * bt.count;
+    auto go = [&](auto kernel, int strip) {
+        kernel<<<dim3((nc + strip - 1) / strip, 1, bt.count), 512, 0, s>>>(A, lda, r0, wb, c0, c1, Li, Bt, ldbt, kofs,
                                                                           bt);
+    };
+    if (cols >= 16384)
+        go(k_nopiv_urows<4>, 32);
+    else if (cols >= 4096)
+        go(k_nopiv_urows<2>, 16);
     else
-        k_nopiv_urows<2><<<dim3((nc + 15) / 16, 1, bt.count), 512, 0, s>>>(A, lda, r0, wb, c0, c1, Li, Bt, ldbt, kofs,
-                                                                          bt);
+        go(k_nopiv_urows<1>, 8);
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
 }
