@@ -14,13 +14,82 @@
 //                       triangle, quadrature moments accumulated in registers
 //   K2 k_fill_singular  FP64 self terms (tf == ts), EFIE.cpp:231-542 and
 //                       Miscellaneous.cpp:32-77
-//   K1b k_fill_gather   Z(m,n) += l_m l_n s_m (Ztri(n+) - Ztri(n-)) per side
+//   K1b k_fill_gather   Z(m,n) = sum over sides of l_m l_n s_m (Ztri(n+) - Ztri(n-))
 #include <cmath>
 
 #include "em_device.h"
 #include "internal.h"
 
 namespace emfa {
+
+// ---------------------------------------------------------------------------
+// Elementary functions of the pair kernel.
+// ---------------------------------------------------------------------------
+// s = sqrt(x), h = 1 / (2 sqrt(x)) for x > 0: the hardware reciprocal root and
+// Goldschmidt steps (s <- s + s e, h <- h + h e, e = 1/2 - h s), then one
+// residual correction of s.
+__device__ __forceinline__ void root(float x, float *s, float *h) {
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y, g2 = 0.5f * y;
+    const float e = fmaf(-g2, g, 0.5f);
+    *h = fmaf(g2, e, g2);
+    const float r = fmaf(g, e, g);
+    *s = fmaf(fmaf(-r, r, x), *h, r);
+}
+__device__ __forceinline__ void root(double x, double *s, double *h) {
+    double y = __builtin_amdgcn_rsq(x), g = x * y, g2 = 0.5 * y;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const double e = fma(-g2, g, 0.5);
+        g2 = fma(g2, e, g2);
+        g = fma(g, e, g);
+    }
+    *h = g2;
+    *s = fma(fma(-g, g, x), g2, g);
+}
+
+// sin and cos of k r: quarter turns n = rint(k r 2/pi) are taken off with k
+// 2/pi as an unevaluated sum kq + kl (fused multiply-adds, so the reduced
+// angle keeps k r's full precision), then Taylor polynomials on [-pi/4, pi/4]
+// (first dropped term below 2e-9 in FP32, 5e-17 in FP64).  For angles below
+// 2^22 (FP32) and 2^31 (FP64) quarter turns.
+__device__ __forceinline__ void sincos_kr(float r, float kq, float kl, float *s, float *c) {
+    const float n = rintf(r * kq);
+    const float x = fmaf(r, kl, fmaf(r, kq, -n)) * 1.57079632679489662f, z = x * x;
+    const float sn = fmaf(x * z, fmaf(z, fmaf(z, fmaf(z, 1.f / 362880, -1.f / 5040), 1.f / 120), -1.f / 6), x);
+    const float cs =
+        fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, -1.f / 3628800, 1.f / 40320), -1.f / 720), 1.f / 24), -0.5f), 1.f);
+    const int q = (int)n;
+    const float a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
+    *s = __int_as_float(__float_as_int(a) ^ ((q & 2) << 30));
+    *c = __int_as_float(__float_as_int(b) ^ (((q + 1) & 2) << 30));
+}
+__device__ __forceinline__ void sincos_kr(double r, double kq, double kl, double *s, double *c) {
+    const double n = rint(r * kq);
+    // pi/2 = 1.5707963267948966 + 6.123233995736766e-17
+    const double f = fma(r, kl, fma(r, kq, -n));
+    const double x = fma(f, 1.5707963267948966, f * 6.123233995736766e-17), z = x * x;
+    double p = 1.0 / 1307674368000.0 * -1.0;
+    p = fma(z, p, 1.0 / 6227020800.0);
+    p = fma(z, p, -1.0 / 39916800.0);
+    p = fma(z, p, 1.0 / 362880.0);
+    p = fma(z, p, -1.0 / 5040.0);
+    p = fma(z, p, 1.0 / 120.0);
+    p = fma(z, p, -1.0 / 6.0);
+    const double sn = fma(x * z, p, x);
+    double u = 1.0 / 20922789888000.0;
+    u = fma(z, u, -1.0 / 87178291200.0);
+    u = fma(z, u, 1.0 / 479001600.0);
+    u = fma(z, u, -1.0 / 3628800.0);
+    u = fma(z, u, 1.0 / 40320.0);
+    u = fma(z, u, -1.0 / 720.0);
+    u = fma(z, u, 1.0 / 24.0);
+    u = fma(z, u, -0.5);
+    const double cs = fma(z, u, 1.0);
+    const int q = (int)n;
+    const double a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
+    *s = (q & 2) ? -a : a;
+    *c = ((q + 1) & 2) ? -b : b;
+}
 
 // ---------------------------------------------------------------------------
 // K1: regular triangle pairs.
@@ -31,15 +100,28 @@ namespace emfa {
 // integrand is accumulated as moments, from which the 9 (a, b) values follow:
 //   rho_f.rho_s = x.y - x.B - A.y + A.B          (A = v_a - c_f, B = v_b - c_s)
 //   rho_f.(n x (u x rho_s)) = (rho_f.u)(n.rho_s) - (rho_f.rho_s)(n.u)
+// Everything but x_p.y_q depends on p or q alone: with e_p = c_f - c_s + x_p,
+// u = e_p - y_q and, since n.x_p = 0, n.u = n.(c_f - c_s) - n.y_q.  So an
+// evaluation adds w G and the magnetic kernel to sums per p, sums per q and sums
+// weighted with x_p.y_q and n.y_q, and the vector moments are formed once per p
+// and per q.
+// VALU-bound: instructions per evaluation.  26.2M CFIE pairs (5120 triangles,
+// 3 points, FP32) PAIRS_F32; EFIE, 7 points, FP64, 3042 triangles PAIRS_F64.
 // ---------------------------------------------------------------------------
+template <typename R>
+__device__ __forceinline__ void axpy3(R *v, R s, const R *x) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[c] += s * x[c];
+}
+
 template <typename R, int Q, int KIND>
-__global__ __launch_bounds__(256) void k_fill_pairs(const R *__restrict__ tg, int T, int t0, int tcount, R k, R ik2,
-                                                    R cE_re, R cE_im, R cM, cx<R> *__restrict__ Ztri) {
-    __shared__ R s_src[15][64];
+__global__ __launch_bounds__(256) void k_fill_pairs(const R *__restrict__ tg, int T, int t0, int tcount, R k, R kq,
+                                                    R kl, R ik2, R cE, R cM, cx<R> *__restrict__ Ztri) {
+    __shared__ R s_src[12][64];
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int tsb = blockIdx.x * 64;
-    for (int i = threadIdx.x; i < 15 * 64; i += 256) {
+    for (int i = threadIdx.x; i < 12 * 64; i += 256) {
         int f = i >> 6, l = i & 63, ts = tsb + l;
         s_src[f][l] = ts < T ? tg[(size_t)f * T + ts] : R(0);
     }
@@ -48,111 +130,132 @@ __global__ __launch_bounds__(256) void k_fill_pairs(const R *__restrict__ tg, in
     if (tfl >= tcount) return;
     const int tf = __builtin_amdgcn_readfirstlane(t0 + tfl);
     const int ts = tsb + lane;
-    if (ts >= T) return;
+    if (ts >= T || ts == tf) return;  // self terms: K2
 
-    R cf[3], Af[3][3], nf[3];
+    R Af[3][3], nf[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        cf[c] = tg[(size_t)c * T + tf];
-        nf[c] = tg[(size_t)(12 + c) * T + tf];
-    }
+    for (int c = 0; c < 3; ++c) nf[c] = tg[(size_t)(12 + c) * T + tf];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int c = 0; c < 3; ++c) Af[i][c] = tg[(size_t)(3 + 3 * i + c) * T + tf];
     R Bs[3][3], d0[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) d0[c] = cf[c] - s_src[c][lane];
+    for (int c = 0; c < 3; ++c) d0[c] = tg[(size_t)c * T + tf] - s_src[c][lane];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int c = 0; c < 3; ++c) Bs[i][c] = s_src[3 + 3 * i + c][lane];
 
-    cx<R> *out = Ztri + (size_t)(tfl * 9) * T + ts;
-    if (ts == tf) {
-#pragma unroll
-        for (int ab = 0; ab < 9; ++ab) out[(size_t)ab * T] = {R(0), R(0)};
-        return;
-    }
-
-    R y[Q][3], wq[Q];
+    R y[Q][3], ny[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        wq[q] = (R)rule<Q>(q, 3);
 #pragma unroll
         for (int c = 0; c < 3; ++c)
             y[q][c] = (R)rule<Q>(q, 0) * Bs[0][c] + (R)rule<Q>(q, 1) * Bs[1][c] + (R)rule<Q>(q, 2) * Bs[2][c];
+        if (KIND == 1) ny[q] = dot3(nf, y[q]);
     }
+    const R nd = KIND == 1 ? dot3(nf, d0) : R(0);
 
-    // EFIE moments (re, im)
-    R S0r = 0, S0i = 0, Sxyr = 0, Sxyi = 0;
-    R Sxr[3] = {0, 0, 0}, Sxi[3] = {0, 0, 0}, Syr[3] = {0, 0, 0}, Syi[3] = {0, 0, 0};
-    // CFIE moments
-    R P1r = 0, P1i = 0, P2r = 0, P2i = 0, T0r = 0, T0i = 0, Txyr = 0, Txyi = 0;
+    // EFIE: sums of w G; per q; weighted with x.y; with x
+    R gqr[Q], gqi[Q], Sxyr = 0, Sxyi = 0, Sxr[3] = {0, 0, 0}, Sxi[3] = {0, 0, 0};
+    // CFIE: sums of the magnetic kernel per q, and per q weighted with x.y; Q1,
+    // Q2 (weights n.y u, u), P1, P2 (n.y x.u, x.u), Tx and the totals
+    R kqr[Q], kqi[Q], aqr[Q], aqi[Q];
+    R P1r = 0, P1i = 0, P2r = 0, P2i = 0, Kr = 0, Ki = 0, Nr = 0, Ni = 0;
     R Q1r[3] = {0, 0, 0}, Q1i[3] = {0, 0, 0}, Q2r[3] = {0, 0, 0}, Q2i[3] = {0, 0, 0};
-    R Txr[3] = {0, 0, 0}, Txi[3] = {0, 0, 0}, Tyr[3] = {0, 0, 0}, Tyi[3] = {0, 0, 0};
+    R Txr[3] = {0, 0, 0}, Txi[3] = {0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < Q; ++q) gqr[q] = gqi[q] = kqr[q] = kqi[q] = aqr[q] = aqi[q] = 0;
 
-#pragma unroll
+#pragma unroll(Q == 3 ? 3 : 1)
     for (int p = 0; p < Q; ++p) {
-        R x[3];
+        R x[3], e[3];
 #pragma unroll
-        for (int c = 0; c < 3; ++c)
+        for (int c = 0; c < 3; ++c) {
             x[c] = (R)rule<Q>(p, 0) * Af[0][c] + (R)rule<Q>(p, 1) * Af[1][c] + (R)rule<Q>(p, 2) * Af[2][c];
-        const R wp = (R)rule<Q>(p, 3);
+            e[c] = d0[c] + x[c];
+        }
+        const R wp2 = R(2) * (R)rule<Q>(p, 3);  // root() gives 1 / 2R
+        R gpr = 0, gpi = 0, kpr = 0, kpi = 0, npr = 0, npi = 0;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             R u[3];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) u[c] = d0[c] + x[c] - y[q][c];
-            R r2 = dot3(u, u);
-            R r = sqrt(r2);
-            R ir = R(1) / r;
-            R sn, cs;
-            sincos_r(k * r, &sn, &cs);
-            R w = wp * wq[q];
-            R gr = w * cs * ir, gi = -w * sn * ir;  // w * exp(-jkR)/R
-            R xy = dot3(x, y[q]);
-            S0r += gr;
-            S0i += gi;
+            for (int c = 0; c < 3; ++c) u[c] = e[c] - y[q][c];
+            R r, h, sn, cs;
+            root(dot3(u, u), &r, &h);
+            sincos_kr(r, kq, kl, &sn, &cs);
+            const R wir = wp2 * (R)rule<Q>(q, 3) * h;
+            const R gr = wir * cs, gi = -wir * sn;  // w * exp(-jkR)/R
+            const R xy = dot3(x, y[q]);
+            gpr += gr;
+            gpi += gi;
+            gqr[q] += gr;
+            gqi[q] += gi;
             Sxyr += gr * xy;
             Sxyi += gi * xy;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                Sxr[c] += gr * x[c];
-                Sxi[c] += gi * x[c];
-                Syr[c] += gr * y[q][c];
-                Syi[c] += gi * y[q][c];
-            }
             if (KIND == 1) {
-                // Kc = w (1 + jkR) G / R^2
-                R ir2 = ir * ir;
-                R kr = k * r;
-                R kcr = (gr - kr * gi) * ir2, kci = (gi + kr * gr) * ir2;
-                R xu = dot3(x, u), ny = dot3(nf, y[q]), nu = dot3(nf, u);
-                P1r += kcr * xu * ny;
-                P1i += kci * xu * ny;
-                P2r += kcr * xu;
-                P2i += kci * xu;
-                R knr = kcr * nu, kni = kci * nu;
-                T0r += knr;
-                T0i += kni;
-                Txyr += knr * xy;
-                Txyi += kni * xy;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    Q1r[c] += kcr * u[c] * ny;
-                    Q1i[c] += kci * u[c] * ny;
-                    Q2r[c] += kcr * u[c];
-                    Q2i[c] += kci * u[c];
-                    Txr[c] += knr * x[c];
-                    Txi[c] += kni * x[c];
-                    Tyr[c] += knr * y[q][c];
-                    Tyi[c] += kni * y[q][c];
-                }
+                // w (1 + jkR) G / R^2
+                const R kr = k * r, ir2 = R(4) * h * h;
+                const R kcr = (gr - kr * gi) * ir2, kci = (gi + kr * gr) * ir2;
+                kpr += kcr;
+                kpi += kci;
+                npr += kcr * ny[q];
+                npi += kci * ny[q];
+                kqr[q] += kcr;
+                kqi[q] += kci;
+                aqr[q] += kcr * xy;
+                aqi[q] += kci * xy;
             }
         }
+        axpy3(Sxr, gpr, x);
+        axpy3(Sxi, gpi, x);
+        if (KIND == 1) {
+            const R xe = dot3(x, e);
+            P1r += xe * npr;
+            P1i += xe * npi;
+            P2r += xe * kpr;
+            P2i += xe * kpi;
+            axpy3(Q1r, npr, e);
+            axpy3(Q1i, npi, e);
+            axpy3(Q2r, kpr, e);
+            axpy3(Q2i, kpi, e);
+            axpy3(Txr, nd * kpr - npr, x);
+            axpy3(Txi, nd * kpi - npi, x);
+            Kr += kpr;
+            Ki += kpi;
+            Nr += npr;
+            Ni += npi;
+        }
     }
+    R S0r = 0, S0i = 0, Syr[3] = {0, 0, 0}, Syi[3] = {0, 0, 0}, Tyr[3] = {0, 0, 0}, Tyi[3] = {0, 0, 0};
+    R Txyr = 0, Txyi = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        S0r += gqr[q];
+        S0i += gqi[q];
+        axpy3(Syr, gqr[q], y[q]);
+        axpy3(Syi, gqi[q], y[q]);
+        if (KIND == 1) {
+            const R nu = nd - ny[q];
+            axpy3(Tyr, nu * kqr[q], y[q]);
+            axpy3(Tyi, nu * kqi[q], y[q]);
+            axpy3(Q2r, -kqr[q], y[q]);
+            axpy3(Q2i, -kqi[q], y[q]);
+            axpy3(Q1r, -ny[q] * kqr[q], y[q]);
+            axpy3(Q1i, -ny[q] * kqi[q], y[q]);
+            P2r -= aqr[q];
+            P2i -= aqi[q];
+            P1r -= ny[q] * aqr[q];
+            P1i -= ny[q] * aqi[q];
+            Txyr += nu * aqr[q];
+            Txyi += nu * aqi[q];
+        }
+    }
+    const R T0r = nd * Kr - Nr, T0i = nd * Ki - Ni;
 
+    cx<R> *out = Ztri + (size_t)(tfl * 9) * T + ts;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
 #pragma unroll
@@ -162,8 +265,8 @@ __global__ __launch_bounds__(256) void k_fill_pairs(const R *__restrict__ tg, in
             R AB = dot3(A, B);
             R Ir = R(0.25) * (Sxyr - dot3(Sxr, B) - dot3(A, Syr) + AB * S0r) - ik2 * S0r;
             R Ii = R(0.25) * (Sxyi - dot3(Sxi, B) - dot3(A, Syi) + AB * S0i) - ik2 * S0i;
-            R zr = cE_re * Ir - cE_im * Ii;
-            R zi = cE_re * Ii + cE_im * Ir;
+            R zr = -cE * Ii;  // the electric part's factor is imaginary
+            R zi = cE * Ir;
             if (KIND == 1) {
                 R nB = dot3(nf, B);
                 R mr = (P1r - nB * P2r - dot3(A, Q1r) + nB * dot3(A, Q2r)) -
@@ -204,46 +307,73 @@ __global__ __launch_bounds__(64) void k_fill_singular(const double *__restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Gather: for rows m whose `side` triangle is in the chunk,
-//   Z(m,n) += l_m l_n s_m [Ztri(tf,a_m; n+, b_n+) - Ztri(tf,a_m; n-, b_n-)]
-//             + l_m l_n [Zsig(tf,a_m,b) for the source triangle equal to tf]
-// Each side is a separate launch, so no two threads update one entry.
+// Gather: for rows m with a triangle in the chunk,
+//   Z(m,n) (+)= l_m l_n s_m [Ztri(tf,a_m; n+, b_n+) - Ztri(tf,a_m; n-, b_n-)]
+//               + l_m l_n [Zsig(tf,a_m,b) for the source triangle equal to tf]
+// summed over the row's sides in the chunk, plus side first.  A row with both
+// triangles in the chunk is written once, by its plus side; one that spans two
+// chunks is written with the first and added to with the second, so every
+// entry is written and none is cleared beforehand.  A workgroup takes
+// kGatherRows half functions (tf, a) on 256 columns and reads the columns'
+// tables once.
+// HBM: the scratch once, Z once.  5120 triangles, FP32: GATHER_F32.
 // ---------------------------------------------------------------------------
+constexpr int kGatherRows = 4;
+
 template <typename R>
 __global__ __launch_bounds__(256) void k_fill_gather(const int *__restrict__ t2r, const int *__restrict__ rtp,
                                                      const int *__restrict__ rtm, const int *__restrict__ rap,
                                                      const int *__restrict__ ram, const R *__restrict__ rlen, int T,
-                                                     int N, int t0, int side, const cx<R> *__restrict__ Ztri,
+                                                     int N, int t0, int tcount, const cx<R> *__restrict__ Ztri,
                                                      const double *__restrict__ Zsig, cx<R> *__restrict__ Z) {
-    const int e = blockIdx.y;  // (tfl, a)
-    const int tfl = e / 3, a = e % 3;
-    const int tf = t0 + tfl;
-    const int code = t2r[(size_t)a * T + tf];
-    if (code == 0) return;
-    if ((code > 0) != (side > 0)) return;
-    const int m = (code > 0 ? code : -code) - 1;
-    const R s = code > 0 ? R(1) : R(-1);
     const int n = blockIdx.x * 256 + threadIdx.x;
     if (n >= N) return;
     const int tp = rtp[n], tm = rtm[n], bp = rap[n], bm = ram[n];
-    const cx<R> *row = Ztri + (size_t)(tfl * 3 + a) * 3 * T;
-    cx<R> zp = row[(size_t)bp * T + tp];
-    cx<R> zm = row[(size_t)bm * T + tm];
-    R vr = s * (zp.re - zm.re), vi = s * (zp.im - zm.im);
-    if (Zsig) {
-        if (tp == tf) {
-            vr += (R)Zsig[2 * ((size_t)(tfl * 3 + a) * 3 + bp)];
-            vi += (R)Zsig[2 * ((size_t)(tfl * 3 + a) * 3 + bp) + 1];
+    const size_t op = (size_t)bp * T + tp, om = (size_t)bm * T + tm;
+    const R ln = rlen[n];
+    // the side of row m on half function h = 3 tfl + a of the chunk
+    auto side = [&](int h, R s, R *vr, R *vi) {
+        const cx<R> *row = Ztri + (size_t)h * 3 * T;
+        const cx<R> zp = row[op], zm = row[om];
+        *vr = s * (zp.re - zm.re);
+        *vi = s * (zp.im - zm.im);
+        if (Zsig) {
+            const int tf = t0 + h / 3;
+            const double *zs = Zsig + 6 * (size_t)h;
+            if (tp == tf) {
+                *vr += (R)zs[2 * bp];
+                *vi += (R)zs[2 * bp + 1];
+            }
+            if (tm == tf) {
+                *vr += (R)zs[2 * bm];
+                *vi += (R)zs[2 * bm + 1];
+            }
         }
-        if (tm == tf) {
-            vr += (R)Zsig[2 * ((size_t)(tfl * 3 + a) * 3 + bm)];
-            vi += (R)Zsig[2 * ((size_t)(tfl * 3 + a) * 3 + bm) + 1];
+    };
+#pragma unroll
+    for (int i = 0; i < kGatherRows; ++i) {
+        const int e = blockIdx.y * kGatherRows + i;
+        if (e >= 3 * tcount) return;
+        const int tf = t0 + e / 3, a = e % 3, code = t2r[(size_t)a * T + tf];
+        if (code == 0) continue;
+        const bool plus = code > 0;
+        const int m = (plus ? code : -code) - 1;
+        const int other = plus ? rtm[m] : rtp[m];
+        const bool both = other >= t0 && other < t0 + tcount;
+        if (both && !plus) continue;
+        R vr, vi;
+        side(e, plus ? R(1) : R(-1), &vr, &vi);
+        const R ll = rlen[m] * ln;
+        cx<R> *z = Z + (size_t)m * N + n;
+        cx<R> old = {R(0), R(0)};
+        if (other < t0) old = *z;
+        cx<R> v = {old.re + ll * vr, old.im + ll * vi};
+        if (both) {
+            side(3 * (other - t0) + ram[m], R(-1), &vr, &vi);
+            v = {v.re + ll * vr, v.im + ll * vi};
         }
+        *z = v;
     }
-    R ll = rlen[m] * rlen[n];
-    cx<R> *z = Z + (size_t)m * N + n;
-    cx<R> old = *z;
-    *z = {old.re + ll * vr, old.im + ll * vi};
 }
 
 template <typename R>
@@ -272,25 +402,25 @@ static emfa_status fill_impl(emfa_ctx *ctx, const emfa_mesh *M, const emfa_fill_
     cx<R> *Ztri = (cx<R> *)scr;
     double *Zsig = sigma ? (double *)((char *)scr + (size_t)chunk * per_tri) : nullptr;
     cx<R> *Z = (cx<R> *)Zm->d;
-    EMFA_HIP_CHECK(hipMemsetAsync(Z, 0, Zm->bytes, ctx->stream));
 
     const double k = p->k;
     const double ce = k * kZ0 / (4.0 * kPi);  // |j k Z0 / 4 pi|
-    R cE_re = 0, cE_im, cM = 0;
-    if (p->kind == EMFA_EFIE) {
-        cE_im = (R)ce;
-    } else {
-        cE_im = (R)(p->alpha * ce);
+    R cE = (R)ce, cM = 0;  // the electric part's factor is j cE
+    if (p->kind == EMFA_CFIE) {
+        cE = (R)(p->alpha * ce);
         cM = (R)((1.0 - p->alpha) * kZ0 / (16.0 * kPi));
     }
     const R kr = (R)k, ik2 = (R)(1.0 / (k * k));
+    // k 2/pi in two parts of R
+    const long double kq2 = (long double)k * 2.0L / 3.14159265358979323846264338327950288L;
+    const R kq = (R)kq2, kl = (R)(kq2 - (long double)kq);
     for (int t0 = 0; t0 < T; t0 += chunk) {
         int tc = std::min(chunk, T - t0);
         {
             ProfScope ps(ctx, "fill_pairs", (double)tc * T * p->quad * p->quad);
             dim3 grid((T + 63) / 64, (tc + 3) / 4);
 #define LAUNCH_PAIRS(Q, KIND) \
-    k_fill_pairs<R, Q, KIND><<<grid, 256, 0, ctx->stream>>>(tg, T, t0, tc, kr, ik2, cE_re, cE_im, cM, Ztri)
+    k_fill_pairs<R, Q, KIND><<<grid, 256, 0, ctx->stream>>>(tg, T, t0, tc, kr, kq, kl, ik2, cE, cM, Ztri)
             if (p->quad == 7) {
                 if (p->kind == EMFA_EFIE)
                     LAUNCH_PAIRS(7, 0);
@@ -319,10 +449,9 @@ static emfa_status fill_impl(emfa_ctx *ctx, const emfa_mesh *M, const emfa_fill_
         }
         {
             ProfScope ps(ctx, "fill_gather", 0);
-            dim3 grid((N + 255) / 256, tc * 3);
-            for (int side = 1; side >= -1; side -= 2)
-                k_fill_gather<R><<<grid, 256, 0, ctx->stream>>>(M->t2r, M->rtp, M->rtm, M->rap, M->ram, rlen, T, N,
-                                                                t0, side, Ztri, Zsig, Z);
+            dim3 grid((N + 255) / 256, (tc * 3 + kGatherRows - 1) / kGatherRows);
+            k_fill_gather<R><<<grid, 256, 0, ctx->stream>>>(M->t2r, M->rtp, M->rtm, M->rap, M->ram, rlen, T, N, t0,
+                                                            tc, Ztri, Zsig, Z);
             EMFA_HIP_CHECK(hipGetLastError());
         }
     }
