@@ -12,7 +12,7 @@
 //   K1 k_fill_pairs     one wavefront per (test triangle, 64 source triangles),
 //                       source geometry staged in LDS, one lane per source
 //                       triangle, quadrature moments accumulated in registers
-//   K2 k_fill_singular  FP64 self terms (tf == ts), EFIE.cpp:231-542 and
+//   K2 k_fill_singular  FP64 self terms (tf == ts) of all triangles, EFIE.cpp:231-542,
 //                       Miscellaneous.cpp:32-77
 //   K1b k_fill_gather   Z(m,n) = sum over sides of l_m l_n s_m (Ztri(n+) - Ztri(n-))
 #include <cmath>
@@ -106,7 +106,9 @@ __device__ __forceinline__ void sincos_kr(double r, double kq, double kl, double
 // weighted with x_p.y_q and n.y_q, and the vector moments are formed once per p
 // and per q.
 // VALU-bound: instructions per evaluation.  26.2M CFIE pairs (5120 triangles,
-// 3 points, FP32) PAIRS_F32; EFIE, 7 points, FP64, 3042 triangles PAIRS_F64.
+// 3 points, FP32) 1.23 -> 0.95 ms (2.5e11 evaluations/s, 2 TB/s of scratch
+// written); EFIE, 7 points, FP64, 3042 triangles 4.0 -> 1.28 ms, against
+// library roots, divisions and sincos and moments formed per evaluation.
 // ---------------------------------------------------------------------------
 template <typename R>
 __device__ __forceinline__ void axpy3(R *v, R s, const R *x) {
@@ -282,27 +284,96 @@ __global__ __launch_bounds__(256) void k_fill_pairs(const R *__restrict__ tg, in
 }
 
 // ---------------------------------------------------------------------------
-// K2: self terms in FP64 (self_term in em_device.h).
+// K2: self terms in FP64 (the formulas of self_term in em_device.h), one lane
+// per triangle and point p: a group of G lanes forms the nine (a, b) values of
+// a triangle, point by point, and adds them over its lanes.  All triangles in
+// one launch: it is a chain of logarithms and divisions, 18 us whatever the
+// count as one thread per (a, b) looping over the points.
 // ---------------------------------------------------------------------------
 template <typename R, int Q>
-__global__ __launch_bounds__(64) void k_fill_singular(const double *__restrict__ tg, int T, int t0, int tcount, int kind,
-                                                      double k, double alpha, double sig_re, double sig_im,
-                                                      int cfie_mode, cx<R> *__restrict__ Ztri,
-                                                      double *__restrict__ Zsig) {
-    int id = blockIdx.x * 64 + threadIdx.x;
-    if (id >= tcount * 9) return;
-    int tfl = id / 9, ab = id % 9, a = ab / 3, b = ab % 3;
-    int tf = t0 + tfl;
-    d3 t[3];
-    for (int i = 0; i < 3; ++i)
-        t[i] = mk3(tg[(size_t)(3 + 3 * i) * T + tf], tg[(size_t)(4 + 3 * i) * T + tf], tg[(size_t)(5 + 3 * i) * T + tf]);
-    double area = tg[(size_t)15 * T + tf];
-    double zr, zi, gr, gi;
-    self_term<Q>(kind, k, alpha, sig_re, sig_im, cfie_mode, t, area, a, b, &zr, &zi, &gr, &gi);
-    Ztri[(size_t)(tfl * 9 + ab) * T + tf] = {(R)zr, (R)zi};
-    if (Zsig) {
-        Zsig[2 * ((size_t)tfl * 9 + ab)] = gr;
-        Zsig[2 * ((size_t)tfl * 9 + ab) + 1] = gi;
+__global__ __launch_bounds__(64) void k_fill_singular(const double *__restrict__ tg, int T, int kind, double k,
+                                                      double alpha, double sig_re, double sig_im, int cfie_mode,
+                                                      cx<R> *__restrict__ Zself, double *__restrict__ Zsig) {
+    constexpr int G = Q == 3 ? 4 : 8;
+    const int p = threadIdx.x % G, tf = blockIdx.x * (64 / G) + threadIdx.x / G;
+    double zr[9], zi[9], gs[9];
+#pragma unroll
+    for (int ab = 0; ab < 9; ++ab) zr[ab] = zi[ab] = gs[ab] = 0;
+    if (tf < T && p < Q) {
+        d3 t[3];
+        for (int i = 0; i < 3; ++i)
+            t[i] = mk3(tg[(size_t)(3 + 3 * i) * T + tf], tg[(size_t)(4 + 3 * i) * T + tf],
+                       tg[(size_t)(5 + 3 * i) * T + tf]);
+        const double area = tg[(size_t)15 * T + tf], ik2 = 1.0 / (k * k), wp = rule<Q>(p, 3);
+        auto point = [&](int q) { return t[0] * rule<Q>(q, 0) + t[1] * rule<Q>(q, 1) + t[2] * rule<Q>(q, 2); };
+        const d3 r = point(p);
+        // Taylor part (exp(-jkR)-1)/R ~ -jk - k^2 R/2 + j k^3 R^2/6 (EFIE.cpp:251-256)
+        double er[9], ei[9];
+#pragma unroll
+        for (int ab = 0; ab < 9; ++ab) er[ab] = ei[ab] = 0;
+#pragma unroll 1
+        for (int q = 0; q < Q; ++q) {
+            const d3 rq = point(q);
+            const double Rd = normd(r - rq), f = wp * rule<Q>(q, 3);
+            const double cr = -0.5 * k * k * Rd * f, ci = (k / 6.0) * (k * k * Rd * Rd - 6.0) * f;
+#pragma unroll
+            for (int ab = 0; ab < 9; ++ab) {
+                const double g = 0.25 * dotd(r - t[ab / 3], rq - t[ab % 3]) - ik2;
+                er[ab] += g * cr;
+                ei[ab] += g * ci;
+            }
+        }
+        const bool quirk = kind == EMFA_CFIE && cfie_mode == 0;
+        d3 Is1 = mk3(0, 0, 0);
+        double pot = 0;
+        if (quirk) {
+            // Miscellaneous.cpp:53-66: in-plane log terms with the last inner rho_s
+#pragma unroll 1
+            for (int i = 0; i < 3; ++i) {
+                const d3 va = t[i], vb = t[i == 2 ? 0 : i + 1], Li = unitd(vb - va);
+                const double Lp = dotd(vb - r, Li), Lm = dotd(va - r, Li), Rp = normd(vb - r), Rm = normd(va - r);
+                const double P0 = normd(va + Li * dotd(r - va, Li) - r);
+                if (P0 > 1e-10) pot += P0 * log((Rp + Lp) / (Rm + Lm));
+            }
+        } else {
+            potentials(t, r, &Is1, &pot);
+        }
+        const double ce = k * kZ0 / (4.0 * kPi);
+        const d3 last = point(Q - 1);
+#pragma unroll
+        for (int ab = 0; ab < 9; ++ab) {
+            const d3 rf = r - t[ab / 3], rs = r - t[ab % 3];
+            const double same = wp * dotd(rf, rs);
+            const double e2 = quirk ? wp * (0.25 * dotd(rf, last - t[ab % 3]) - ik2) * pot
+                                    : wp * (0.25 * dotd(rf, Is1 + rs * pot) - pot * ik2);
+            // coefE = j k Z0 / 4 pi applied to (Ze1 + Ze2 / area)
+            const double vr = -ce * ei[ab], vi = ce * (er[ab] + e2 / area);
+            if (kind == EMFA_EFIE) {
+                zr[ab] = vr;
+                zi[ab] = vi;
+                // Sigma term (EFIE.cpp:297-306), coefE included: 1 / (4 S)
+                gs[ab] = same / (4.0 * area);
+            } else {
+                zr[ab] = alpha * vr + (1.0 - alpha) * kZ0 * same / (8.0 * area);
+                zi[ab] = alpha * vi;
+            }
+        }
+    }
+#pragma unroll
+    for (int ab = 0; ab < 9; ++ab) {
+#pragma unroll
+        for (int o = 1; o < G; o *= 2) {
+            zr[ab] += __shfl_xor(zr[ab], o);
+            zi[ab] += __shfl_xor(zi[ab], o);
+            if (Zsig) gs[ab] += __shfl_xor(gs[ab], o);
+        }
+        if (tf < T && p == ab % G) {
+            Zself[(size_t)tf * 9 + ab] = {(R)zr[ab], (R)zi[ab]};
+            if (Zsig) {
+                Zsig[2 * ((size_t)tf * 9 + ab)] = gs[ab] * sig_re;
+                Zsig[2 * ((size_t)tf * 9 + ab) + 1] = gs[ab] * sig_im;
+            }
+        }
     }
 }
 
@@ -316,7 +387,9 @@ __global__ __launch_bounds__(64) void k_fill_singular(const double *__restrict__
 // entry is written and none is cleared beforehand.  A workgroup takes
 // kGatherRows half functions (tf, a) on 256 columns and reads the columns'
 // tables once.
-// HBM: the scratch once, Z once.  5120 triangles, FP32: GATHER_F32.
+// HBM: the scratch once, Z once.  5120 triangles, FP32: 0.51 ms, 4.6 TB/s
+// (clearing Z and adding each side in a launch of its own: 0.88 ms).  Gathering
+// a chunk on a second stream during the next one's pairs gained nothing.
 // ---------------------------------------------------------------------------
 constexpr int kGatherRows = 4;
 
@@ -325,6 +398,7 @@ __global__ __launch_bounds__(256) void k_fill_gather(const int *__restrict__ t2r
                                                      const int *__restrict__ rtm, const int *__restrict__ rap,
                                                      const int *__restrict__ ram, const R *__restrict__ rlen, int T,
                                                      int N, int t0, int tcount, const cx<R> *__restrict__ Ztri,
+                                                     const cx<R> *__restrict__ Zself,
                                                      const double *__restrict__ Zsig, cx<R> *__restrict__ Z) {
     const int n = blockIdx.x * 256 + threadIdx.x;
     if (n >= N) return;
@@ -334,12 +408,13 @@ __global__ __launch_bounds__(256) void k_fill_gather(const int *__restrict__ t2r
     // the side of row m on half function h = 3 tfl + a of the chunk
     auto side = [&](int h, R s, R *vr, R *vi) {
         const cx<R> *row = Ztri + (size_t)h * 3 * T;
-        const cx<R> zp = row[op], zm = row[om];
+        const int tf = t0 + h / 3;
+        const cx<R> *own = Zself + 9 * (size_t)t0 + 3 * (size_t)h;
+        const cx<R> zp = tp == tf ? own[bp] : row[op], zm = tm == tf ? own[bm] : row[om];
         *vr = s * (zp.re - zm.re);
         *vi = s * (zp.im - zm.im);
         if (Zsig) {
-            const int tf = t0 + h / 3;
-            const double *zs = Zsig + 6 * (size_t)h;
+            const double *zs = Zsig + 18 * (size_t)t0 + 6 * (size_t)h;
             if (tp == tf) {
                 *vr += (R)zs[2 * bp];
                 *vi += (R)zs[2 * bp + 1];
@@ -389,18 +464,20 @@ static emfa_status fill_impl(emfa_ctx *ctx, const emfa_mesh *M, const emfa_fill_
         rlen = (const R *)M->rlen64;
     }
     const bool sigma = p->kind == EMFA_EFIE && std::hypot(p->sigma_re, p->sigma_im) > 1e-8;
-    size_t per_tri = 9 * (size_t)T * sizeof(cx<R>);
+    const size_t per_tri = 9 * (size_t)T * sizeof(cx<R>);
     size_t budget = (size_t)2 << 30;
     if (const char *s = getenv("EMFA_FILL_SCRATCH_MB")) budget = (size_t)atol(s) << 20;
     int chunk = (int)std::min<size_t>((size_t)T, std::max<size_t>(4, budget / per_tri));
     chunk = std::min(chunk, 16384);
     chunk = (chunk + 3) & ~3;
-    size_t bytes = (size_t)chunk * per_tri + (sigma ? (size_t)chunk * 9 * 2 * sizeof(double) : 0);
+    const size_t buf_b = ((size_t)chunk * per_tri + 255) & ~(size_t)255;
+    const size_t self_b = (9 * (size_t)T * sizeof(cx<R>) + 255) & ~(size_t)255;
     void *scr = nullptr;
-    emfa_status st = ctx_scratch(ctx, bytes, &scr);
+    emfa_status st = ctx_scratch(ctx, buf_b + self_b + (sigma ? 18 * (size_t)T * sizeof(double) : 0), &scr);
     if (st != EMFA_OK) return st;
     cx<R> *Ztri = (cx<R> *)scr;
-    double *Zsig = sigma ? (double *)((char *)scr + (size_t)chunk * per_tri) : nullptr;
+    cx<R> *Zself = (cx<R> *)((char *)scr + buf_b);
+    double *Zsig = sigma ? (double *)((char *)Zself + self_b) : nullptr;
     cx<R> *Z = (cx<R> *)Zm->d;
 
     const double k = p->k;
@@ -414,6 +491,16 @@ static emfa_status fill_impl(emfa_ctx *ctx, const emfa_mesh *M, const emfa_fill_
     // k 2/pi in two parts of R
     const long double kq2 = (long double)k * 2.0L / 3.14159265358979323846264338327950288L;
     const R kq = (R)kq2, kl = (R)(kq2 - (long double)kq);
+    {
+        constexpr int per7 = 64 / 8, per3 = 64 / 4;  // triangles per workgroup
+        if (p->quad == 7)
+            k_fill_singular<R, 7><<<(T + per7 - 1) / per7, 64, 0, ctx->stream>>>(
+                M->tg64, T, p->kind, k, p->alpha, p->sigma_re, p->sigma_im, p->cfie_mode, Zself, Zsig);
+        else
+            k_fill_singular<R, 3><<<(T + per3 - 1) / per3, 64, 0, ctx->stream>>>(
+                M->tg64, T, p->kind, k, p->alpha, p->sigma_re, p->sigma_im, p->cfie_mode, Zself, Zsig);
+        EMFA_HIP_CHECK(hipGetLastError());
+    }
     for (int t0 = 0; t0 < T; t0 += chunk) {
         int tc = std::min(chunk, T - t0);
         {
@@ -436,22 +523,10 @@ static emfa_status fill_impl(emfa_ctx *ctx, const emfa_mesh *M, const emfa_fill_
             EMFA_HIP_CHECK(hipGetLastError());
         }
         {
-            dim3 grid((tc * 9 + 63) / 64);
-            if (p->quad == 7)
-                k_fill_singular<R, 7><<<grid, 64, 0, ctx->stream>>>(M->tg64, T, t0, tc, p->kind, k, p->alpha,
-                                                                     p->sigma_re, p->sigma_im, p->cfie_mode, Ztri,
-                                                                     Zsig);
-            else
-                k_fill_singular<R, 3><<<grid, 64, 0, ctx->stream>>>(M->tg64, T, t0, tc, p->kind, k, p->alpha,
-                                                                     p->sigma_re, p->sigma_im, p->cfie_mode, Ztri,
-                                                                     Zsig);
-            EMFA_HIP_CHECK(hipGetLastError());
-        }
-        {
             ProfScope ps(ctx, "fill_gather", 0);
             dim3 grid((N + 255) / 256, (tc * 3 + kGatherRows - 1) / kGatherRows);
             k_fill_gather<R><<<grid, 256, 0, ctx->stream>>>(M->t2r, M->rtp, M->rtm, M->rap, M->ram, rlen, T, N, t0,
-                                                            tc, Ztri, Zsig, Z);
+                                                            tc, Ztri, Zself, Zsig, Z);
             EMFA_HIP_CHECK(hipGetLastError());
         }
     }
