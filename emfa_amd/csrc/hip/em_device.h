@@ -35,6 +35,83 @@ __device__ __forceinline__ R dot3(const R *a, const R *b) {
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
 }
 
+// ---------------------------------------------------------------------------
+// Elementary functions of the fill, excitation and far-field kernels.
+// ---------------------------------------------------------------------------
+// s = sqrt(x), h = 1 / (2 sqrt(x)) for x > 0: the hardware reciprocal root and
+// Goldschmidt steps (s <- s + s e, h <- h + h e, e = 1/2 - h s), then one
+// residual correction of s.
+__device__ __forceinline__ void root(float x, float *s, float *h) {
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y, g2 = 0.5f * y;
+    const float e = fmaf(-g2, g, 0.5f);
+    *h = fmaf(g2, e, g2);
+    const float r = fmaf(g, e, g);
+    *s = fmaf(fmaf(-r, r, x), *h, r);
+}
+__device__ __forceinline__ void root(double x, double *s, double *h) {
+    double y = __builtin_amdgcn_rsq(x), g = x * y, g2 = 0.5 * y;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const double e = fma(-g2, g, 0.5);
+        g2 = fma(g2, e, g2);
+        g = fma(g, e, g);
+    }
+    *h = g2;
+    *s = fma(fma(-g, g, x), g2, g);
+}
+
+// sin and cos of k r: quarter turns n = rint(k r 2/pi) are taken off with k
+// 2/pi as an unevaluated sum kq + kl (fused multiply-adds, so the reduced
+// angle keeps k r's full precision), then Taylor polynomials on [-pi/4, pi/4]
+// (first dropped term below 2e-9 in FP32, 5e-17 in FP64).  For angles below
+// 2^22 (FP32) and 2^31 (FP64) quarter turns; r may have either sign.
+__device__ __forceinline__ void sincos_kr(float r, float kq, float kl, float *s, float *c) {
+    const float n = rintf(r * kq);
+    const float x = fmaf(r, kl, fmaf(r, kq, -n)) * 1.57079632679489662f, z = x * x;
+    const float sn = fmaf(x * z, fmaf(z, fmaf(z, fmaf(z, 1.f / 362880, -1.f / 5040), 1.f / 120), -1.f / 6), x);
+    const float cs =
+        fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, -1.f / 3628800, 1.f / 40320), -1.f / 720), 1.f / 24), -0.5f), 1.f);
+    const int q = (int)n;
+    const float a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
+    *s = __int_as_float(__float_as_int(a) ^ ((q & 2) << 30));
+    *c = __int_as_float(__float_as_int(b) ^ (((q + 1) & 2) << 30));
+}
+__device__ __forceinline__ void sincos_kr(double r, double kq, double kl, double *s, double *c) {
+    const double n = rint(r * kq);
+    // pi/2 = 1.5707963267948966 + 6.123233995736766e-17
+    const double f = fma(r, kl, fma(r, kq, -n));
+    const double x = fma(f, 1.5707963267948966, f * 6.123233995736766e-17), z = x * x;
+    double p = 1.0 / 1307674368000.0 * -1.0;
+    p = fma(z, p, 1.0 / 6227020800.0);
+    p = fma(z, p, -1.0 / 39916800.0);
+    p = fma(z, p, 1.0 / 362880.0);
+    p = fma(z, p, -1.0 / 5040.0);
+    p = fma(z, p, 1.0 / 120.0);
+    p = fma(z, p, -1.0 / 6.0);
+    const double sn = fma(x * z, p, x);
+    double u = 1.0 / 20922789888000.0;
+    u = fma(z, u, -1.0 / 87178291200.0);
+    u = fma(z, u, 1.0 / 479001600.0);
+    u = fma(z, u, -1.0 / 3628800.0);
+    u = fma(z, u, 1.0 / 40320.0);
+    u = fma(z, u, -1.0 / 720.0);
+    u = fma(z, u, 1.0 / 24.0);
+    u = fma(z, u, -0.5);
+    const double cs = fma(z, u, 1.0);
+    const int q = (int)n;
+    const double a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
+    *s = (q & 2) ? -a : a;
+    *c = ((q + 1) & 2) ? -b : b;
+}
+
+// k 2/pi in two parts of R, the factors of sincos_kr
+template <typename R>
+inline void quarter_turns(double k, R *kq, R *kl) {
+    const long double q = (long double)k * 2.0L / 3.14159265358979323846264338327950288L;
+    *kq = (R)q;
+    *kl = (R)(q - (long double)*kq);
+}
+
 struct d3 {
     double x, y, z;
 };

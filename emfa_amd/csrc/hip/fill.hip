@@ -23,75 +23,6 @@
 namespace emfa {
 
 // ---------------------------------------------------------------------------
-// Elementary functions of the pair kernel.
-// ---------------------------------------------------------------------------
-// s = sqrt(x), h = 1 / (2 sqrt(x)) for x > 0: the hardware reciprocal root and
-// Goldschmidt steps (s <- s + s e, h <- h + h e, e = 1/2 - h s), then one
-// residual correction of s.
-__device__ __forceinline__ void root(float x, float *s, float *h) {
-    const float y = __builtin_amdgcn_rsqf(x), g = x * y, g2 = 0.5f * y;
-    const float e = fmaf(-g2, g, 0.5f);
-    *h = fmaf(g2, e, g2);
-    const float r = fmaf(g, e, g);
-    *s = fmaf(fmaf(-r, r, x), *h, r);
-}
-__device__ __forceinline__ void root(double x, double *s, double *h) {
-    double y = __builtin_amdgcn_rsq(x), g = x * y, g2 = 0.5 * y;
-#pragma unroll
-    for (int it = 0; it < 2; ++it) {
-        const double e = fma(-g2, g, 0.5);
-        g2 = fma(g2, e, g2);
-        g = fma(g, e, g);
-    }
-    *h = g2;
-    *s = fma(fma(-g, g, x), g2, g);
-}
-
-// sin and cos of k r: quarter turns n = rint(k r 2/pi) are taken off with k
-// 2/pi as an unevaluated sum kq + kl (fused multiply-adds, so the reduced
-// angle keeps k r's full precision), then Taylor polynomials on [-pi/4, pi/4]
-// (first dropped term below 2e-9 in FP32, 5e-17 in FP64).  For angles below
-// 2^22 (FP32) and 2^31 (FP64) quarter turns.
-__device__ __forceinline__ void sincos_kr(float r, float kq, float kl, float *s, float *c) {
-    const float n = rintf(r * kq);
-    const float x = fmaf(r, kl, fmaf(r, kq, -n)) * 1.57079632679489662f, z = x * x;
-    const float sn = fmaf(x * z, fmaf(z, fmaf(z, fmaf(z, 1.f / 362880, -1.f / 5040), 1.f / 120), -1.f / 6), x);
-    const float cs =
-        fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, -1.f / 3628800, 1.f / 40320), -1.f / 720), 1.f / 24), -0.5f), 1.f);
-    const int q = (int)n;
-    const float a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
-    *s = __int_as_float(__float_as_int(a) ^ ((q & 2) << 30));
-    *c = __int_as_float(__float_as_int(b) ^ (((q + 1) & 2) << 30));
-}
-__device__ __forceinline__ void sincos_kr(double r, double kq, double kl, double *s, double *c) {
-    const double n = rint(r * kq);
-    // pi/2 = 1.5707963267948966 + 6.123233995736766e-17
-    const double f = fma(r, kl, fma(r, kq, -n));
-    const double x = fma(f, 1.5707963267948966, f * 6.123233995736766e-17), z = x * x;
-    double p = 1.0 / 1307674368000.0 * -1.0;
-    p = fma(z, p, 1.0 / 6227020800.0);
-    p = fma(z, p, -1.0 / 39916800.0);
-    p = fma(z, p, 1.0 / 362880.0);
-    p = fma(z, p, -1.0 / 5040.0);
-    p = fma(z, p, 1.0 / 120.0);
-    p = fma(z, p, -1.0 / 6.0);
-    const double sn = fma(x * z, p, x);
-    double u = 1.0 / 20922789888000.0;
-    u = fma(z, u, -1.0 / 87178291200.0);
-    u = fma(z, u, 1.0 / 479001600.0);
-    u = fma(z, u, -1.0 / 3628800.0);
-    u = fma(z, u, 1.0 / 40320.0);
-    u = fma(z, u, -1.0 / 720.0);
-    u = fma(z, u, 1.0 / 24.0);
-    u = fma(z, u, -0.5);
-    const double cs = fma(z, u, 1.0);
-    const int q = (int)n;
-    const double a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
-    *s = (q & 2) ? -a : a;
-    *c = ((q + 1) & 2) ? -b : b;
-}
-
-// ---------------------------------------------------------------------------
 // K1: regular triangle pairs.
 //   KIND 0 (EFIE):  Ztri = cE * sum w (1/4 rho_f.rho_s - 1/k^2) G
 //   KIND 1 (CFIE):  Ztri = cE * (same) + cM * sum w rho_f.(n_f x (u x rho_s)) (1+jkR) G/R^2
@@ -488,9 +419,8 @@ static emfa_status fill_impl(emfa_ctx *ctx, const emfa_mesh *M, const emfa_fill_
         cM = (R)((1.0 - p->alpha) * kZ0 / (16.0 * kPi));
     }
     const R kr = (R)k, ik2 = (R)(1.0 / (k * k));
-    // k 2/pi in two parts of R
-    const long double kq2 = (long double)k * 2.0L / 3.14159265358979323846264338327950288L;
-    const R kq = (R)kq2, kl = (R)(kq2 - (long double)kq);
+    R kq, kl;
+    quarter_turns(k, &kq, &kl);
     {
         constexpr int per7 = 64 / 8, per3 = 64 / 4;  // triangles per workgroup
         if (p->quad == 7)
