@@ -10,15 +10,86 @@
 
 namespace emfa {
 
+struct tri_abs {
+    double v[3][3];
+    double n[3];
+};
+
+__device__ __forceinline__ void load_tri(const double *__restrict__ tg, int T, int t, tri_abs *o) {
+    for (int i = 0; i < 3; ++i)
+        for (int c = 0; c < 3; ++c) o->v[i][c] = tg[(size_t)c * T + t] + tg[(size_t)(3 + 3 * i + c) * T + t];
+    for (int c = 0; c < 3; ++c) o->n[c] = tg[(size_t)(12 + c) * T + t];
+}
+
 // V(u, j) = 1/2 l_u sum_{+,-} sum_a w_a rho . [alpha e + (1-alpha) n x h] exp(-jk k.r)
 // EFIE (kind 0): 7-point rule, e only (EMSolver/EFIE.cpp:568-601,698-722).
 // CFIE (kind 1): 3-point rule (EMSolver/Miscellaneous.cpp:152-189).
 // MFIE (kind 2): 7-point rule, n x h part only (EMSolver/MFIE.cpp:289-322,
 // 435-436 without its 1/Z0, matching the Z0-scaled MFIE operator of the fill).
-// One thread per u and JB consecutive j (the points and rho are formed once for
-// them), j fastest so the row-major writes coalesce.  VALU-bound: Q sines and
-// cosines per side and value.  7680 unknowns x 181 CFIE
-// columns: 72 -> 36 us against one thread per value and the library sincos.
+//
+// Few values: one thread per (u, j), j fastest so the row-major writes coalesce.
+// A launch's latency either way (122880 x 1 columns 15 us, 10 as k_rhs with one
+// column per thread); it keeps the library's sincos and absolute points, and so
+// the bits that an iterative solver's step count can hang on.
+template <typename R>
+__global__ __launch_bounds__(256) void k_rhs_few(const double *__restrict__ tg, const int *__restrict__ rtp,
+                                             const int *__restrict__ rtm, const int *__restrict__ rap,
+                                             const int *__restrict__ ram, const double *__restrict__ rlen, int T,
+                                             int N, int nrhs, const double *__restrict__ inc, int kind, double k,
+                                             double alpha, cx<R> *__restrict__ B) {
+    long long id = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (id >= (long long)N * nrhs) return;
+    int u = (int)(id / nrhs), j = (int)(id % nrhs);
+    const double *c = inc + 9 * j;
+    double kv[3] = {c[0], c[1], c[2]}, ev[3] = {c[3], c[4], c[5]}, hv[3] = {c[6], c[7], c[8]};
+    double vr = 0, vi = 0, mr = 0, mi = 0;
+    for (int side = 0; side < 2; ++side) {
+        int t = side == 0 ? rtp[u] : rtm[u];
+        int a = side == 0 ? rap[u] : ram[u];
+        tri_abs ta;
+        load_tri(tg, T, t, &ta);
+        double sg = side == 0 ? 1.0 : -1.0;
+        double nxh[3] = {ta.n[1] * hv[2] - ta.n[2] * hv[1], ta.n[2] * hv[0] - ta.n[0] * hv[2],
+                         ta.n[0] * hv[1] - ta.n[1] * hv[0]};
+        int Q = kind == EMFA_CFIE ? 3 : 7;
+        for (int p = 0; p < Q; ++p) {
+            const double *rw = Q == 7 ? c_rule7[p] : c_rule3[p];
+            double r[3];
+            for (int cc = 0; cc < 3; ++cc) r[cc] = rw[0] * ta.v[0][cc] + rw[1] * ta.v[1][cc] + rw[2] * ta.v[2][cc];
+            double rho[3];
+            for (int cc = 0; cc < 3; ++cc) rho[cc] = sg * (r[cc] - ta.v[a][cc]);
+            double ph = k * (r[0] * kv[0] + r[1] * kv[1] + r[2] * kv[2]);
+            double s, co;
+            sincos(ph, &s, &co);
+            double w = rw[3];
+            double de = rho[0] * ev[0] + rho[1] * ev[1] + rho[2] * ev[2];
+            vr += w * de * co;
+            vi -= w * de * s;
+            if (kind != EMFA_EFIE) {
+                double dm = rho[0] * nxh[0] + rho[1] * nxh[1] + rho[2] * nxh[2];
+                mr += w * dm * co;
+                mi -= w * dm * s;
+            }
+        }
+    }
+    double outr, outi;
+    if (kind == EMFA_EFIE) {
+        outr = vr;
+        outi = vi;
+    } else if (kind == EMFA_MFIE) {
+        outr = mr;
+        outi = mi;
+    } else {
+        outr = alpha * vr + (1.0 - alpha) * mr;
+        outi = alpha * vi + (1.0 - alpha) * mi;
+    }
+    double h = 0.5 * rlen[u];
+    B[(size_t)u * nrhs + j] = {(R)(h * outr), (R)(h * outi)};
+}
+
+// Many values: one thread per u and JB consecutive j, for which the points and
+// rho are formed once.  VALU-bound: Q sines and cosines per side and value.  7680
+// unknowns x 181 CFIE columns: 72 -> 36 us against k_rhs_few.
 template <typename R, int Q, int JB>
 __global__ __launch_bounds__(256) void k_rhs(const double *__restrict__ tg, const int *__restrict__ rtp,
                                              const int *__restrict__ rtm, const int *__restrict__ rap,
@@ -261,13 +332,22 @@ extern "C" emfa_status emfa_rhs_fill(emfa_ctx *ctx, const emfa_mesh *M, int kind
         };
         using std::integral_constant;
         // four columns per thread once that still gives every CU eight waves
-        const bool wide = (long long)M->n * nrhs >= 4LL * 512 * ctx->num_cu;
-        if (kind == EMFA_CFIE)
-            wide ? go(integral_constant<int, 3>{}, integral_constant<int, 4>{})
-                 : go(integral_constant<int, 3>{}, integral_constant<int, 1>{});
-        else
-            wide ? go(integral_constant<int, 7>{}, integral_constant<int, 4>{})
-                 : go(integral_constant<int, 7>{}, integral_constant<int, 1>{});
+        if ((long long)M->n * nrhs >= 4LL * 512 * ctx->num_cu) {
+            if (kind == EMFA_CFIE)
+                go(integral_constant<int, 3>{}, integral_constant<int, 4>{});
+            else
+                go(integral_constant<int, 7>{}, integral_constant<int, 4>{});
+        } else {
+            const unsigned blocks = (unsigned)(((long long)M->n * nrhs + 255) / 256);
+            if (B->prec == EMFA_F32)
+                k_rhs_few<float><<<blocks, 256, 0, ctx->stream>>>(M->tg64, M->rtp, M->rtm, M->rap, M->ram, M->rlen64,
+                                                                  M->nt, M->n, nrhs, (const double *)dinc, kind, k,
+                                                                  alpha, (cx<float> *)B->d);
+            else
+                k_rhs_few<double><<<blocks, 256, 0, ctx->stream>>>(M->tg64, M->rtp, M->rtm, M->rap, M->ram, M->rlen64,
+                                                                   M->nt, M->n, nrhs, (const double *)dinc, kind, k,
+                                                                   alpha, (cx<double> *)B->d);
+        }
     }
     hipError_t e = hipGetLastError();
     (void)hipStreamSynchronize(ctx->stream);
