@@ -56,11 +56,14 @@ struct MlLevel {
     cf *trans = nullptr;  // 343 x K
     int *far_ptr_d = nullptr, *far_idx_d = nullptr, *far_code_d = nullptr;
     int *ch_ptr_d = nullptr, *ch_idx_d = nullptr, *oct_d = nullptr, *parent_d = nullptr;
-    int *ip_col = nullptr;  // interpolation from the child level: K x 9
+    int *ip_col = nullptr;  // interpolation from the child level: 9 x K
     float *ip_w = nullptr;
     cf *ph = nullptr;       // 8 x K: exp(-j k khat.(c_parent - c_child)) per child octant
-    int *an_ptr = nullptr, *an_kp = nullptr;  // anterpolation from the parent level
-    float *an_w = nullptr;
+    // anterpolation from the parent level: terms per sample, parent sample of
+    // term j [an_terms][K], weight times conjugate phase [8][an_terms][K]
+    int an_terms = 0;
+    int *an_cnt = nullptr, *an_kp = nullptr;
+    cf *an_f = nullptr;
     int *ubeg_d = nullptr, *uend_d = nullptr;  // leaf level: unknown ranges (box order)
     int *near_ptr_d = nullptr, *near_idx_d = nullptr, *ix_d = nullptr;
 };
@@ -457,22 +460,36 @@ __global__ __launch_bounds__(256) void k_ml_agg(const int *__restrict__ ubeg, co
     for (int c = 0; c < NC; ++c) o[c] = a[c];
 }
 
+// The box and 64-sample chunk of a workgroup of one wave.  The dispatcher hands
+// workgroup i to XCD i % 8, and each XCD has its own L2: consecutive boxes (octree
+// order, so neighbours) go to one XCD, whose L2 then holds the patterns that
+// their far lists share.  Box and chunk are scalars, and with them every list
+// entry and base address.
+__device__ __forceinline__ void box_chunk(int chunks, int *b, int *chunk) {
+    const int n = (int)gridDim.x, xcd = (int)blockIdx.x & 7, q = n >> 3, r = n & 7;
+    const int t = xcd * q + min(xcd, r) + ((int)blockIdx.x >> 3);
+    *b = t / chunks;
+    *chunk = t - *b * chunks;
+}
+
 // upward: up_p[q] = sum_children ph[oct][q] * sum_9 w * up_c[col]; U children
-// per loop step with their loads issued together (sums in child order)
+// per loop step with their loads issued together (sums in child order); the
+// interpolation's columns and weights are stored term by term, [9][K]
 template <int NC, int U>
-__global__ __launch_bounds__(256) void k_ml_up(const int *__restrict__ ch_ptr, const int *__restrict__ ch_idx,
-                                               const int *__restrict__ ch_oct, const int *__restrict__ ip_col,
-                                               const float *__restrict__ ip_w, const cf *__restrict__ ph, int K,
-                                               int Kc, int nbox, const cf *__restrict__ upc, cf *__restrict__ upp) {
-    const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-    const int p = (int)(idx / K), q = (int)(idx % K);
-    if (p >= nbox) return;
+__global__ __launch_bounds__(64) void k_ml_up(const int *__restrict__ ch_ptr, const int *__restrict__ ch_idx,
+                                              const int *__restrict__ ch_oct, const int *__restrict__ ip_col,
+                                              const float *__restrict__ ip_w, const cf *__restrict__ ph, int K,
+                                              int Kc, const cf *__restrict__ upc, cf *__restrict__ upp) {
+    int p, chunk;
+    box_chunk((K + 63) / 64, &p, &chunk);
+    const int q = chunk * 64 + threadIdx.x;
+    if (q >= K) return;
     int cols[9];
     float ws[9];
 #pragma unroll
     for (int j = 0; j < 9; ++j) {
-        cols[j] = ip_col[q * 9 + j];
-        ws[j] = ip_w[q * 9 + j];
+        cols[j] = ip_col[j * K + q];
+        ws[j] = ip_w[j * K + q];
     }
     cf a[NC];
 #pragma unroll
@@ -515,20 +532,27 @@ __global__ __launch_bounds__(256) void k_ml_up(const int *__restrict__ ch_ptr, c
 
 // downward at one level: translation from far boxes + anterpolation from the
 // parent.  U > 1 takes the far list and the anterpolation list U entries at a
-// time, their indices and operands loaded before the U products, so that U
-// gathers are in flight per thread instead of one; the sums run in the same
-// order for every U (the results are bitwise those of U = 1).
+// time, their operands loaded before the U products, so that U gathers are in
+// flight per thread instead of one; the sums run in the same order for every U
+// (the results are bitwise those of U = 1).  Anterpolation terms are stored term
+// by term: term j of sample q at [j][q], its parent sample in an_kp and, per
+// octant, its weight times the conjugate phase in an_f, so that 64 lanes read
+// runs (as a list per sample each lane's entry was a line of its own).  Bound by
+// L2 traffic and latency: 160 -> 127 us per level at 122880 unknowns, 67 -> 51 us
+// on the 70272-unknown IP-SIE cube, with vector lists and boxes round-robin over
+// the XCDs before.
 template <int NC, int U>
-__global__ __launch_bounds__(256) void k_ml_down(const int *__restrict__ far_ptr, const int *__restrict__ far_idx,
-                                                 const int *__restrict__ far_code, const cf *__restrict__ trans,
-                                                 const cf *__restrict__ up, int K, const int *__restrict__ parent,
-                                                 const int *__restrict__ oct, const int *__restrict__ an_ptr,
-                                                 const int *__restrict__ an_kp, const float *__restrict__ an_w,
-                                                 const cf *__restrict__ php, int Kp, const cf *__restrict__ downp,
-                                                 int nbox, cf *__restrict__ down) {
-    const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
-    const int b = (int)(idx / K), q = (int)(idx % K);
-    if (b >= nbox) return;
+__global__ __launch_bounds__(64) void k_ml_down(const int *__restrict__ far_ptr, const int *__restrict__ far_idx,
+                                                const int *__restrict__ far_code, const cf *__restrict__ trans,
+                                                const cf *__restrict__ up, int K, const int *__restrict__ parent,
+                                                const int *__restrict__ oct, const int *__restrict__ an_cnt,
+                                                const int *__restrict__ an_kp, const cf *__restrict__ an_f,
+                                                int an_terms, int Kp, const cf *__restrict__ downp,
+                                                cf *__restrict__ down) {
+    int b, chunk;
+    box_chunk((K + 63) / 64, &b, &chunk);
+    const int q = chunk * 64 + threadIdx.x;
+    if (q >= K) return;
     cf a[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) a[c] = {0, 0};
@@ -561,37 +585,31 @@ __global__ __launch_bounds__(256) void k_ml_down(const int *__restrict__ far_ptr
         for (int c = 0; c < NC; ++c) a[c] = cfma(a[c], t, u[c]);
     }
     if (downp) {
-        const int p = parent[b], o = oct[b];
-        const cf *dp = downp + (size_t)p * Kp * NC;
-        const cf *phase = php + (size_t)o * Kp;
-        int g = an_ptr[q];
-        const int g_end = an_ptr[q + 1];
-        for (; g + U <= g_end; g += U) {
+        const cf *dp = downp + (size_t)parent[b] * Kp * NC;
+        const cf *fo = an_f + (size_t)oct[b] * an_terms * K + q;
+        const int *ko = an_kp + q;
+        const int cnt = an_cnt[q];
+        int g = 0;
+        for (; g + U <= cnt; g += U) {
             int kp[U];
-            float w[U];
-#pragma unroll
-            for (int j = 0; j < U; ++j) {
-                kp[j] = an_kp[g + j];
-                w[j] = an_w[g + j];
-            }
             cf f[U], v[U][NC];
 #pragma unroll
             for (int j = 0; j < U; ++j) {
-                const cf f0 = phase[kp[j]];
-                f[j] = {w[j] * f0.re, -w[j] * f0.im};  // conj: exp(+j k khat.(c_p - c_b))
+                kp[j] = ko[(size_t)(g + j) * K];
+                f[j] = fo[(size_t)(g + j) * K];
+            }
+#pragma unroll
+            for (int j = 0; j < U; ++j)
 #pragma unroll
                 for (int c = 0; c < NC; ++c) v[j][c] = dp[(size_t)kp[j] * NC + c];
-            }
 #pragma unroll
             for (int j = 0; j < U; ++j)
 #pragma unroll
                 for (int c = 0; c < NC; ++c) a[c] = cfma(a[c], f[j], v[j][c]);
         }
-        for (; g < g_end; ++g) {
-            const int kq = an_kp[g];
-            const cf f0 = phase[kq];
-            const cf f = {an_w[g] * f0.re, -an_w[g] * f0.im};
-            const cf *v = dp + (size_t)kq * NC;
+        for (; g < cnt; ++g) {
+            const cf f = fo[(size_t)g * K];
+            const cf *v = dp + (size_t)ko[(size_t)g * K] * NC;
 #pragma unroll
             for (int c = 0; c < NC; ++c) a[c] = cfma(a[c], f, v[c]);
         }
@@ -609,8 +627,8 @@ __global__ __launch_bounds__(256) void k_ml_down(const int *__restrict__ far_ptr
 __global__ __launch_bounds__(256) void k_ml_down_sib(
     const int *__restrict__ pnear_ptr, const int *__restrict__ pnear_idx, const int *__restrict__ pch_ptr,
     const int *__restrict__ pch_idx, int nparent, const int *__restrict__ ix, const int *__restrict__ oct,
-    const cf *__restrict__ trans, const cf *__restrict__ up, int K, const int *__restrict__ an_ptr,
-    const int *__restrict__ an_kp, const float *__restrict__ an_w, const cf *__restrict__ php, int Kp,
+    const cf *__restrict__ trans, const cf *__restrict__ up, int K, const int *__restrict__ an_cnt,
+    const int *__restrict__ an_kp, const cf *__restrict__ an_f, int an_terms, int Kp,
     const cf *__restrict__ downp, cf *__restrict__ down) {
     const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
     const int P = (int)(idx / K), q = (int)(idx % K);
@@ -652,10 +670,9 @@ __global__ __launch_bounds__(256) void k_ml_down_sib(
         if (s >= nch) break;
         const int b = pch_idx[c0 + s], o = oct[b];
         cf a0 = a[s][0], a1 = a[s][1], a2 = a[s][2];
-        for (int e = an_ptr[q]; e < an_ptr[q + 1]; ++e) {
-            const int kp = an_kp[e];
-            const cf f0 = php[o * Kp + kp];
-            const cf f = {an_w[e] * f0.re, -an_w[e] * f0.im};
+        for (int e = 0; e < an_cnt[q]; ++e) {
+            const int kp = an_kp[(size_t)e * K + q];
+            const cf f = an_f[((size_t)o * an_terms + e) * K + q];
             const cf *v = dp + (size_t)kp * 3;
             a0 = cfma(a0, f, v[0]);
             a1 = cfma(a1, f, v[1]);
@@ -1270,8 +1287,8 @@ static emfa_status ml_tree(emfa_ctx *ctx, const emfa_mesh *mesh, const emfa_mlfm
                         for (int ib = 0; ib < 3; ++ib, ++j) {
                             const int colc = ploc[3 * p + ia] * N.L + tloc[3 * t + ib];
                             const double w = pel[3 * p + ia] * tel[3 * t + ib];
-                            ipc[(size_t)q * 9 + j] = colc;
-                            ipw[(size_t)q * 9 + j] = (float)w;
+                            ipc[(size_t)j * C.K + q] = colc;
+                            ipw[(size_t)j * C.K + q] = (float)w;
                             tr_list[colc].push_back({q, w * C.W[q] / N.W[colc]});
                         }
                 }
@@ -1289,19 +1306,32 @@ static emfa_status ml_tree(emfa_ctx *ctx, const emfa_mesh *mesh, const emfa_mlfm
             std::vector<int> chp(C.ch_ptr), chi(C.ch_idx);
             ML_TRY(ml_upload(M, &C.ch_ptr_d, chp));
             ML_TRY(ml_upload(M, &C.ch_idx_d, chi.empty() ? std::vector<int>{0} : chi));
-            // anterpolation into level l+1 (transpose, weighted by the quadrature weights)
-            std::vector<int> anp(N.K + 1, 0), ank;
-            std::vector<float> anw;
+            // anterpolation into level l+1 (transpose, weighted by the quadrature
+            // weights): term j of sample qc at [j][qc], per octant with the phase
+            std::vector<int> ancnt(N.K);
+            N.an_terms = 0;
             for (int qc = 0; qc < N.K; ++qc) {
-                for (auto &e : tr_list[qc]) {
-                    ank.push_back(e.first);
-                    anw.push_back((float)e.second);
-                }
-                anp[qc + 1] = (int)ank.size();
+                ancnt[qc] = (int)tr_list[qc].size();
+                N.an_terms = std::max(N.an_terms, ancnt[qc]);
             }
-            ML_TRY(ml_upload(M, &N.an_ptr, anp));
+            const size_t J = (size_t)std::max(1, N.an_terms);
+            std::vector<int> ank(J * N.K, 0);
+            std::vector<cf> anf(8 * J * N.K, cf{0, 0});
+            for (int qc = 0; qc < N.K; ++qc)
+                for (int j = 0; j < ancnt[qc]; ++j) {
+                    const int kq = tr_list[qc][j].first;
+                    const float w = (float)tr_list[qc][j].second;
+                    ank[(size_t)j * N.K + qc] = kq;
+                    for (int o = 0; o < 8; ++o) {
+                        const cf f0 = ph[(size_t)o * C.K + kq];
+                        // conj: exp(+j k khat.(c_p - c_b))
+                        anf[((size_t)o * J + j) * N.K + qc] = {w * f0.re, -w * f0.im};
+                    }
+                }
+            N.an_terms = (int)J;
+            ML_TRY(ml_upload(M, &N.an_cnt, ancnt));
             ML_TRY(ml_upload(M, &N.an_kp, ank));
-            ML_TRY(ml_upload(M, &N.an_w, anw));
+            ML_TRY(ml_upload(M, &N.an_f, anf));
         }
     }
     *Mout = M;
@@ -1716,10 +1746,9 @@ static emfa_status ml_apply(emfa_ctx *ctx, emfa_mlfma *M, const double2 *x, doub
     for (int l = lvl - 1; l >= 2; --l) {
         MlLevel &C = M->lv[l], &N = M->lv[l + 1];
         ProfScope ps(ctx, "mlfma_up", 0);
-        const unsigned g = (unsigned)(((long long)C.nbox * C.K + 255) / 256);
-#define ML_UP(NC, U)                                                                                               \
-    k_ml_up<NC, U><<<g, 256, 0, s>>>(C.ch_ptr_d, C.ch_idx_d, N.oct_d, C.ip_col, C.ip_w, C.ph, C.K, N.K, C.nbox, N.up, \
-                                     C.up)
+        const unsigned g = (unsigned)C.nbox * ((C.K + 63) / 64);
+#define ML_UP(NC, U) \
+    k_ml_up<NC, U><<<g, 64, 0, s>>>(C.ch_ptr_d, C.ch_idx_d, N.oct_d, C.ip_col, C.ip_w, C.ph, C.K, N.K, N.up, C.up)
         if (M->nc == 4) {
             if (unroll == 4)
                 ML_UP(4, 2);
@@ -1754,14 +1783,14 @@ static emfa_status ml_apply(emfa_ctx *ctx, emfa_mlfma *M, const double2 *x, doub
         if (P && sib) {
             k_ml_down_sib<<<(unsigned)(((long long)P->nbox * C.K + 255) / 256), 256, 0, s>>>(
                 P->near_ptr_d, P->near_idx_d, P->ch_ptr_d, P->ch_idx_d, P->nbox, C.ix_d, C.oct_d, C.trans, C.up,
-                C.K, C.an_ptr, C.an_kp, C.an_w, P->ph, P->K, P->down, C.down);
+                C.K, C.an_cnt, C.an_kp, C.an_f, C.an_terms, P->K, P->down, C.down);
             continue;
         }
-        const unsigned g = (unsigned)(((long long)C.nbox * C.K + 255) / 256);
-#define ML_DOWN(NC, U)                                                                                            \
-    k_ml_down<NC, U><<<g, 256, 0, s>>>(C.far_ptr_d, C.far_idx_d, C.far_code_d, C.trans, C.up, C.K, C.parent_d,     \
-                                       C.oct_d, C.an_ptr, C.an_kp, C.an_w, P ? P->ph : nullptr, P ? P->K : 0,      \
-                                       P ? P->down : nullptr, C.nbox, C.down)
+        const unsigned g = (unsigned)C.nbox * ((C.K + 63) / 64);
+#define ML_DOWN(NC, U)                                                                                             \
+    k_ml_down<NC, U><<<g, 64, 0, s>>>(C.far_ptr_d, C.far_idx_d, C.far_code_d, C.trans, C.up, C.K, C.parent_d,       \
+                                      C.oct_d, C.an_cnt, C.an_kp, C.an_f, C.an_terms, P ? P->K : 0,                \
+                                      P ? P->down : nullptr, C.down)
         if (M->nc == 4) {
             if (down_unroll == 4)
                 ML_DOWN(4, 4);
