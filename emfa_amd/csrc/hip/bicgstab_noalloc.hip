@@ -56,8 +56,11 @@ extern "C" emfa_status emfa_bicgstab_noalloc(emfa_ctx *ctx, const emfa_mat *Z, c
     void *ptr = nullptr;
     emfa_status st = device_scratch(ctx->device, &ptr);
     if (st) return st;
+    int group = kGemvCols;
+    while (group > 1 && bicgstab_work_bytes(n, group) > kNoAllocScratchBytes) --group;
     return bicgstab_impl(
-        ctx, n, [&](const double2 *in, double2 *out) { return gemv(ctx, Z, in, out); }, B, X, tol, max_iter, variant,
-        rep, ptr, kNoAllocScratchBytes);
+        ctx, n,
+        [&](int nc, const double2 *const *in, double2 *const *out) { return gemv(ctx, Z, nc, in, out); }, B, X, tol,
+        max_iter, variant, rep, group, ptr, kNoAllocScratchBytes);
 }
 

@@ -9,32 +9,70 @@
 #include <cmath>
 #include <complex>
 #include <functional>
+#include <type_traits>
 #include <vector>
 
 #include "internal.h"
 
 namespace emfa {
 
-// y = Z x, one wavefront per row, FP64 accumulation
-template <typename TA>
-__global__ __launch_bounds__(256) void k_gemv(const cx<TA> *__restrict__ Z, int n, const double2 *__restrict__ x,
-                                              double2 *__restrict__ y) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+// y_c = Z x_c for NC vectors, R rows per wavefront, FP64 accumulation.  Every
+// vector element is 16 bytes against 8 of an FP32 matrix element: with one row
+// per wave the vectors' trips from L2, not the matrix's from HBM, bound the
+// product, so R rows share them, and NC vectors share the matrix.  A row's sum
+// runs over its lanes and elements in the same order, with the same fused
+// operations, for every R and NC: a column's result does not depend on its group.
+// A step's share of a solve in us, one row a wave and one vector at a time
+// against this, FP32: 12288 unknowns 341 and 243 for one vector, 681 and 256 for
+// two, 1286 and 316 for four; FP64 474 and 445, 945 and 470, 1786 and 468.
+// Unrolling by four gains 4 to 8 % at most sizes and loses 4 % at 4096 unknowns
+// in FP64, where the matrix just misses the last cache.
+template <int NC>
+struct GemvCols {
+    const double2 *x[NC];
+    double2 *y[NC];
+};
+
+template <typename TA, int R, int NC>
+__global__ __launch_bounds__(256) void k_gemv(const cx<TA> *__restrict__ Z, int n, GemvCols<NC> v) {
+    const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
     const int lane = threadIdx.x & 63;
     if (row >= n) return;
-    const cx<TA> *zr = Z + (size_t)row * n;
-    double sr = 0, si = 0;
+    const cx<TA> *zr[R];
+    double sr[R][NC], si[R][NC];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        zr[i] = Z + (size_t)min(row + i, n - 1) * n;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) sr[i][c] = si[i][c] = 0;
+    }
+#pragma unroll 4
     for (int j = lane; j < n; j += 64) {
-        cx<TA> a = zr[j];
-        double2 b = x[j];
-        sr += (double)a.re * b.x - (double)a.im * b.y;
-        si += (double)a.re * b.y + (double)a.im * b.x;
+        cx<TA> a[R];
+        double2 b[NC];
+#pragma unroll
+        for (int i = 0; i < R; ++i) a[i] = zr[i][j];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) b[c] = v.x[c][j];
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const double ar = a[i].re, ai = a[i].im;
+                sr[i][c] = fma(-ai, b[c].y, fma(ar, b[c].x, sr[i][c]));
+                si[i][c] = fma(ai, b[c].x, fma(ar, b[c].y, si[i][c]));
+            }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        sr += __shfl_down(sr, off, 64);
-        si += __shfl_down(si, off, 64);
-    }
-    if (lane == 0) y[row] = make_double2(sr, si);
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            for (int off = 32; off > 0; off >>= 1) {
+                sr[i][c] += __shfl_down(sr[i][c], off, 64);
+                si[i][c] += __shfl_down(si[i][c], off, 64);
+            }
+            if (lane == 0 && row + i < n) v.y[c][row + i] = make_double2(sr[i][c], si[i][c]);
+        }
 }
 
 // Dot products h[i] = V_i^H w for i < k in two deterministic passes:
@@ -269,14 +307,50 @@ emfa_status gmres_impl(emfa_ctx *ctx, int n, const std::function<emfa_status(con
 
 using namespace emfa;
 
-emfa_status emfa::gemv(emfa_ctx *ctx, const emfa_mat *Z, const double2 *in, double2 *out) {
+emfa_status emfa::gemv(emfa_ctx *ctx, const emfa_mat *Z, int nc, const double2 *const *in, double2 *const *out) {
     const int n = Z->rows;
     hipStream_t s = ctx->stream;
+    EMFA_REQUIRE(nc >= 1 && nc <= kGemvCols, EMFA_E_INVALID, "gemv: %d vectors", nc);
     ProfScope ps(ctx, "gmres_matvec", (double)n * n * elem_bytes(Z->prec));
-    if (Z->prec == EMFA_F32)
-        k_gemv<float><<<(n + 3) / 4, 256, 0, s>>>((const cx<float> *)Z->d, n, in, out);
+    // Rows per wave: the fewest (1, 2, 4) whose matrix bytes match the vectors'
+    // per trip, as long as the waves left fill the chip: 7 a CU, and 12 for one
+    // vector, where the chip's latency rather than L2 is short of waves.  Per
+    // product with 1, 2, 4 rows, FP32, two vectors: 56 / 57 / 63 us at 2304
+    // unknowns, 87 / 83 / 86 at 5120, 132 / 109 / 119 at 6144, 416 / 311 / 255 at
+    // 12288 (a whole step's share, launches and read-backs of 40 us included).
+    const int fit = n / ((nc == 1 ? 12 : 7) * std::max(1, ctx->num_cu));
+    int r = 1;
+    while (r < 4 && 2 * r <= fit && r * elem_bytes(Z->prec) < sizeof(double2) * nc) r *= 2;
+    auto go = [&](auto cols) {
+        constexpr int NC = decltype(cols)::value;
+        GemvCols<NC> v;
+        for (int c = 0; c < NC; ++c) {
+            v.x[c] = in[c];
+            v.y[c] = out[c];
+        }
+        auto rows = [&](auto r) {
+            constexpr int R = decltype(r)::value;
+            const int g = (n + 4 * R - 1) / (4 * R);
+            if (Z->prec == EMFA_F32)
+                k_gemv<float, R, NC><<<g, 256, 0, s>>>((const cx<float> *)Z->d, n, v);
+            else
+                k_gemv<double, R, NC><<<g, 256, 0, s>>>((const cx<double> *)Z->d, n, v);
+        };
+        if (r == 4)
+            rows(std::integral_constant<int, 4>{});
+        else if (r == 2)
+            rows(std::integral_constant<int, 2>{});
+        else
+            rows(std::integral_constant<int, 1>{});
+    };
+    if (nc == 1)
+        go(std::integral_constant<int, 1>{});
+    else if (nc == 2)
+        go(std::integral_constant<int, 2>{});
+    else if (nc == 3)
+        go(std::integral_constant<int, 3>{});
     else
-        k_gemv<double><<<(n + 3) / 4, 256, 0, s>>>((const cx<double> *)Z->d, n, in, out);
+        go(std::integral_constant<int, 4>{});
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
 }
@@ -286,6 +360,6 @@ extern "C" emfa_status emfa_gmres(emfa_ctx *ctx, const emfa_mat *Z, const emfa_m
     EMFA_REQUIRE(ctx && Z && B && X, EMFA_E_INVALID, "emfa_gmres: null argument");
     const int n = Z->rows;
     EMFA_REQUIRE(Z->cols == n, EMFA_E_INVALID, "emfa_gmres: Z must be square");
-    auto matvec = [&](const double2 *in, double2 *out) -> emfa_status { return gemv(ctx, Z, in, out); };
+    auto matvec = [&](const double2 *in, double2 *out) -> emfa_status { return gemv(ctx, Z, 1, &in, &out); };
     return gmres_impl(ctx, n, matvec, B, X, m, tol, max_restart, rep);
 }

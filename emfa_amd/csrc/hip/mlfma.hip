@@ -2319,7 +2319,11 @@ emfa_status emfa_mlfma_bicgstab(emfa_ctx *ctx, emfa_mlfma *m, const emfa_mat *B,
                                 int max_iter, int variant, emfa_bicgstab_report *rep) {
     EMFA_REQUIRE(ctx && m && B && X, EMFA_E_INVALID, "emfa_mlfma_bicgstab: null argument");
     EMFA_HIP_CHECK(hipSetDevice(ctx->device));
-    auto op = [&](const double2 *in, double2 *out) -> emfa_status { return ml_apply(ctx, m, in, out); };
+    auto op = [&](int nc, const double2 *const *in, double2 *const *out) -> emfa_status {
+        emfa_status s2 = EMFA_OK;
+        for (int c = 0; c < nc && !s2; ++c) s2 = ml_apply(ctx, m, in[c], out[c]);
+        return s2;
+    };
     emfa_mat *Bp = nullptr;
     emfa_status st = ml_rhs(ctx, m, B, &Bp);
     if (st) return st;
