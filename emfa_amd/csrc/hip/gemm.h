@@ -36,12 +36,14 @@ struct GemmArgs {
     Batch bt;               // FP32 launchers: A and C in the batch's matrices, Bt in its scratch slabs
 };
 
-// Three-term bf16 product from pre-split operand planes.  Each operand is
-// given as two bf16 planes (hi = bf16(x), lo = bf16(x - hi)), row-major with
-// ld elements per row; rows are padded with zeros to a multiple of 256
-// from the given pointer and K to a multiple of 16 (Kp), so the kernel
-// reads whole tiles with no bounds checks.  C (FP32, M x Nr, ldc) gets
-// beta C -/+ (Ah Bh^T + Ah Bl^T + Al Bh^T) on rows < M, columns < Nr.
+// Three-term bf16 product of complex matrices from pre-split operand planes.
+// Each operand is given as two bf16 planes (hi = bf16(x), lo = bf16(x - hi)),
+// row-major with ld elements per row: A's rows as (re, im) pairs along K, B's
+// one row per complex column as (re, -im) pairs.  Rows are padded to a multiple
+// of 256 (A) and 128 (B) from the given pointer and K with zeros to a multiple
+// of 32 (Kp), so the kernel reads whole tiles with no bounds checks.  C (M x
+// Nr FP32, Nr / 2 complex columns, ldc) gets beta C -/+ (Ah Bh + Ah Bl + Al Bh)
+// on rows < M, columns < Nr.
 struct Bf3Planes {
     int M, Nr, Kp;
     const __bf16 *Ah, *Al;
@@ -53,7 +55,6 @@ struct Bf3Planes {
     int alpha_neg, beta;
     int max_wgs = 0;     // > 0: at most this many workgroups (rounded down to a multiple of 8), looping over tiles
     int persistent = 0;  // set by the launcher
-    int kernel = 0;      // 1: k_gemm_bf3p, 2: k_gemm_bf3q, 4: k_gemm_bf3r, 0: EMFA_BF3_KERNEL (p, q) or bf3r
     Batch bt;            // C in the batch's matrices, the planes in its scratch slabs
 };
 

@@ -432,191 +432,69 @@ __global__ __launch_bounds__(256) void k_split_bf16(const float *__restrict__ sr
 }
 
 // ---------------------------------------------------------------------------
-// Three-term bf16 GEMM from pre-split planes (Bf3Planes).  Workgroup tile
-// 256 x 256, 8 waves as 4 x 2 with wave tiles 64 x 128 (2 x 4 MFMA 32x32x16).
-// The operand tiles go straight from global memory into LDS with 16-byte
-// direct loads (global_load_lds_dwordx4: lane l of a wave writes LDS bytes
-// base + 16 l), four stages of K = 16 in flight: stage kt + 3 is issued while
-// stage kt is multiplied.  No registers stage the operands and no VALU work
-// sits in the loop.  An LDS plane row holds 16 bf16 (two 16-byte chunks);
-// chunk c of row r is stored at position c ^ swz(r), swz(r) = bit 2 ^ bit 3
-// of r: the sixteen rows that one ds_read_b128 cycle serves (sixteen lanes,
-// 64 banks of 4 bytes) fall on sixteen distinct 4-bank groups.  (With bit 2
-// alone, rows r and r + 8 shared banks: the counters showed four conflict
-// cycles per LDS read.)
-// Each wave waits (s_waitcnt vmcnt) for its own loads of the stage, then the
-// workgroup barrier publishes every wave's loads; the same barrier tells the
-// issuing waves that all reads of the buffer being refilled are done.
+// Three-term bf16 product from pre-split planes (Bf3Planes), complex columns.
+// A's rows hold (re, im) pairs along K and B's rows the (re, -im) pairs of a
+// complex column: that row, as it is, gives the real part, and with its pairs
+// turned round and their lower signs flipped, (im, re), the imaginary part.  A
+// lane that holds row c of B thus feeds two MFMA column tiles, the real and the
+// imaginary parts of 32 columns, from one fragment, and leaves with whole
+// complex results.
+//
+// Workgroup tile 32 WM MT rows x 32 WN NC complex columns; wave tile 32 MT x 32
+// NC.  K = 32 per stage, two LDS buffers of the four planes.  Each thread loads
+// its 16-byte chunks of the next stage into registers with ordinary loads and
+// stores them to the other buffer.  Fragments of a stage's second K = 16 are
+// read from LDS while the first is multiplied, and those of the next stage's
+// first while the second is: the one barrier per stage, between the two, finds
+// the stores done and every read of the buffer that is filled next.  A row's
+// stage holds 4 chunks; chunk c sits at position c ^ ((r >> 2) & 3), so the
+// sixteen rows one ds_read_b128 cycle serves cover all 64 banks.
+// Per accumulator the products are added as Al Bh, Ah Bl, Ah Bh, K ascending.
+// Against one fragment per real column (16 rather than 24 LDS reads per 24 MFMA
+// and 96 rather than 128 KB of LDS): 8321 unknowns factorised in 18.7 ms from
+// 19.4, 30720 solved in 372 from 390.  What is left beside the MFMA is C: at K
+// 1024 a tile's 0.5 MB take a quarter of the time that its products take.
 // ---------------------------------------------------------------------------
-namespace bf3p {
-constexpr int BM = 256, BN = 256, BK = 16, NS = 4, PLANE = 256 * BK;
+namespace bf3 {
+constexpr int BK = 32;
 }
 
-__device__ __forceinline__ int bf3_swz(int r) { return ((r >> 2) ^ (r >> 3)) & 1; }
-__device__ __forceinline__ int bf3p_off(int r, int kg) { return r * bf3p::BK + ((kg ^ bf3_swz(r)) << 3); }
+__device__ __forceinline__ int bf3_off(int r, int c) { return r * bf3::BK + ((c ^ ((r >> 2) & 3)) << 3); }
 
-typedef __attribute__((address_space(3))) void lds_void;
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(512) void k_gemm_bf3p(Bf3Planes g) {
-    using namespace bf3p;
-    __shared__ __attribute__((aligned(16))) __bf16 sm[NS][4][PLANE];  // stage, plane (Ah Al Bh Bl)
+// the (re, -im) pairs of a fragment as (im, re)
+__device__ __forceinline__ bf16x8 bf3_turn(bf16x8 f) {
+    u32x4 u = __builtin_bit_cast(u32x4, f);
+    u.x = __builtin_amdgcn_alignbit(u.x, u.x, 16) ^ 0x8000u;
+    u.y = __builtin_amdgcn_alignbit(u.y, u.y, 16) ^ 0x8000u;
+    u.z = __builtin_amdgcn_alignbit(u.z, u.z, 16) ^ 0x8000u;
+    u.w = __builtin_amdgcn_alignbit(u.w, u.w, 16) ^ 0x8000u;
+    return __builtin_bit_cast(bf16x8, u);
+}
+
+template <int WM, int WN, int MT, int NC>
+__global__ __launch_bounds__(64 * WM * WN, 2) void k_gemm_bf3(Bf3Planes g) {
+    constexpr int BK = bf3::BK, T = 64 * WM * WN, BM = 32 * WM * MT, BN = 32 * WN * NC;
+    constexpr int CA = BM * 4 / T, CB = BN * 4 / T;  // chunks per thread and plane
+    static_assert(CA * T == BM * 4 && CB * T == BN * 4, "chunks divide among the threads");
+    __shared__ __attribute__((aligned(16))) __bf16 sa[2][2][BM * BK], sb[2][2][BN * BK];  // buffer, plane (hi lo)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int TX = (g.Nr + BN - 1) / BN, TY = (g.M + BM - 1) / BM, TT = TX * TY;
+    const int wm = wave / WN, wn = wave % WN;
+    const int ncols = g.Nr >> 1;
+    const int TX = (ncols + BN - 1) / BN, TY = (g.M + BM - 1) / BM, TT = TX * TY;
     // one tile per workgroup, or (persistent grid) tiles blockIdx.x, + gridDim.x, ...
     // over the tiles of every matrix of the batch (matrix tl / TT)
     const int t0 = g.persistent ? (int)blockIdx.x : (int)((blockIdx.z * TY + blockIdx.y) * gridDim.x + blockIdx.x);
     const int tstep = g.persistent ? (int)gridDim.x : TT * g.bt.count;
-    for (int tl = t0; tl < TT * g.bt.count; tl += tstep) {
-    if (tl != t0) __syncthreads();  // the previous tile's LDS reads are done
-    const int zb = tl / TT;
-    int ty, tx;
-    tile_of_linear(tl - zb * TT, TX, TY, &ty, &tx);
-    const long long bm = (long long)ty * BM, bn = (long long)tx * BN;
-    const int nk = g.Kp / BK;
-
-    // this wave's direct loads: plane pl, rows half * 128 + 32 i + lane / 2
-    const int pl = wave >> 1, half = wave & 1;
-    const __bf16 *src = batch_scr(g.bt, pl == 0 ? g.Ah : pl == 1 ? g.Al : pl == 2 ? g.Bh : g.Bl, zb);
-    const long long ld = pl < 2 ? g.lda : g.ldb;
-    const long long row0 = pl < 2 ? bm : bn;
-    const __bf16 *gp[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = half * 128 + 32 * i + (lane >> 1);
-        const int c = (lane & 1) ^ bf3_swz(r);
-        gp[i] = src + (row0 + r) * ld + 8 * c;
-    }
-    auto issue = [&](int kt) {
-        const int st = kt & (NS - 1);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds((const void *)(gp[i] + (long long)kt * BK),
-                                             (lds_void *)&sm[st][pl][(half * 128 + 32 * i) * BK], 16, 0, 0);
-    };
-
-    floatx16 acc[2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-
-    issue(0);
-    if (nk > 1) issue(1);
-    if (nk > 2) issue(2);
     const int r32 = lane & 31, kg = lane >> 5;
-    for (int kt = 0; kt < nk; ++kt) {
-        // loads of stages kt+1, kt+2 (4 per stage) may stay in flight
-        if (kt + 2 < nk)
-            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else if (kt + 1 < nk)
-            asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (kt + 3 < nk) issue(kt + 3);
-        const int st = kt & (NS - 1);
-        bf16x8 ah[2], al[2], bh[4], bl[4];
+    // this thread's chunks: q = i T + tid, row q >> 2, chunk q & 3 (same in both planes)
+    const int row = tid >> 2;
+    unsigned oa[CA], ob[CB];  // byte offsets in a tile's planes
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            const int o = bf3p_off(wm * 64 + mt * 32 + r32, kg);
-            ah[mt] = *(const bf16x8 *)&sm[st][0][o];
-            al[mt] = *(const bf16x8 *)&sm[st][1][o];
-        }
+    for (int i = 0; i < CA; ++i) oa[i] = 2u * ((i * (T / 4) + row) * (unsigned)g.lda + 8 * (tid & 3));
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            const int o = bf3p_off(wn * 128 + nt * 32 + r32, kg);
-            bh[nt] = *(const bf16x8 *)&sm[st][2][o];
-            bl[nt] = *(const bf16x8 *)&sm[st][3][o];
-        }
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[mt], bh[nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mt], bl[nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mt], bh[nt], acc[mt][nt], 0, 0, 0);
-    }
-
-    // epilogue: all C loads of a 32-row slab are issued before its stores;
-    // tiles wholly inside C skip the per-element bounds checks
-    const float sgn = g.alpha_neg ? -1.f : 1.f;
-    float *__restrict__ C = batch_mat(g.bt, g.C, zb) + (bm + wm * 64 + 4 * (lane >> 5)) * g.ldc + bn + wn * 128 + r32;
-    const int mrem = (int)min((long long)BM, g.M - bm) - wm * 64 - 4 * (lane >> 5);
-    const int nrem = (int)min((long long)BN, (long long)g.Nr - bn) - wn * 128 - r32;
-    const bool full = bm + BM <= g.M && bn + BN <= g.Nr;
-    auto epilogue = [&](auto guarded) {
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            float cv[4][16];
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int i = mt * 32 + 8 * (v >> 2) + (v & 3), j = nt * 32;
-                    const bool in = !guarded.value || (i < mrem && j < nrem);
-                    cv[nt][v] = (g.beta && in) ? C[i * g.ldc + j] : 0.f;
-                }
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int i = mt * 32 + 8 * (v >> 2) + (v & 3), j = nt * 32;
-                    if (!guarded.value || (i < mrem && j < nrem)) C[i * g.ldc + j] = cv[nt][v] + sgn * acc[mt][nt][v];
-                }
-        }
-    };
-    if (full)
-        epilogue(std::false_type{});
-    else
-        epilogue(std::true_type{});
-    }  // tiles
-}
-
-// ---------------------------------------------------------------------------
-// The same product with register-staged operand loads and K = 32 per stage.
-// Workgroup tile 256 x 256, 8 waves of 64 x 128 as in k_gemm_bf3p; two LDS
-// buffers of 4 planes x 256 rows x 32 K (128 KB).  Each thread loads eight
-// 16-byte chunks per stage (two per plane; four threads cover the 64 bytes of
-// a row's stage) into registers with ordinary global loads, and stores them
-// to the other LDS buffer after multiplying the current one; one barrier per
-// stage publishes the stores and frees the buffer just read.  A row's stage
-// holds 4 chunks; chunk c sits at position c ^ ((r >> 2) & 3), so the
-// sixteen rows one ds_read_b128 cycle serves cover all 64 banks.  The K = 16
-// halves of a stage are multiplied in order with bf3p's product order, so the
-// bits equal k_gemm_bf3p's.  Needs Kp % 32 == 0.
-// ---------------------------------------------------------------------------
-namespace bf3r {
-constexpr int BM = 256, BN = 256, BK = 32, PLANE = 256 * BK;
-}
-
-__device__ __forceinline__ int bf3r_off(int r, int c) { return r * bf3r::BK + ((c ^ ((r >> 2) & 3)) << 3); }
-
-__global__ __launch_bounds__(512) void k_gemm_bf3r(Bf3Planes g) {
-    using namespace bf3r;
-    __shared__ __attribute__((aligned(16))) __bf16 sm[2][4][PLANE];  // buffer, plane (Ah Al Bh Bl)
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int TX = (g.Nr + BN - 1) / BN, TY = (g.M + BM - 1) / BM, TT = TX * TY;
-    const int t0 = g.persistent ? (int)blockIdx.x : (int)((blockIdx.z * TY + blockIdx.y) * gridDim.x + blockIdx.x);
-    const int tstep = g.persistent ? (int)gridDim.x : TT * g.bt.count;
-    const int r32 = lane & 31, kg = lane >> 5;
-    // this thread's chunks: q = i * 512 + tid, row q >> 2, chunk q & 3 (same in every plane)
-    const int q0 = tid, q1 = 512 + tid;
-    const int oa0 = (q0 >> 2) * (int)g.lda + 8 * (q0 & 3), oa1 = (q1 >> 2) * (int)g.lda + 8 * (q1 & 3);
-    const int ob0 = (q0 >> 2) * (int)g.ldb + 8 * (q0 & 3), ob1 = (q1 >> 2) * (int)g.ldb + 8 * (q1 & 3);
-    const int ol0 = bf3r_off(q0 >> 2, q0 & 3), ol1 = bf3r_off(q1 >> 2, q1 & 3);
+    for (int i = 0; i < CB; ++i) ob[i] = 2u * ((i * (T / 4) + row) * (unsigned)g.ldb + 8 * (tid & 3));
     for (int tl = t0; tl < TT * g.bt.count; tl += tstep) {
         if (tl != t0) __syncthreads();  // the previous tile's LDS reads are done
         const int zb = tl / TT;
@@ -624,277 +502,123 @@ __global__ __launch_bounds__(512) void k_gemm_bf3r(Bf3Planes g) {
         tile_of_linear(tl - zb * TT, TX, TY, &ty, &tx);
         const long long bm = (long long)ty * BM, bn = (long long)tx * BN;
         const int nk = g.Kp / BK;
-        const __bf16 *pah = batch_scr(g.bt, g.Ah, zb) + bm * g.lda, *pal = batch_scr(g.bt, g.Al, zb) + bm * g.lda;
-        const __bf16 *pbh = batch_scr(g.bt, g.Bh, zb) + bn * g.ldb, *pbl = batch_scr(g.bt, g.Bl, zb) + bn * g.ldb;
-        // staging registers (named, so that they stay in registers)
-        uint4 s00, s01, s10, s11, s20, s21, s30, s31;
-#define BF3R_GLOAD(kt)                                            \
-    do {                                                          \
-        const int k0_ = (kt) * BK;                                \
-        s00 = *(const uint4 *)(pah + k0_ + oa0);                  \
-        s01 = *(const uint4 *)(pah + k0_ + oa1);                  \
-        s10 = *(const uint4 *)(pal + k0_ + oa0);                  \
-        s11 = *(const uint4 *)(pal + k0_ + oa1);                  \
-        s20 = *(const uint4 *)(pbh + k0_ + ob0);                  \
-        s21 = *(const uint4 *)(pbh + k0_ + ob1);                  \
-        s30 = *(const uint4 *)(pbl + k0_ + ob0);                  \
-        s31 = *(const uint4 *)(pbl + k0_ + ob1);                  \
-    } while (0)
-#define BF3R_LSTORE(b)                                            \
-    do {                                                          \
-        *(uint4 *)&sm[(b)][0][ol0] = s00;                         \
-        *(uint4 *)&sm[(b)][0][ol1] = s01;                         \
-        *(uint4 *)&sm[(b)][1][ol0] = s10;                         \
-        *(uint4 *)&sm[(b)][1][ol1] = s11;                         \
-        *(uint4 *)&sm[(b)][2][ol0] = s20;                         \
-        *(uint4 *)&sm[(b)][2][ol1] = s21;                         \
-        *(uint4 *)&sm[(b)][3][ol0] = s30;                         \
-        *(uint4 *)&sm[(b)][3][ol1] = s31;                         \
-    } while (0)
-        floatx16 acc[2][4];
+        const __bf16 *ah = batch_scr(g.bt, g.Ah, zb) + bm * g.lda, *al = batch_scr(g.bt, g.Al, zb) + bm * g.lda;
+        const __bf16 *bh = batch_scr(g.bt, g.Bh, zb) + bn * g.ldb, *bl = batch_scr(g.bt, g.Bl, zb) + bn * g.ldb;
+        u32x4 ra[2][CA], rb[2][CB];
+        auto gload = [&](int kt) {
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+            for (int p = 0; p < 2; ++p) {
+                const char *pa = (const char *)((p ? al : ah) + kt * BK), *pb = (const char *)((p ? bl : bh) + kt * BK);
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+                for (int i = 0; i < CA; ++i) ra[p][i] = *(const u32x4 *)(pa + oa[i]);
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-        BF3R_GLOAD(0);
-        BF3R_LSTORE(0);
-        if (nk > 1) BF3R_GLOAD(1);
+                for (int i = 0; i < CB; ++i) rb[p][i] = *(const u32x4 *)(pb + ob[i]);
+            }
+        };
+        auto lstore = [&](int b) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+#pragma unroll
+                for (int i = 0; i < CA; ++i) *(u32x4 *)&sa[b][p][bf3_off(i * (T / 4) + row, tid & 3)] = ra[p][i];
+#pragma unroll
+                for (int i = 0; i < CB; ++i) *(u32x4 *)&sb[b][p][bf3_off(i * (T / 4) + row, tid & 3)] = rb[p][i];
+            }
+        };
+        struct Frag {
+            bf16x8 ah[MT], al[MT], bh[NC], bl[NC];
+        } f0, f1;
+        auto read = [&](Frag &f, int b, int kk) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int o = bf3_off((wm * MT + mt) * 32 + r32, 2 * kk + kg);
+                f.ah[mt] = *(const bf16x8 *)&sa[b][0][o];
+                f.al[mt] = *(const bf16x8 *)&sa[b][1][o];
+            }
+#pragma unroll
+            for (int nt = 0; nt < NC; ++nt) {
+                const int o = bf3_off((wn * NC + nt) * 32 + r32, 2 * kk + kg);
+                f.bh[nt] = *(const bf16x8 *)&sb[b][0][o];
+                f.bl[nt] = *(const bf16x8 *)&sb[b][1][o];
+            }
+        };
+        floatx16 acc[MT][NC][2];  // real and imaginary parts
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+#pragma unroll
+            for (int b = 0; b < NC; ++b)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[a][b][0][v] = acc[a][b][1][v] = 0.f;
+        auto mult = [&](const Frag &f) {
+            bf16x8 bh[NC][2], bl[NC][2];
+#pragma unroll
+            for (int nt = 0; nt < NC; ++nt) {
+                bh[nt][0] = f.bh[nt];
+                bh[nt][1] = bf3_turn(f.bh[nt]);
+                bl[nt][0] = f.bl[nt];
+                bl[nt][1] = bf3_turn(f.bl[nt]);
+            }
+#pragma unroll
+            for (int term = 0; term < 3; ++term)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int nt = 0; nt < NC; ++nt)
+#pragma unroll
+                        for (int p = 0; p < 2; ++p)
+                            acc[mt][nt][p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                                term == 0 ? f.al[mt] : f.ah[mt], term == 1 ? bl[nt][p] : bh[nt][p], acc[mt][nt][p], 0, 0,
+                                0);
+        };
+        gload(0);
+        lstore(0);
+        if (nk > 1) gload(1);
         __syncthreads();
+        read(f0, 0, 0);
         for (int kt = 0; kt < nk; ++kt) {
             const int buf = kt & 1;
-#pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                bf16x8 ah[2], al[2], bh[4], bl[4];
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt) {
-                    const int o = bf3r_off(wm * 64 + mt * 32 + r32, 2 * kk + kg);
-                    ah[mt] = *(const bf16x8 *)&sm[buf][0][o];
-                    al[mt] = *(const bf16x8 *)&sm[buf][1][o];
-                }
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt) {
-                    const int o = bf3r_off(wn * 128 + nt * 32 + r32, 2 * kk + kg);
-                    bh[nt] = *(const bf16x8 *)&sm[buf][2][o];
-                    bl[nt] = *(const bf16x8 *)&sm[buf][3][o];
-                }
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                    for (int nt = 0; nt < 4; ++nt)
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[mt], bh[nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                    for (int nt = 0; nt < 4; ++nt)
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mt], bl[nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-                for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-                    for (int nt = 0; nt < 4; ++nt)
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mt], bh[nt], acc[mt][nt], 0, 0, 0);
-            }
+            read(f1, buf, 1);
+            mult(f0);
             if (kt + 1 < nk) {
-                BF3R_LSTORE(buf ^ 1);  // last read in step kt - 1, before the previous barrier
-                if (kt + 2 < nk) BF3R_GLOAD(kt + 2);
+                lstore(buf ^ 1);  // last read in step kt - 1, before that step's barrier
+                if (kt + 2 < nk) gload(kt + 2);
             }
             __syncthreads();
+            if (kt + 1 < nk) read(f0, buf ^ 1, 0);
+            mult(f1);
         }
-#undef BF3R_GLOAD
-#undef BF3R_LSTORE
 
+        // epilogue: all C loads of a 32-row slab are issued before its stores;
+        // tiles wholly inside C skip the per-element bounds checks
         const float sgn = g.alpha_neg ? -1.f : 1.f;
-        float *__restrict__ C =
-            batch_mat(g.bt, g.C, zb) + (bm + wm * 64 + 4 * (lane >> 5)) * g.ldc + bn + wn * 128 + r32;
-        const int mrem = (int)min((long long)BM, g.M - bm) - wm * 64 - 4 * (lane >> 5);
-        const int nrem = (int)min((long long)BN, (long long)g.Nr - bn) - wn * 128 - r32;
-        const bool full = bm + BM <= g.M && bn + BN <= g.Nr;
+        int ldc = (int)(g.ldc >> 1);
+        asm volatile("" : "+s"(ldc));  // its multiples are formed here, not kept over the K loop
+        const int rowc = wm * 32 * MT + 4 * kg, colc = wn * 32 * NC + r32;
+        float2 *__restrict__ C = (float2 *)batch_mat(g.bt, g.C, zb) + bm * ldc + bn;
+        const unsigned oc = 8u * (unsigned)(rowc * ldc + colc);  // bytes
+        auto at = [&](int i, int j) -> float2 & { return *(float2 *)((char *)(C + ((long long)i * ldc + j)) + oc); };
+        const int mrem = (int)min((long long)BM, g.M - bm) - rowc;
+        const int nrem = (int)min((long long)BN, ncols - bn) - colc;
+        const bool full = bm + BM <= g.M && bn + BN <= ncols;
         auto epilogue = [&](auto guarded) {
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt) {
-                float cv[4][16];
+            for (int mt = 0; mt < MT; ++mt) {
+                float2 cv[NC][16];
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
+                for (int nt = 0; nt < NC; ++nt)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) {
                         const int i = mt * 32 + 8 * (v >> 2) + (v & 3), j = nt * 32;
                         const bool in = !guarded.value || (i < mrem && j < nrem);
-                        cv[nt][v] = (g.beta && in) ? C[i * g.ldc + j] : 0.f;
+                        cv[nt][v] = (g.beta && in) ? at(i, j) : make_float2(0.f, 0.f);
                     }
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
+                for (int nt = 0; nt < NC; ++nt)
 #pragma unroll
                     for (int v = 0; v < 16; ++v) {
                         const int i = mt * 32 + 8 * (v >> 2) + (v & 3), j = nt * 32;
-                        if (!guarded.value || (i < mrem && j < nrem)) C[i * g.ldc + j] = cv[nt][v] + sgn * acc[mt][nt][v];
-                    }
-            }
-        };
-        if (full)
-            epilogue(std::false_type{});
-        else
-            epilogue(std::true_type{});
-    }  // tiles
-}
-
-// ---------------------------------------------------------------------------
-// The same product with one wave per SIMD and register-double-buffered
-// operand fragments.  Workgroup tile 256 x 256, 4 waves as 2 x 2 with wave
-// tiles 128 x 128 (4 x 4 MFMA 32x32x16 tiles: 256 accumulators per lane,
-// which the compiler keeps in the accumulation registers), LDS ring of four
-// K = 16 stages filled by direct global -> LDS loads (wave w loads plane w:
-// Ah, Al, Bh, Bl).  At step kt the wave multiplies the fragments of stage kt,
-// already in registers, while it reads the fragments of stage kt + 1 from
-// LDS into the other register set (one LDS read per three MFMAs, the order
-// pinned with scheduling barriers); the one barrier per step publishes stage
-// kt + 1 and frees the slot of stage kt - 1 for the loads of stage kt + 3.  Per
-// accumulator the products are added in bf3p's order (Al Bh, Ah Bl, Ah Bh per
-// stage, stages in order), so the two kernels give the same bits.
-// ---------------------------------------------------------------------------
-namespace bf3q {
-constexpr int BM = 256, BN = 256, BK = 16, NS = 4, PLANE = 256 * BK;
-}
-
-__global__ __launch_bounds__(256, 1) void k_gemm_bf3q(Bf3Planes g) {
-    using namespace bf3q;
-    __shared__ __attribute__((aligned(16))) __bf16 sm[NS][4][PLANE];  // stage, plane (Ah Al Bh Bl)
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int TX = (g.Nr + BN - 1) / BN, TY = (g.M + BM - 1) / BM, TT = TX * TY;
-    const int t0 = g.persistent ? (int)blockIdx.x : (int)((blockIdx.z * TY + blockIdx.y) * gridDim.x + blockIdx.x);
-    const int tstep = g.persistent ? (int)gridDim.x : TT * g.bt.count;
-    const int r32 = lane & 31, kg = lane >> 5;
-    for (int tl = t0; tl < TT * g.bt.count; tl += tstep) {
-        if (tl != t0) __syncthreads();  // the previous tile's LDS reads are done
-        const int zb = tl / TT;
-        int ty, tx;
-        tile_of_linear(tl - zb * TT, TX, TY, &ty, &tx);
-        const long long bm = (long long)ty * BM, bn = (long long)tx * BN;
-        const int nk = g.Kp / BK;
-
-        // this wave's direct loads: plane `wave`, rows 32 i + lane / 2 (i < 8),
-        // chunk (lane & 1) stored at its swizzled position
-        const __bf16 *src = batch_scr(g.bt, wave == 0 ? g.Ah : wave == 1 ? g.Al : wave == 2 ? g.Bh : g.Bl, zb);
-        const long long ld = wave < 2 ? g.lda : g.ldb;
-        const long long row0 = wave < 2 ? bm : bn;
-        const int lr = lane >> 1;
-        const __bf16 *gbase = src + (row0 + lr) * ld + 8 * ((lane & 1) ^ bf3_swz(lr));
-        const long long rstep = 32 * ld;
-        auto issue = [&](int kt) {
-            const int st = kt & (NS - 1);
-            const __bf16 *gp = gbase + (long long)kt * BK;
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                __builtin_amdgcn_global_load_lds((const void *)(gp + i * rstep), (lds_void *)&sm[st][wave][32 * i * BK],
-                                                 16, 0, 0);
-        };
-        int offa[4], offb[4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            offa[t] = bf3p_off(wm * 128 + t * 32 + r32, kg);
-            offb[t] = bf3p_off(wn * 128 + t * 32 + r32, kg);
-        }
-        bf16x8 ah[2][4], al[2][4], bh[2][4], bl[2][4];
-        auto read = [&](int kt, int buf) {
-            const int st = kt & (NS - 1);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                ah[buf][t] = *(const bf16x8 *)&sm[st][0][offa[t]];
-                al[buf][t] = *(const bf16x8 *)&sm[st][1][offa[t]];
-                bh[buf][t] = *(const bf16x8 *)&sm[st][2][offb[t]];
-                bl[buf][t] = *(const bf16x8 *)&sm[st][3][offb[t]];
-            }
-        };
-        floatx16 acc[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-
-        issue(0);
-        if (nk > 1) issue(1);
-        if (nk > 2) issue(2);
-        if (nk > 2)
-            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        else if (nk > 1)
-            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        read(0, 0);
-        // one step: fragments of stage kt in set cur, stage kt + 1 read into set nxt
-        auto step = [&](int kt, int cur, int nxt) {
-            if (kt + 2 < nk)
-                asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-            else
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            if (kt + 3 < nk) issue(kt + 3);
-            read(kt + 1 < nk ? kt + 1 : kt, nxt);
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[cur][mt], bh[cur][nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[cur][mt], bl[cur][nt], acc[mt][nt], 0, 0, 0);
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[cur][mt], bh[cur][nt], acc[mt][nt], 0, 0, 0);
-            // one LDS read of the next set, then three MFMAs, sixteen times
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-            }
-        };
-        // set 1 is read while set 0 is multiplied, then becomes set 0
-        for (int kt = 0; kt < nk; ++kt) {
-            step(kt, 0, 1);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                ah[0][t] = ah[1][t];
-                al[0][t] = al[1][t];
-                bh[0][t] = bh[1][t];
-                bl[0][t] = bl[1][t];
-            }
-        }
-
-        // epilogue: all C loads of a 32-row slab are issued before its stores
-        const float sgn = g.alpha_neg ? -1.f : 1.f;
-        float *__restrict__ C =
-            batch_mat(g.bt, g.C, zb) + (bm + wm * 128 + 4 * (lane >> 5)) * g.ldc + bn + wn * 128 + r32;
-        const int mrem = (int)min((long long)BM, g.M - bm) - wm * 128 - 4 * (lane >> 5);
-        const int nrem = (int)min((long long)BN, (long long)g.Nr - bn) - wn * 128 - r32;
-        const bool full = bm + BM <= g.M && bn + BN <= g.Nr;
-        auto epilogue = [&](auto guarded) {
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt) {
-                float cv[4][16];
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int i = mt * 32 + 8 * (v >> 2) + (v & 3), j = nt * 32;
-                        const bool in = !guarded.value || (i < mrem && j < nrem);
-                        cv[nt][v] = (g.beta && in) ? C[i * g.ldc + j] : 0.f;
-                    }
-#pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int i = mt * 32 + 8 * (v >> 2) + (v & 3), j = nt * 32;
-                        if (!guarded.value || (i < mrem && j < nrem)) C[i * g.ldc + j] = cv[nt][v] + sgn * acc[mt][nt][v];
+                        if (!guarded.value || (i < mrem && j < nrem))
+                            at(i, j) = make_float2(cv[nt][v].x + sgn * acc[mt][nt][0][v],
+                                                         cv[nt][v].y + sgn * acc[mt][nt][1][v]);
                     }
             }
         };
@@ -1115,40 +839,30 @@ emfa_status split_bf16_launch(hipStream_t s, const float *src, long long ld, int
 
 emfa_status gemm_launch_bf3_planes(hipStream_t s, const Bf3Planes &g) {
     auto al16 = [](const void *p) { return ((uintptr_t)p % 16) == 0; };
-    EMFA_REQUIRE(g.M > 0 && g.Nr > 0 && g.Kp > 0 && g.Kp % bf3p::BK == 0 && g.lda >= g.Kp && g.ldb >= g.Kp &&
-                     g.lda % 8 == 0 && g.ldb % 8 == 0 && al16(g.Ah) && al16(g.Al) && al16(g.Bh) && al16(g.Bl) &&
-                     g.M <= 65535LL * bf3p::BM && g.Nr <= 65535LL * bf3p::BN,
+    EMFA_REQUIRE(g.M > 0 && g.Nr > 0 && g.Nr % 2 == 0 && g.Kp > 0 && g.Kp % bf3::BK == 0 && g.lda >= g.Kp &&
+                     g.ldb >= g.Kp && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.lda <= (1LL << 22) && g.ldb <= (1LL << 22) &&
+                     g.ldc % 2 == 0 && g.ldc <= (1LL << 22) && (uintptr_t)g.C % 8 == 0 && al16(g.Ah) && al16(g.Al) && al16(g.Bh) &&
+                     al16(g.Bl) && g.M <= 65535LL * 128 && g.Nr <= 65535LL * 128,
                  EMFA_E_INVALID, "gemm bf16x3 planes: bad shape M=%d Nr=%d Kp=%d", g.M, g.Nr, g.Kp);
-    const int TX = (g.Nr + bf3p::BN - 1) / bf3p::BN, TY = (g.M + bf3p::BM - 1) / bf3p::BM;
     EMFA_REQUIRE(g.bt.count >= 1 && g.bt.count <= 65535, EMFA_E_INVALID, "gemm bf16x3 planes: batch %d", g.bt.count);
     Bf3Planes gg = g;
-    // the register-staged kernel when K is a multiple of 32, else the
-    // direct-load one; EMFA_BF3_KERNEL=p / q select the direct-load or the
-    // one-wave-per-SIMD kernel (all give the same bits)
-    static const int env_kernel = [] {
-        const char *e = getenv("EMFA_BF3_KERNEL");
-        return e && e[0] == 'q' ? 2 : e && e[0] == 'p' ? 1 : 4;
-    }();
-    int kern = g.kernel ? g.kernel : env_kernel;
-    if (kern == 4 && g.Kp % bf3r::BK != 0) kern = 1;
-    EMFA_REQUIRE(kern == 4 ? (g.lda <= (1LL << 23) && g.ldb <= (1LL << 23)) : true, EMFA_E_INVALID,
-                 "gemm bf16x3 planes: plane stride too large");
-    const int threads = kern == 2 ? 256 : 512;
-    auto launch = [&](dim3 grid) {
-        if (kern == 2)
-            k_gemm_bf3q<<<grid, threads, 0, s>>>(gg);
-        else if (kern == 4)
-            k_gemm_bf3r<<<grid, threads, 0, s>>>(gg);
-        else
-            k_gemm_bf3p<<<grid, threads, 0, s>>>(gg);
+    auto launch = [&](auto kernel, int bm, int bn, int threads, int cap) {
+        const int TX = (g.Nr / 2 + bn - 1) / bn, TY = (g.M + bm - 1) / bm;
+        gg.persistent = cap >= 8 && (long long)TX * TY * g.bt.count > cap;
+        const dim3 grid = gg.persistent ? dim3((cap / 8) * 8) : dim3(TX, TY, g.bt.count);
+        kernel<<<grid, threads, 0, s>>>(gg);
     };
-    if (g.max_wgs >= 8 && (long long)TX * TY * g.bt.count > g.max_wgs) {
-        gg.persistent = 1;
-        launch(dim3((g.max_wgs / 8) * 8));
-    } else {
-        gg.persistent = 0;
-        launch(dim3(TX, TY, g.bt.count));
-    }
+    // 256 x 256 tiles (reals) move the fewest operand bytes, 128 x 128 ones fill
+    // the chip from a quarter of the size on and come two to a CU, so that one's
+    // C and first loads hide behind the other's products.  The line is at 1.5
+    // large tiles a CU: 1920 unknowns (at most 49) 2.26 ms a factorisation with
+    // large tiles and 2.13 with small ones, 8321 (1024 at first, 400 half way)
+    // 18.84 and 18.92, 18.68 with this line; 30720 372 and 399.
+    const long long large = (long long)((g.Nr + 255) / 256) * ((g.M + 255) / 256) * g.bt.count;
+    if (large >= 400)
+        launch(k_gemm_bf3<4, 2, 2, 2>, 256, 128, 512, g.max_wgs);
+    else
+        launch(k_gemm_bf3<2, 2, 2, 1>, 128, 64, 256, 2 * g.max_wgs);
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
 }

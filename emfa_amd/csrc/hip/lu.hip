@@ -949,20 +949,20 @@ static emfa_status gemm_update(emfa_ctx *ctx, const char *fam, int M, int ncols,
 }
 
 // Operand planes of the three-term bf16 trailing update (FP32 factorisations):
-// the outer panel's L block (M x 2jb reals) and expanded U rows (2(N-next) x
-// 2jb reals), split once per outer step and read by both update halves.
+// the outer panel's L block (M x 2jb reals) and U rows (N - next columns x 2jb
+// reals), split once per outer step and read by both update halves.
 struct UpdatePlanes {
     __bf16 *ah = nullptr, *al = nullptr, *bh = nullptr, *bl = nullptr;
     int a_rows = 0, b_rows = 0, kp = 0;  // allocated rows per plane, K stride
     static int rup(int a, int b) { return (a + b - 1) / b * b; }
     static size_t bytes(int N, int nb) {
-        const size_t kp = (size_t)rup(2 * nb, 16);
-        return 2 * kp * sizeof(__bf16) * ((size_t)rup(N, 256) + (size_t)rup(2 * N, 256) + 256) + 1024;
+        const size_t kp = (size_t)rup(2 * nb, 32);
+        return 2 * kp * sizeof(__bf16) * ((size_t)rup(N, 256) + (size_t)rup(N, 128) + 128) + 1024;
     }
     void carve(void *p, int N, int nb) {
-        kp = rup(2 * nb, 16);
+        kp = rup(2 * nb, 32);
         a_rows = rup(N, 256);
-        b_rows = rup(2 * N, 256) + 256;
+        b_rows = rup(N, 128) + 128;
         char *q = (char *)p;
         auto take = [&](size_t b) {
             char *r = q;
@@ -974,16 +974,17 @@ struct UpdatePlanes {
         bh = take((size_t)b_rows * kp * sizeof(__bf16));
         bl = take((size_t)b_rows * kp * sizeof(__bf16));
     }
-    // split L (M x K complex at Aop, lda) and the U rows (2*ncols x 2K reals, ldb)
+    // split L (M x K complex at Aop, lda) and the U rows: of the expanded
+    // operand (2 ncols x 2K reals, ldb) the rows of the real parts, (re, -im)
     emfa_status split(emfa_ctx *ctx, int M, int ncols, int K, const cx<float> *Aop, long long lda, const float *Bt,
                       long long ldb) {
         ProfScope ps(ctx, "lu_split", 0);
-        const int kr = 2 * K, k16 = rup(kr, 16);
+        const int kr = 2 * K, k32 = rup(kr, 32);
         emfa_status st = split_bf16_launch(ctx->stream, (const float *)Aop, 2 * lda, M, kr, ah, al, kp,
-                                           rup(M, 256), k16, ctx->batch, true);
+                                           rup(M, 256), k32, ctx->batch, true);
         if (st) return st;
-        return split_bf16_launch(ctx->stream, Bt, ldb, 2 * ncols, kr, bh, bl, kp,
-                                 std::min(b_rows, rup(2 * ncols, 256) + 256), k16, ctx->batch, false);
+        return split_bf16_launch(ctx->stream, Bt, 2 * ldb, ncols, kr, bh, bl, kp,
+                                 std::min(b_rows, rup(ncols, 128) + 128), k32, ctx->batch, false);
     }
     // C (M x ncols complex) -= L * U[:, c0 : c0 + ncols]
     emfa_status update(emfa_ctx *ctx, int M, int c0, int ncols, int K, cx<float> *C, long long ldc,
@@ -993,12 +994,12 @@ struct UpdatePlanes {
         Bf3Planes g;
         g.M = M;
         g.Nr = 2 * ncols;
-        g.Kp = rup(2 * K, 16);
+        g.Kp = rup(2 * K, 32);
         g.Ah = ah;
         g.Al = al;
         g.lda = kp;
-        g.Bh = bh + (size_t)2 * c0 * kp;
-        g.Bl = bl + (size_t)2 * c0 * kp;
+        g.Bh = bh + (size_t)c0 * kp;
+        g.Bl = bl + (size_t)c0 * kp;
         g.ldb = kp;
         g.C = (float *)C;
         g.ldc = 2 * ldc;
