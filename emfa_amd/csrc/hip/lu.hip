@@ -248,16 +248,22 @@ __global__ __launch_bounds__(256) void k_panel(cx<R> *__restrict__ A, long long 
 // workgroup writes one 64-bit packet per column into its own slot (double
 // buffered by column parity) and every workgroup polls the G packets, so the
 // barrier and the candidate values travel together.
-//   complex FP32: packet = value bits | row << 32 | (epoch & 0xFFF) << 52;
-//     candidate rows are 64-bit words {float bits, epoch}, two per element,
-//     so a reader can tell a fresh word from a stale one and the writer never
-//     waits for its stores.
-//   complex FP64: packet = row | epoch << 32; the value and the row are
-//     written first and ordered before the packet by s_waitcnt.
+//   FP32: packet = value bits | row << 32 | (epoch & 0xFFF) << 52;
+//   FP64: two words, the first as for FP32 with the value's upper half, the
+//     second the lower half | epoch << 32;
+//   candidate rows and the current row are words of 32 bits | epoch << 32, two
+//     per element in FP32 and four in FP64, so a reader can tell a fresh word
+//     from a stale one and no writer waits for its stores.
 // The epoch of column jc is jc + 1; the slots are zeroed before each
 // factorisation.  Rows live in LDS column-major (stride RB + 1) and one
 // thread owns a row in the update, which also yields the next column's local
 // candidate, so a column costs two workgroup barriers.
+// Bound by the trips through memory that the workgroups see each other by:
+// the packets' and the winning row's, one after the other; the current row is
+// polled beside the packets.  With
+// the FP64 value in its packet (it was read after it, and stored ahead of it
+// with a wait between) 4256 unknowns in FP64 take 37.2 ms from 40.9, pivots and
+// factors the same.
 // --------------------------------------------------------------------------
 constexpr int kPanelMaxG = 256;
 
@@ -267,22 +273,55 @@ __device__ __forceinline__ void st64(unsigned long long *p, unsigned long long v
 __device__ __forceinline__ unsigned long long ld64(const unsigned long long *p) {
     return __hip_atomic_load((unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ unsigned long long tag32(float x, unsigned ep) {
-    return (unsigned long long)__float_as_uint(x) | ((unsigned long long)ep << 32);
+__device__ __forceinline__ unsigned long long tag32(unsigned x, unsigned ep) {
+    return (unsigned long long)x | ((unsigned long long)ep << 32);
 }
 
-// FP32 self-validating pair load; false if the bounded spin ran out
-__device__ __forceinline__ bool ld_tagged(const unsigned long long *p, unsigned ep, cx<float> *out, bool active,
+// 32-bit words of a value
+template <typename R>
+constexpr int kWords = (int)sizeof(R) / 4;
+
+// an element as tagged words
+template <typename R>
+__device__ __forceinline__ void st_tagged(unsigned long long *d, cx<R> x, unsigned ep) {
+    unsigned w[2 * kWords<R>];
+    __builtin_memcpy(w, &x, sizeof(x));
+#pragma unroll
+    for (int k = 0; k < 2 * kWords<R>; ++k) st64(d + k, tag32(w[k], ep));
+}
+
+// one look at an element's tagged words; false if any is stale
+template <typename R>
+struct TaggedWords {
+    unsigned long long v[2 * kWords<R>];
+    __device__ __forceinline__ void load(const unsigned long long *p) {
+#pragma unroll
+        for (int k = 0; k < 2 * kWords<R>; ++k) v[k] = ld64(p + k);
+    }
+    __device__ __forceinline__ bool get(unsigned ep, cx<R> *out) const {
+        unsigned w[2 * kWords<R>];
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < 2 * kWords<R>; ++k) {
+            w[k] = (unsigned)v[k];
+            ok = ok && (unsigned)(v[k] >> 32) == ep;
+        }
+        if (ok) __builtin_memcpy(out, w, sizeof(*out));
+        return ok;
+    }
+};
+
+// load of a tagged element; false if the bounded spin ran out
+template <typename R>
+__device__ __forceinline__ bool ld_tagged(const unsigned long long *p, unsigned ep, cx<R> *out, bool active,
                                           int *flags) {
     unsigned spins = 0;
     bool ok = !active;
     for (;;) {
         if (!ok) {
-            unsigned long long a = ld64(p), b = ld64(p + 1);
-            if ((unsigned)(a >> 32) == ep && (unsigned)(b >> 32) == ep) {
-                *out = {__uint_as_float((unsigned)a), __uint_as_float((unsigned)b)};
-                ok = true;
-            }
+            TaggedWords<R> t;
+            t.load(p);
+            ok = t.get(ep, out);
         }
         if (__ballot(!ok) == 0) return true;
         if (++spins > kSpinLimit) {
@@ -296,9 +335,8 @@ __device__ __forceinline__ bool ld_tagged(const unsigned long long *p, unsigned 
 template <typename R>
 __global__ __launch_bounds__(256) void k_panel_x(cx<R> *__restrict__ A, long long lda, int j0, int M, int w, int RB,
                                                  int *__restrict__ ipiv, unsigned long long *pk,
-                                                 unsigned long long *rw, unsigned long long *cw, R *sval,
-                                                 int *flags) {
-    constexpr bool kF32 = sizeof(R) == 4;
+                                                 unsigned long long *rw, unsigned long long *cw, int *flags) {
+    constexpr int kV = kWords<R>, kE = 2 * kV;  // words of a packet, of an element
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cx<R> *cols = (cx<R> *)smem_raw;  // [w][RBp]
     const int RBp = RB + 1;
@@ -343,58 +381,50 @@ __global__ __launch_bounds__(256) void k_panel_x(cx<R> *__restrict__ A, long lon
                 }
             const bool own_jc = jc >= rbeg && jc < rend;
             // publish this workgroup's candidate
-            if (kF32) {
-                if (br >= 0 && lane < w) {
-                    cx<R> x = cols[lane * RBp + (br - rbeg)];
-                    unsigned long long *d = rw + ((size_t)par * G + g) * (2 * kPanelMaxW) + 2 * lane;
-                    st64(d, tag32((float)x.re, ep));
-                    st64(d + 1, tag32((float)x.im, ep));
-                }
-                if (own_jc && lane < w) {
-                    cx<R> x = cols[lane * RBp + (jc - rbeg)];
-                    unsigned long long *d = cw + (size_t)par * (2 * kPanelMaxW) + 2 * lane;
-                    st64(d, tag32((float)x.re, ep));
-                    st64(d + 1, tag32((float)x.im, ep));
-                }
-                if (lane == 0) {
-                    unsigned idx = br >= 0 ? (unsigned)br : 0xFFFFFu;
-                    float v = br >= 0 ? (float)bv : 0.f;
-                    st64(&pk[par * kPanelMaxG + g], (unsigned long long)__float_as_uint(v) |
-                                                        ((unsigned long long)idx << 32) |
-                                                        ((unsigned long long)(ep & 0xFFFu) << 52));
-                }
-            } else {
-                cx<R> *rwc = (cx<R> *)rw, *cwc = (cx<R> *)cw;
-                if (br >= 0 && lane < w)
-                    st_co(&rwc[((size_t)par * G + g) * kPanelMaxW + lane], cols[lane * RBp + (br - rbeg)]);
-                if (own_jc && lane < w) st_co(&cwc[(size_t)par * kPanelMaxW + lane], cols[lane * RBp + (jc - rbeg)]);
-                if (lane == 0) st_co(&sval[par * kPanelMaxG + g], bv);
-                __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                if (lane == 0)
-                    st64(&pk[par * kPanelMaxG + g],
-                         (unsigned long long)(br >= 0 ? (unsigned)br : 0xFFFFFFFFu) | ((unsigned long long)ep << 32));
+            if (br >= 0 && lane < w)
+                st_tagged<R>(rw + (((size_t)par * G + g) * kPanelMaxW + lane) * kE, cols[lane * RBp + (br - rbeg)], ep);
+            const unsigned long long *cwl = cw + ((size_t)par * kPanelMaxW + min(lane, w - 1)) * kE;
+            if (own_jc && lane < w)
+                st_tagged<R>(cw + ((size_t)par * kPanelMaxW + lane) * kE, cols[lane * RBp + (jc - rbeg)], ep);
+            if (lane == 0) {
+                const R v = br >= 0 ? bv : R(0);
+                unsigned b[kV];
+                __builtin_memcpy(b, &v, sizeof(v));
+                unsigned long long *d = pk + ((size_t)par * kPanelMaxG + g) * kV;
+                const unsigned idx = br >= 0 ? (unsigned)br : 0xFFFFFu;
+                st64(d, (unsigned long long)b[kV - 1] | ((unsigned long long)idx << 32) |
+                            ((unsigned long long)(ep & 0xFFFu) << 52));
+                if constexpr (kV == 2) st64(d + 1, tag32(b[0], ep));
             }
-            // gather the G packets (up to four per lane)
-            unsigned long long pkv[4] = {0, 0, 0, 0};
+            // gather the G packets (up to four per lane) and the current row
+            unsigned long long pkv[4][kV];
+            cx<R> u = {R(0), R(0)}, o = {R(0), R(0)};
+            bool o_ok = false;
             int okm = 0;
             unsigned spins = 0;
             while (!dead) {
                 bool all = true;
+                TaggedWords<R> ow;
+                if (!o_ok) ow.load(cwl);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int q = lane + 64 * k;
-                    if (q < G && !((okm >> k) & 1)) {
-                        unsigned long long v = ld64(&pk[par * kPanelMaxG + q]);
-                        bool ok = kF32 ? (unsigned)(v >> 52) == (ep & 0xFFFu) : (unsigned)(v >> 32) == ep;
-                        if (ok) {
-                            pkv[k] = v;
-                            okm |= 1 << k;
-                        } else {
-                            all = false;
-                        }
+                for (int k = 0; k < 4; ++k)
+                    if (64 * k < G && !((okm >> k) & 1)) {
+                        const unsigned long long *d = pk + ((size_t)par * kPanelMaxG + min(lane + 64 * k, G - 1)) * kV;
+#pragma unroll
+                        for (int h = 0; h < kV; ++h) pkv[k][h] = ld64(d + h);
                     }
-                }
-                if (__ballot(!all) == 0) break;
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (64 * k < G && !((okm >> k) & 1)) {
+                        bool ok = (unsigned)(pkv[k][0] >> 52) == (ep & 0xFFFu);
+                        if constexpr (kV == 2) ok = ok && (unsigned)(pkv[k][1] >> 32) == ep;
+                        if (ok)
+                            okm |= 1 << k;
+                        else
+                            all = false;
+                    }
+                if (!o_ok) o_ok = ow.get(ep, &o);
+                if (__ballot(!(all && o_ok)) == 0) break;
                 if (++spins > kSpinLimit ||
                     __builtin_amdgcn_readfirstlane(
                         __hip_atomic_load(&flags[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) {
@@ -411,17 +441,13 @@ __global__ __launch_bounds__(256) void k_panel_x(cx<R> *__restrict__ A, long lon
                 for (int k = 0; k < 4; ++k) {
                     const int q = lane + 64 * k;
                     if (q < G) {
+                        const unsigned idx = (unsigned)(pkv[k][0] >> 32) & 0xFFFFFu;
+                        const int r = idx == 0xFFFFFu ? -1 : (int)idx;
+                        unsigned b[kV];
+                        b[kV - 1] = (unsigned)pkv[k][0];
+                        if constexpr (kV == 2) b[0] = (unsigned)pkv[k][1];
                         R v;
-                        int r;
-                        if (kF32) {
-                            unsigned idx = (unsigned)(pkv[k] >> 32) & 0xFFFFFu;
-                            r = idx == 0xFFFFFu ? -1 : (int)idx;
-                            v = (R)__uint_as_float((unsigned)pkv[k]);
-                        } else {
-                            unsigned idx = (unsigned)pkv[k];
-                            r = idx == 0xFFFFFFFFu ? -1 : (int)idx;
-                            v = r >= 0 ? ld_co(&sval[par * kPanelMaxG + q]) : R(-1);
-                        }
+                        __builtin_memcpy(&v, b, sizeof(v));
                         if (better(v, r, wv, wr)) {
                             wv = v;
                             wr = r;
@@ -434,24 +460,10 @@ __global__ __launch_bounds__(256) void k_panel_x(cx<R> *__restrict__ A, long lon
             int p = singular ? jc : wr;
             if (p < j0 || p >= j0 + M) p = jc;  // only after a failed wait
             const int wg = (p - j0) / RB;
-            cx<R> u = {R(0), R(0)}, o = {R(0), R(0)};
             if (!dead) {
-                if (kF32) {
-                    cx<float> t;
-                    bool ok = ld_tagged(cw + (size_t)par * (2 * kPanelMaxW) + 2 * lane, ep, &t, lane < w, flags);
-                    o = {(R)t.re, (R)t.im};
-                    if (ok && p != jc) {
-                        ok = ld_tagged(rw + ((size_t)par * G + wg) * (2 * kPanelMaxW) + 2 * lane, ep, &t, lane < w,
-                                       flags);
-                        u = {(R)t.re, (R)t.im};
-                    } else {
-                        u = o;
-                    }
-                    if (!ok) dead = true;
-                } else if (lane < w) {
-                    o = ld_co(&((cx<R> *)cw)[(size_t)par * kPanelMaxW + lane]);
-                    u = p != jc ? ld_co(&((cx<R> *)rw)[((size_t)par * G + wg) * kPanelMaxW + lane]) : o;
-                }
+                u = o;
+                if (p != jc && !ld_tagged<R>(rw + (((size_t)par * G + wg) * kPanelMaxW + lane) * kE, ep, &u, lane < w, flags))
+                    dead = true;
             }
             if (lane < w) {
                 urow[lane] = u;
@@ -1491,7 +1503,13 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     int G_max = std::max(1, share > 0 ? std::min(share, ctx->num_cu) : ctx->num_cu);
     if (ctx->panel_g > 0) G_max = std::max(1, std::min(G_max, ctx->panel_g));
     if (const char *s = getenv("EMFA_PANEL_G")) G_max = std::max(1, std::min(G_max, atoi(s)));
-    int panel_rows_min = 16;
+    // at least 48 rows of a panel per workgroup: every workgroup polls every
+    // other's packet, so fewer of them make a column's exchange shorter until the
+    // update of more rows takes longer.  16 / 32 / 48 / 64 / 96 rows, FP64: 1920
+    // unknowns 14.8 / 14.3 / 14.5 / 14.5 / 15.0 ms, 4256 37.8 / 36.0 / 35.8 / 35.7 /
+    // 37.1, 8321 98.4 / 95.0 / 94.5 / 92.6 / 100.1; FP32 with interchanges: 1920
+    // 11.6 / 11.1 / 11.1 / 11.1 / 11.5, 8321 70.2 / 68.2 / 67.1 / 66.5 / 67.3.
+    int panel_rows_min = 48;
     if (const char *s = getenv("EMFA_PANEL_ROWS_MIN")) panel_rows_min = std::max(1, atoi(s));
     // scratch: slots + Bt workspace
     size_t slot_rows_b = 2ull * G_max * kPanelMaxW * sizeof(cx<R>);
@@ -1501,9 +1519,9 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     size_t bar_b = 256;
     size_t bt_b = (size_t)2 * N * 2 * nb * sizeof(R);
     size_t perm_b = PermWs<R>::bytes(N);
-    // packet-exchange slots: packets, candidate rows, current row (zeroed below), values
-    size_t x_pk_b = 2ull * kPanelMaxG * 8, x_rw_b = 2ull * kPanelMaxG * kPanelMaxW * 16,
-           x_cw_b = 2ull * kPanelMaxW * 16, x_val_b = 2ull * kPanelMaxG * sizeof(R);
+    // packet-exchange slots: packets, candidate rows, current row (zeroed below)
+    size_t x_pk_b = 2ull * kPanelMaxG * 8 * kWords<R>, x_rw_b = 2ull * kPanelMaxG * kPanelMaxW * 16 * kWords<R>,
+           x_cw_b = 2ull * kPanelMaxW * 16 * kWords<R>;
     // FP32 factorisations with the bf16-split trailing update keep split operand planes
     bool split_update = false;
     if constexpr (sizeof(R) == 4) {
@@ -1515,7 +1533,7 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     const int nli = (nb + kInvB - 1) / kInvB;
     const size_t uinv_b = ((size_t)kNoPivW * kNoPivW + (size_t)nli * kInvB * kInvB) * sizeof(cx<R>);
     size_t total = slot_rows_b + slot_val_b + slot_idx_b + rowc_b + bar_b + 2 * bt_b + perm_b + x_pk_b + x_rw_b +
-                   x_cw_b + x_val_b + planes_b + uinv_b + 8192;
+                   x_cw_b + planes_b + uinv_b + 8192;
     // a batch: one slab of this layout per matrix (plus its flags and pivots)
     const size_t slab = batched ? (total + 256 + (size_t)N * sizeof(int) + 4096 + 4095) & ~(size_t)4095 : total;
     if (batched) {
@@ -1543,7 +1561,6 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     pws.carve(take(perm_b));
     unsigned long long *x_pk = (unsigned long long *)take(x_pk_b + x_rw_b + x_cw_b);
     unsigned long long *x_rw = x_pk + x_pk_b / 8, *x_cw = x_rw + x_rw_b / 8;
-    R *x_val = (R *)take(x_val_b);
     UpdatePlanes planes;
     if (split_update) planes.carve(take(planes_b), N, nb);
     cx<R> *uinv = (cx<R> *)take(uinv_b);
@@ -1572,7 +1589,7 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     if (ctx->panel_x >= 0) xchg = ctx->panel_x != 0;
     if (const char *s = getenv("EMFA_PANEL_X")) xchg = atoi(s) != 0;
     EMFA_REQUIRE(G_max <= kPanelMaxG, EMFA_E_INVALID, "panel grid %d exceeds %d", G_max, kPanelMaxG);
-    if (sizeof(R) == 4 && N >= 0xFFFFF) xchg = false;  // the FP32 packet holds a 20-bit row index
+    if (N >= 0xFFFFF) xchg = false;  // the packet holds a 20-bit row index
     if (const char *s = getenv("EMFA_LU_LOOKAHEAD")) lookahead = atoi(s) != 0;
     // FP32 factorisations may run without interchanges (panel variant 2)
     bool nopiv = false;
@@ -1629,10 +1646,10 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
                 if (xchg) {
                     void *args[] = {(void *)&A,    (void *)&lda,  (void *)&js,    (void *)&M,
                                     (void *)&w,    (void *)&RB,   (void *)&ipiv,  (void *)&x_pk,
-                                    (void *)&x_rw, (void *)&x_cw, (void *)&x_val, (void *)&ctx->flags};
+                                    (void *)&x_rw, (void *)&x_cw, (void *)&ctx->flags};
                     if (!(coop && coop_launch(ctx->stream, (const void *)k_panel_x<R>, G, args, lds_x, &coop))) {
                         k_panel_x<R><<<G, 256, lds_x, ctx->stream>>>(A, lda, js, M, w, RB, ipiv, x_pk, x_rw, x_cw,
-                                                                     x_val, ctx->flags);
+                                                                     ctx->flags);
                         EMFA_HIP_CHECK(hipGetLastError());
                     }
                 } else {
