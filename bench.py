@@ -492,12 +492,11 @@ def main():
     ctx.prof(False)
     # the FP32 fill: k_fill_pairs (T^2 Q^2 Green's evaluations, writing the
     # per-triangle-pair scratch of 9 complex values per pair) and k_fill_gather
-    # (per side of every RWG: two scratch reads and a read-modify-write of Z
-    # per entry), beside the N^2 complex entries of Z itself
+    # (four scratch reads and one write of Z per entry)
     T = int(tri.shape[0])
     pairs_ms, gather_ms = fams["fill_pairs"]["ms_per_step"], fams["fill_gather"]["ms_per_step"]
     scratch_b = 9.0 * T * T * 8
-    gather_b = 2 * (2 * 8.0 + 2 * 8.0) * n * n
+    gather_b = (4 * 8.0 + 8.0) * n * n
     z_b = 8.0 * n * n
     fill_roof = {
         "pairs": {"ms": pairs_ms, "green_evals": fams["fill_pairs"]["work_per_step"],
@@ -510,18 +509,18 @@ def main():
                    "frac_hbm": gather_b / (gather_ms * 1e-3) / 1e9 / PEAK["hbm"] if gather_ms > 0 else 0.0,
                    "bound": "hbm"},
         "z_bytes": z_b,
-        "traffic_over_z": (scratch_b + gather_b + z_b) / z_b,
-        "note": "bytes as the kernels move them (scratch write, two scratch reads and a read-modify-write of Z "
-                "per entry and side, the zeroing of Z), not counter readings",
+        "traffic_over_z": (scratch_b + gather_b) / z_b,
+        "note": "bytes as the kernels move them (scratch write, four scratch reads and one write of Z per entry), "
+                "not counter readings",
     }
     # the dominant kernel: the trailing update of the outer panels -- bf16-split
-    # planes (k_gemm_bf3r, bf16 MFMA) when the tuner chose them, else FP32 MFMA
+    # planes (k_gemm_bf3, bf16 MFMA) when the tuner chose them, else FP32 MFMA
     split = fams["lu_gemm_split"]["launches_per_step"] > 0
     g = fams["lu_gemm_split" if split else "lu_gemm"]
     gemm_tflops = g["work_per_step"] / (g["ms_per_step"] * 1e-3) / 1e12 if g["ms_per_step"] > 0 else 0.0
     avg_launch_ms = g["ms_per_step"] / max(g["launches_per_step"], 1)
     if split:
-        roof = {"bound": "mfma", "kernel": "lu_gemm_split (k_gemm_bf3r, V_MFMA_F32_32X32X16_BF16, 3 products)",
+        roof = {"bound": "mfma", "kernel": "lu_gemm_split (k_gemm_bf3, V_MFMA_F32_32X32X16_BF16, 3 products)",
                 "achieved": gemm_tflops, "peak": PEAK["bf16_mfma"], "unit": "TFLOP/s",
                 "frac": gemm_tflops / PEAK["bf16_mfma"],
                 "traffic": TRAFFIC_SPLIT_30720["measured"] if n == 30720 else None,

@@ -1102,9 +1102,8 @@ static emfa_status trsm_blocked(emfa_ctx *ctx, const cx<R> *F, long long ldf, cx
 // factor, turn each diagonal solve of a triangular solve into a product:
 // a solve is then two launches per 256-row block (k_dinv_apply and the MFMA
 // update of the remaining rows).
-// k_tri_inv (FP64 factors; FP32 factors use k_dinv_diag / k_dinv_off below,
-// the same recurrences spread over one workgroup per tile): one workgroup
-// per block and triangle.  The block is handled as 4 x 4 tiles of 64: each
+// k_tri_inv (FP64 factors; FP32 factors use the inverses of nopiv.hip): one
+// workgroup per block and triangle.  The block is handled as 4 x 4 tiles of 64: each
 // diagonal tile is inverted in LDS (one lane per column, unit diagonal for
 // L), the off-diagonal tiles of the inverse follow from
 //   L: X_ij = -D_i sum_{k=j}^{i-1} T_ik X_kj   (i > j, i ascending)
