@@ -1528,9 +1528,8 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
         if (const char *e = getenv("EMFA_LU_BF16X3")) split_update = atoi(e) != 0;
     }
     size_t planes_b = split_update ? UpdatePlanes::bytes(N, nb) : 0;
-    // pivot-free panels: U11^-1 of the current one, L^-1 of the outer block's 256-blocks
-    const int nli = (nb + kInvB - 1) / kInvB;
-    const size_t uinv_b = ((size_t)kNoPivW * kNoPivW + (size_t)nli * kInvB * kInvB) * sizeof(cx<R>);
+    // pivot-free panels: U11^-1 of the current one, L11^-1 of the outer block's
+    const size_t tile = (size_t)kNoPivW * kNoPivW, uinv_b = (1 + (nb + kNoPivW - 1) / kNoPivW) * tile * sizeof(cx<R>);
     size_t total = slot_rows_b + slot_val_b + slot_idx_b + rowc_b + bar_b + 2 * bt_b + perm_b + x_pk_b + x_rw_b +
                    x_cw_b + planes_b + uinv_b + 8192;
     // a batch: one slab of this layout per matrix (plus its flags and pivots)
@@ -1563,7 +1562,7 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     UpdatePlanes planes;
     if (split_update) planes.carve(take(planes_b), N, nb);
     cx<R> *uinv = (cx<R> *)take(uinv_b);
-    cx<R> *linv = uinv + kNoPivW * kNoPivW;
+    cx<R> *linv = uinv + tile;
     // growth flags and pivots: the context's for one matrix, each slab's for a batch
     int *flagsp = batched ? (int *)take(256) : ctx->flags;
     int *ipivp = batched ? (int *)take((size_t)N * sizeof(int)) : ipiv;
@@ -1609,11 +1608,10 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
             const bool right = js + w < j0 + jb;  // panel columns right of the block
             if constexpr (sizeof(R) == 4) {
                 ProfScope ps(ctx, "lu_panel", 0);
-                const int o = js - j0, t = o % kInvB;
-                cx<R> *li = linv + (size_t)(o / kInvB) * kInvB * kInvB + (size_t)t * kInvB + t;
-                st = nopiv_diag_launch(ctx->stream, A, lda, js, w, ipivp, flagsp, tau2, uinv, li, kInvB, ctx->batch);
+                cx<R> *li = linv + (js - j0) / kNoPivW * tile;
+                st = nopiv_diag_launch(ctx->stream, A, lda, js, w, ipivp, flagsp, tau2, uinv, li, ctx->batch);
                 if (!st)
-                    st = nopiv_rows_launch(ctx->stream, A, lda, js, w, N, uinv, li, kInvB, flagsp, tau2, js + w,
+                    st = nopiv_rows_launch(ctx->stream, A, lda, js, w, N, uinv, li, flagsp, tau2, js + w,
                                            right ? j0 + jb : 0, Bt_in, 2LL * w, ctx->batch);
                 if (st) return st;
             }
@@ -1625,11 +1623,6 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
             }
             js += w;
         }
-        if constexpr (sizeof(R) == 4)
-            if (nopiv && j0 + jb < N) {
-                ProfScope ps(ctx, "lu_panel", 0);
-                return nopiv_linv_launch(ctx->stream, A + (size_t)j0 * lda + j0, lda, jb, linv, ctx->batch);
-            }
         while (js < j0 + jb) {
             const int M = N - js;
             int w = std::min(plan.w, j0 + jb - js);
@@ -1686,17 +1679,17 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
         emfa_status s2 = nopiv ? EMFA_OK : laswp_launch<R>(ctx, A, lda, ipiv, j0, j0 + jb, 0, j0, j0 + jb, N, pws);
         if (s2) return s2;
         if constexpr (sizeof(R) == 4) {
-            // U rows through the inverses of L's 256-blocks
-            for (int o = 0; nopiv && o < jb && j0 + jb < N; o += kInvB) {
-                const int wb = std::min(kInvB, jb - o), r0 = j0 + o;
-                for (int u = 0; u < o; u += kInvB) {
-                    s2 = gemm_update<R>(ctx, "trsm_gemm", wb, N - j0 - jb, kInvB, A + (size_t)r0 * lda + j0 + u, lda,
+            for (int o = 0; nopiv && o < jb && j0 + jb < N; o += kURows) {
+                const int wb = std::min(kURows, jb - o), r0 = j0 + o;
+                for (int u = 0; u < o; u += kURows) {
+                    s2 = gemm_update<R>(ctx, "trsm_gemm", wb, N - j0 - jb, kURows, A + (size_t)r0 * lda + j0 + u, lda,
                                         Bt_out + 2 * u, 2LL * jb, A + (size_t)r0 * lda + j0 + jb, lda);
                     if (s2) return s2;
                 }
                 ProfScope ps(ctx, "lu_trsm", 0);
                 s2 = nopiv_urows_launch(ctx->stream, A, lda, r0, wb, j0 + jb, N,
-                                        linv + (size_t)(o / kInvB) * kInvB * kInvB, Bt_out, 2LL * jb, o, ctx->batch);
+                                        linv + o / kNoPivW * tile, Bt_out, 2LL * jb, o,
+                                        share > 0 ? std::min(share, ctx->num_cu) : ctx->num_cu, ctx->batch);
                 if (s2) return s2;
             }
             if (nopiv) return EMFA_OK;

@@ -26,12 +26,15 @@ __device__ __forceinline__ f4 mfma(float a, float b, f4 acc) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
 }
 
-// two complex steps of K: a = {A[.][k], A[.][k+1]}, x0 / x1 = column values
-__device__ __forceinline__ f4 mac2(f4 acc, f4 a, cf x0, cf x1, bool odd) {
+// two complex steps of K: a = {A[.][k], A[.][k+1]}, x0 / x1 = column values.  One
+// sum in K's order: in products with the inverse of a block of large multipliers
+// neighbouring terms cancel, and two sums of half the terms each made factors 2
+// to 3 times less accurate.
+__device__ __forceinline__ void mac2(f4 &acc, f4 a, cf x0, cf x1, bool odd) {
     acc = mfma(a.x, odd ? x0.im : x0.re, acc);
     acc = mfma(a.y, odd ? x0.re : -x0.im, acc);
     acc = mfma(a.z, odd ? x1.im : x1.re, acc);
-    return mfma(a.w, odd ? x1.re : -x1.im, acc);
+    acc = mfma(a.w, odd ? x1.re : -x1.im, acc);
 }
 
 __device__ __forceinline__ float rlane(float v, int l) {
@@ -42,6 +45,87 @@ __device__ __forceinline__ void fms(cf &x, cf a, cf b) {  // x -= a b
     x.re = fmaf(-a.re, b.re, fmaf(a.im, b.im, x.re));
     x.im = fmaf(-a.re, b.im, fmaf(-a.im, b.re, x.im));
 }
+
+// Orders a wave's own LDS accesses: its lanes read what other lanes of it wrote.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Forward substitution with a unit-lower 64 x 64 block for 8 complex columns by
+// one wave, 16 rows at a time: the tiles below the diagonal and the inverses of
+// the 16 x 16 diagonal tiles less the identity, as left operands.  Inverses no
+// larger than 16 keep the error at |L| |U| as substitution by single rows has
+// it; a 256-row inverse in its place (U = L^-1 A) made factors of matrices with
+// multipliers of 10 to 90 four to eight times less accurate at 1100 unknowns.
+struct Sub64 {
+    f4 d[4][2], l[6][2];
+
+    // L: the factored block (w x w), inv: L^-1 - I (64 x 64)
+    __device__ __forceinline__ void load(const cf *L, long long ldl, const cf *inv, int w, int lane) {
+        const int l16 = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                d[i][q] = *(const f4 *)(inv + (16 * i + l16) * kNoPivW + 16 * i + 8 * q + 2 * g);
+        // rows past the block read its last one and count as zero
+#pragma unroll
+        for (int b = 1; b < 4; ++b) {
+            const cf *Lr = L + min(16 * b + l16, w - 1) * ldl + 2 * g;
+#pragma unroll
+            for (int i = 0; i < b; ++i)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) l[b * (b - 1) / 2 + i][q] = *(const f4_a8 *)(Lr + 16 * i + 8 * q);
+        }
+        if (w < 64) {
+#pragma unroll
+            for (int b = 1; b < 4; ++b)
+#pragma unroll
+                for (int i = 0; i < 2 * b; ++i)
+                    if (16 * b + l16 >= w) l[b * (b - 1) / 2 + (i >> 1)][i & 1] = f4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+
+    // v: the columns, tile i holding rows 16 i + 4 g + r, real column l16; X: 64
+    // rows of 8 columns in LDS (row stride ldx), left with the result as v is
+    __device__ __forceinline__ void solve(f4 *v, cf *X, int ldx, int lane) const {
+        const int l16 = lane & 15, g = lane >> 4;
+        const bool odd = l16 & 1;
+        f4 p[4];
+        cf x[4], y[4];  // a tile's rows and those of the last finished tile, as right operands
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = f4{0.f, 0.f, 0.f, 0.f};
+        auto turn = [&](int i, cf *o) {
+            cf *Xi = X + 16 * i * ldx;
+            wave_sync();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ((float *)(Xi + (4 * g + r) * ldx))[l16] = v[i][r];
+            wave_sync();
+#pragma unroll
+            for (int h = 0; h < 4; ++h) o[h] = Xi[(8 * (h >> 1) + 2 * g + (h & 1)) * ldx + (l16 >> 1)];
+        };
+        auto off = [&](int b, int i) {  // p[b] += L's tile (b, i) times tile i
+#pragma unroll
+            for (int q = 0; q < 2; ++q) mac2(p[b], l[b * (b - 1) / 2 + i][q], y[2 * q], y[2 * q + 1], odd);
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i) off(i, i - 1);
+            v[i] -= p[i];
+            turn(i, x);
+            // behind the trip through LDS
+#pragma unroll
+            for (int b = i + 1; i && b < 4; ++b) off(b, i - 1);
+            f4 e = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < 2; ++q) mac2(e, d[i][q], x[2 * q], x[2 * q + 1], odd);
+            v[i] += e;
+            turn(i, y);
+        }
+    }
+};
 
 // A 64 x 64 triangular pair in LDS: the factored block and the inverses of its
 // unit-lower and upper triangles, one array so that join64's operands are
@@ -119,7 +203,7 @@ __device__ __forceinline__ void join64(Tri64 &T, int tris, int wave, int lane) {
                 f4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma nounroll
                 for (int k = k0; k < k1; k += 8)
-                    acc = mac2(acc, *(const f4 *)(Al + k), Bl[k * kLd], Bl[(k + 1) * kLd], odd);
+                    mac2(acc, *(const f4 *)(Al + k), Bl[k * kLd], Bl[(k + 1) * kLd], odd);
                 const float sign = step == 0 ? 1.f : -1.f;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -146,15 +230,14 @@ __device__ __forceinline__ void join64(Tri64 &T, int tris, int wave, int lane) {
 // earlier ones only.
 // Then both 64 x 64 inverses: 8 x 8 blocks by substitution, one column per lane,
 // joined on the matrix cores.
-// 23 us per block (LU 14, inverses 6); 39 us with a barrier per four columns
+// 21 us per block (LU 14, inverses 6); 39 us with a barrier per four columns
 // and one VALU inverse by doubling.
 // ---------------------------------------------------------------------------
 constexpr int kDiagThreads = 1024;
 
 __global__ __launch_bounds__(kDiagThreads) void k_nopiv_diag(cf *__restrict__ A, long long lda, int js, int w,
                                                              int *__restrict__ ipiv, int *flags, float tau2,
-                                                             cf *__restrict__ uinv, cf *__restrict__ linv,
-                                                             long long ldl, Batch bt) {
+                                                             cf *__restrict__ uinv, cf *__restrict__ linv, Batch bt) {
     A = batch_mat(bt, A);
     ipiv = batch_scr(bt, ipiv);
     flags = batch_scr(bt, flags);
@@ -264,35 +347,65 @@ __global__ __launch_bounds__(kDiagThreads) void k_nopiv_diag(cf *__restrict__ A,
     join64(T, 3, v, lane);
     for (int r = v; r < 64; r += 16) {
         uinv[(size_t)r * kNoPivW + lane] = lane >= r ? T.m[2][r][lane] : cf{0.f, 0.f};
-        linv[(size_t)r * ldl + lane] = lane <= r ? T.m[1][r][lane] : cf{0.f, 0.f};
+        linv[(size_t)r * kNoPivW + lane] = lane < r ? T.m[1][r][lane] : cf{0.f, 0.f};
     }
     if (tid == 0 && s_bad) flags[2] = 1;
 }
 
 // ---------------------------------------------------------------------------
-// The two products that follow the diagonal block, in one launch: workgroups
-// [0, nl) form 16 rows of L21 = A21 U^-1 (a wave two of the eight column
-// tiles), the others 16 columns of U12 = L^-1 A12 (a wave 16 of the 64 rows).
-// In place: a workgroup's loads are done before its first store, and the
-// workgroups touch disjoint parts of A.  K = 64 throughout: 64 MFMAs per wave
-// behind one round of loads.  6.4 us per launch at 1920 unknowns; 17 us as a
-// VALU product and substitution through LDS.
+// What follows the diagonal block, in one launch: workgroups [0, nl) form 16 rows
+// of L21 = A21 U^-1 (a wave two of the eight column tiles, K = 64: 64 MFMAs
+// behind one round of loads), the others 32 columns of U12 by substitution with
+// L (a wave 8 columns).  In place: a workgroup's (U12: a wave's) loads are done
+// before its first store, and they touch disjoint parts of A.  8.1 us per launch
+// at 1920 unknowns (6.4 with U12 = L^-1 A12 by an explicit inverse, 17 as a VALU
+// product and substitution through LDS).
 // ---------------------------------------------------------------------------
+constexpr int kSubLd = 10;  // sixteen lanes' rows four apart on different banks
+
 __global__ __launch_bounds__(256) void k_nopiv_rows(cf *__restrict__ A, long long lda, int js, int w, int N,
                                                     const cf *__restrict__ uinv, const cf *__restrict__ linv,
-                                                    long long ldl, int *flags, float tau2, int nl, int c0, int c1,
+                                                    int *flags, float tau2, int nl, int c0, int c1,
                                                     float *__restrict__ Bt, long long ldbt, Batch bt) {
+    __shared__ cf Xs[4][64 * kSubLd];
     A = batch_mat(bt, A);
     uinv = batch_scr(bt, uinv);
     linv = batch_scr(bt, linv);
     flags = batch_scr(bt, flags);
     Bt = batch_scr(bt, Bt);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
-    const bool odd = l16 & 1, low = (int)blockIdx.x < nl;
-    // rows of the left operand, columns of the right one
-    const int r0 = low ? js + w + 16 * (int)blockIdx.x : 16 * wave;
-    const int cb = low ? 16 * wave : c0 + 16 * ((int)blockIdx.x - nl);
-    const cf *Ar = low ? A + (size_t)min(r0 + l16, N - 1) * lda + js : linv + (size_t)(r0 + l16) * ldl;
+    const bool odd = l16 & 1;
+    if ((int)blockIdx.x >= nl) {
+        const int cb = c0 + 32 * ((int)blockIdx.x - nl) + 8 * wave, j = cb + (l16 >> 1);
+        if (cb >= c1) return;
+        Sub64 op;
+        op.load(A + (size_t)js * lda + js, lda, linv, w, lane);
+        f4 v[4];
+        const float *Aj = (const float *)(A + (size_t)js * lda + min(j, c1 - 1)) + odd;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * i + 4 * g + r;
+                const float x = Aj[2 * min(row, w - 1) * lda];
+                v[i][r] = row < w ? x : 0.f;
+            }
+        op.solve(v, Xs[wave], kSubLd, lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * i + 4 * g + r;
+                const float x = v[i][r], other = __shfl_xor(x, 1);
+                if (row >= w || j >= c1) continue;
+                ((float *)(A + (size_t)(js + row) * lda + j))[odd] = x;
+                // expanded operand: rows 2j {Re, -Im}, 2j + 1 {Im, Re}
+                *(float2 *)(Bt + (2LL * (j - c0) + odd) * ldbt + 2 * row) = make_float2(x, odd ? other : -other);
+            }
+        return;
+    }
+    const int r0 = js + w + 16 * (int)blockIdx.x;
+    const cf *Ar = A + (size_t)min(r0 + l16, N - 1) * lda + js;
     f4 a[8];
     if (w == 64) {
 #pragma unroll
@@ -308,42 +421,26 @@ __global__ __launch_bounds__(256) void k_nopiv_rows(cf *__restrict__ A, long lon
     f4 acc[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int j = cb + 8 * t + (l16 >> 1);
-        const cf *X = low ? uinv + j : A + (size_t)js * lda + min(j, c1 - 1);
-        const long long ldx = low ? kNoPivW : lda;
+        const cf *X = uinv + 16 * wave + 8 * t + (l16 >> 1);
         acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-        cf x[16];
 #pragma unroll
-        for (int q = 0; q < 8; ++q)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int k = 8 * q + 2 * g + h;
-                x[2 * q + h] = k < w ? X[k * ldx] : cf{0.f, 0.f};
-            }
-#pragma unroll
-        for (int q = 0; q < 8; ++q) acc[t] = mac2(acc[t], a[q], x[2 * q], x[2 * q + 1], odd);
+        for (int q = 0; q < 8; ++q) {
+            const int k = 8 * q + 2 * g;
+            mac2(acc[t], a[q], X[k * kNoPivW], X[(k + 1) * kNoPivW], odd);
+        }
     }
     __syncthreads();
     bool bad = false;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int j = cb + 8 * t + (l16 >> 1);
+        const int j = 16 * wave + 8 * t + (l16 >> 1);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float v = acc[t][i], other = __shfl_xor(v, 1);
             const int r = r0 + 4 * g + i;
-            if (low) {
-                if (r < N && j < w) {
-                    ((float *)(A + (size_t)r * lda + js + j))[odd] = v;
-                    if (v * v + other * other > tau2) bad = true;
-                }
-            } else if (r < w && j < c1) {
-                ((float *)(A + (size_t)(js + r) * lda + j))[odd] = v;
-                // expanded operand: rows 2j {Re, -Im}, 2j + 1 {Im, Re}
-                float *b = Bt + (2LL * (j - c0) + odd) * ldbt + 2 * r;
-                b[0] = v;
-                b[1] = odd ? other : -other;
-            }
+            if (r >= N || j >= w) continue;
+            ((float *)(A + (size_t)r * lda + js + j))[odd] = v;
+            if (v * v + other * other > tau2) bad = true;
         }
     }
     if (bad) flags[2] = 1;
@@ -398,11 +495,11 @@ __global__ __launch_bounds__(kDiagThreads) void k_inv_diag(const cf *__restrict_
 
 template <int B>
 __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long long ldf, int N,
-                                                  cf *__restrict__ Dinv, int nblk, int scr, Batch bf, Batch bd) {
+                                                  cf *__restrict__ Dinv, int nblk, Batch bf, Batch bd) {
     constexpr int STRIPS = B / 8, PAIRS = kInvB / (2 * B), RT = B / 64;  // 16-row tiles per wave
     __shared__ cf C[B][12];
     F = batch_mat(bf, F);
-    Dinv = scr ? batch_scr(bd, Dinv) : batch_mat(bd, Dinv);
+    Dinv = batch_mat(bd, Dinv);
     const int c = 8 * ((int)blockIdx.x % STRIPS), pr = (int)blockIdx.x / STRIPS, blk = pr / PAIRS;
     const int s0 = 2 * B * (pr % PAIRS), s1 = s0 + B, r0 = blk * kInvB;
     const bool up = blockIdx.y != 0;
@@ -428,8 +525,7 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
 #pragma unroll
                 for (int k = h; k < h + 64; k += 8) {
                     const int ka = k + 2 * g;
-                    acc = mac2(acc, *(const f4_a8 *)(Ar + ka), Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB],
-                               odd);
+                    mac2(acc, *(const f4_a8 *)(Ar + ka), Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB], odd);
                 }
             }
         } else {
@@ -444,7 +540,7 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
                     a.z = Ar[ka + 1].re;
                     a.w = Ar[ka + 1].im;
                 }
-                acc = mac2(acc, a, Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB], odd);
+                mac2(acc, a, Xs[(size_t)ka * kInvB], Xs[(size_t)(ka + 1) * kInvB], odd);
             }
         }
 #pragma unroll
@@ -463,7 +559,7 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
 #pragma unroll
             for (int k = h; k < h + 64; k += 8) {
                 const int ka = k + 2 * g;
-                acc = mac2(acc, *(const f4 *)(Ar + ka), C[ka][l16 >> 1], C[ka + 1][l16 >> 1], odd);
+                mac2(acc, *(const f4 *)(Ar + ka), C[ka][l16 >> 1], C[ka + 1][l16 >> 1], odd);
             }
         }
 #pragma unroll
@@ -472,121 +568,153 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
 }
 
 // ---------------------------------------------------------------------------
-// U rows of a 256-row block: U = L^-1 A on its rows, for 8 CT columns per
-// workgroup, in place (the columns go to LDS first).  Wave v takes 16-row
-// tiles v and 15 - v, so the triangle's work is even.  Against the blocked
-// substitution it replaces (per 64 rows one substitution and one update
-// launch, 15 launches and 176 us per 512 rows at 1920 unknowns) it is one
-// launch per 256 rows: 50 us with the update between the two.
+// U rows of a 256-row block by substitution with L, for 8 CT columns per
+// workgroup, in place (the columns in LDS): per 64 rows a wave and column tile
+// substitutes (Sub64) while the other waves take the last 64 rows' part off the
+// tiles below.  Wave v owns the 16-row tiles v and 15 - v, so the triangle's
+// work is even.  L's tiles and the substitution's operands are loaded a block ahead.
+// A chain of four substitutions: 21 us per launch at 1920 unknowns, where the
+// product with L's explicit inverse took 15 and that inverse 20 more per block,
+// and blocked substitution in launches of 64 rows 176 us per 512 rows.
 // ---------------------------------------------------------------------------
 template <int CT>
 __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long long lda, int r0, int wb, int c0,
-                                                     int c1, const cf *__restrict__ Li, float *__restrict__ Bt,
+                                                     int c1, const cf *__restrict__ linv, float *__restrict__ Bt,
                                                      long long ldbt, int kofs, Batch bt) {
-    constexpr int S = 8 * CT;
-    __shared__ cf Xs[kInvB][S + 4];
+    constexpr int S = 8 * CT, LD = S + 2;
+    __shared__ cf Xs[kURows * LD];
     A = batch_mat(bt, A);
-    Li = batch_scr(bt, Li);
+    linv = batch_scr(bt, linv);
     Bt = batch_scr(bt, Bt);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15,
+              g = lane >> 4;
     const bool odd = l16 & 1;
-    const int cb = c0 + S * (int)blockIdx.x;
-#pragma unroll 4
-    for (int e = tid; e < kInvB * S; e += 512) {
-        const int k = e / S, j = e % S;
-        Xs[k][j] = (k < wb && cb + j < c1) ? A[(size_t)(r0 + k) * lda + cb + j] : cf{0.f, 0.f};
-    }
-    __syncthreads();
+    const int cb = c0 + S * (int)blockIdx.x, nc = min(S, c1 - cb);
+    const cf *L = A + (size_t)r0 * lda + r0;
+    const int tile[2] = {wave, 15 - wave}, solver = wave - (8 - CT);  // column tile that the wave substitutes
+    const int nst = (wb + 63) / 64;
+    f4 l[2][8];
+    Sub64 op;
+    // L's tile in block column s
+    auto load_l = [&](int h, int s) {
+        const cf *Lr = L + (size_t)min(16 * tile[h] + l16, wb - 1) * lda + 64 * s + 2 * g;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const int r = 16 * (half ? 15 - wave : wave);
-        if (r >= wb) continue;
-        const cf *Ar = Li + (size_t)(r + l16) * kInvB + 2 * g;
-        f4 acc[CT], a[4];
-#pragma unroll
-        for (int t = 0; t < CT; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-        // steps of 32 of K, the next step's rows of L^-1 loaded ahead; the
-        // last step may reach past the tile's diagonal, where L^-1 is zero
-#pragma unroll
-        for (int q = 0; q < 4; ++q) a[q] = *(const f4 *)(Ar + 8 * q);
-        for (int k = 0; k < r + 16; k += 32) {
-            f4 nx[4];
-            const int kn = min(k + 32, kInvB - 32);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) nx[q] = *(const f4 *)(Ar + kn + 8 * q);
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int t = 0; t < CT; ++t)
-                    acc[t] = mac2(acc[t], a[q], Xs[k + 8 * q + 2 * g][8 * t + (l16 >> 1)],
-                                  Xs[k + 8 * q + 2 * g + 1][8 * t + (l16 >> 1)], odd);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) a[q] = nx[q];
-        }
+        for (int q = 0; q < 8; ++q) l[h][q] = *(const f4_a8 *)(Lr + 8 * q);
+    };
+    auto load_op = [&](int s) {
+        op.load(L + (size_t)64 * s * lda + 64 * s, lda, linv + (size_t)s * kNoPivW * kNoPivW,
+                min(64, wb - 64 * s), lane);
+    };
+    // the tile's columns less L's tile times the rows of block s
+    auto update = [&](int h, int s) {
+        const cf *X = Xs + (64 * s + 2 * g) * LD + (l16 >> 1);
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
-            const int j = cb + 8 * t + (l16 >> 1);
-            float o[4];
+            f4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = __shfl_xor(acc[t][i], 1) * (odd ? 1.f : -1.f);
-            if (j >= c1) continue;
-            // expanded operand: rows 2j {Re, -Im}, 2j + 1 {Im, Re}
-            float *b = Bt + (2LL * (j - c0) + odd) * ldbt + 2 * (kofs + r + 4 * g);
+            for (int q = 0; q < 8; ++q) mac2(p, l[h][q], X[8 * q * LD + 8 * t], X[(8 * q + 1) * LD + 8 * t], odd);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (r + 4 * g + i >= wb) continue;
-                ((float *)(A + (size_t)(r0 + r + 4 * g + i) * lda + j))[odd] = acc[t][i];
-                *(float2 *)(b + 2 * i) = make_float2(acc[t][i], o[i]);
-            }
+            for (int i = 0; i < 4; ++i) ((float *)(Xs + (16 * tile[h] + 4 * g + i) * LD + 8 * t))[l16] -= p[i];
+        }
+    };
+    if (solver >= 0) load_op(0);
+    {
+        cf x[kURows * S / 512];
+#pragma unroll
+        for (int i = 0; i < kURows * S / 512; ++i) {
+            const int e = tid + 512 * i;
+            x[i] = A[(size_t)(r0 + min(e / S, wb - 1)) * lda + cb + min(e % S, nc - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < kURows * S / 512; ++i) {
+            const int e = tid + 512 * i;
+            Xs[e / S * LD + e % S] = (e / S < wb && e % S < nc) ? x[i] : cf{0.f, 0.f};
         }
     }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        if (tile[h] >= 4 && 16 * tile[h] < wb) load_l(h, 0);
+    __syncthreads();
+    for (int s = 0; s < nst; ++s) {
+        if (s) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (tile[h] >> 2 == s && 16 * tile[h] < wb) update(h, s - 1);
+            __syncthreads();
+        }
+        if (solver >= 0) {
+            cf *X = Xs + 64 * s * LD + 8 * solver;
+            f4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[i][r] = ((const float *)(X + (16 * i + 4 * g + r) * LD))[l16];
+            op.solve(v, X, LD, lane);
+            if (s + 1 < nst) load_op(s + 1);
+        }
+        // beside it, the tiles of later blocks
+        if (s) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (tile[h] >> 2 > s && 16 * tile[h] < wb) {
+                    update(h, s - 1);
+                    load_l(h, s);
+                }
+        }
+        __syncthreads();
+    }
+    for (int e = tid; e < wb * S; e += 512) {
+        const int k = e / S, j = e % S;
+        if (j < nc) A[(size_t)(r0 + k) * lda + cb + j] = Xs[k * LD + j];
+    }
+    // expanded operand: rows 2j {Re, -Im}, 2j + 1 {Im, Re}
+    for (int j = wave; j < nc; j += 8)
+        for (int k = lane; k < wb; k += 64) {
+            const cf x = Xs[k * LD + j];
+            float *b = Bt + 2LL * (cb - c0 + j) * ldbt + 2 * (kofs + k);
+            *(float2 *)b = make_float2(x.re, -x.im);
+            *(float2 *)(b + ldbt) = make_float2(x.im, x.re);
+        }
 }
 
 }  // namespace
 
 emfa_status nopiv_diag_launch(hipStream_t s, cf *A, long long lda, int js, int w, int *ipiv, int *flags, float tau2,
-                              cf *uinv, cf *linv, long long ldl, const Batch &bt) {
-    EMFA_REQUIRE(w >= 1 && w <= kNoPivW && ldl >= kNoPivW, EMFA_E_INVALID, "pivot-free panel of width %d", w);
-    k_nopiv_diag<<<dim3(1, 1, bt.count), kDiagThreads, 0, s>>>(A, lda, js, w, ipiv, flags, tau2, uinv, linv, ldl, bt);
+                              cf *uinv, cf *linv, const Batch &bt) {
+    EMFA_REQUIRE(w >= 1 && w <= kNoPivW, EMFA_E_INVALID, "pivot-free panel of width %d", w);
+    k_nopiv_diag<<<dim3(1, 1, bt.count), kDiagThreads, 0, s>>>(A, lda, js, w, ipiv, flags, tau2, uinv, linv, bt);
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
 }
 
 emfa_status nopiv_rows_launch(hipStream_t s, cf *A, long long lda, int js, int w, int N, const cf *uinv,
-                              const cf *linv, long long ldl, int *flags, float tau2, int c0, int c1, float *Bt,
-                              long long ldbt, const Batch &bt) {
-    const int nl = (N - js - w + 15) / 16, nu = std::max(0, (c1 - c0 + 15) / 16);
+                              const cf *linv, int *flags, float tau2, int c0, int c1, float *Bt, long long ldbt,
+                              const Batch &bt) {
+    const int nl = (N - js - w + 15) / 16, nu = std::max(0, (c1 - c0 + 31) / 32);
     if (nl + nu <= 0) return EMFA_OK;
-    k_nopiv_rows<<<dim3(nl + nu, 1, bt.count), 256, 0, s>>>(A, lda, js, w, N, uinv, linv, ldl, flags, tau2, nl, c0,
-                                                            c1, Bt, ldbt, bt);
+    k_nopiv_rows<<<dim3(nl + nu, 1, bt.count), 256, 0, s>>>(A, lda, js, w, N, uinv, linv, flags, tau2, nl, c0, c1, Bt,
+                                                            ldbt, bt);
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
 }
 
-emfa_status nopiv_linv_launch(hipStream_t s, const cf *F, long long ldf, int n, cf *Li, const Batch &bt) {
-    const int nblk = (n + kInvB - 1) / kInvB;
-    if (n > 64) k_inv_join<64><<<dim3(nblk * 16, 1, bt.count), 256, 0, s>>>(F, ldf, n, Li, nblk, 1, bt, bt);
-    if (n > 128) k_inv_join<128><<<dim3(nblk * 16, 1, bt.count), 256, 0, s>>>(F, ldf, n, Li, nblk, 1, bt, bt);
-    EMFA_HIP_CHECK(hipGetLastError());
-    return EMFA_OK;
-}
-
-emfa_status nopiv_urows_launch(hipStream_t s, cf *A, long long lda, int r0, int wb, int c0, int c1, const cf *Li,
-                               float *Bt, long long ldbt, int kofs, const Batch &bt) {
+emfa_status nopiv_urows_launch(hipStream_t s, cf *A, long long lda, int r0, int wb, int c0, int c1, const cf *linv,
+                               float *Bt, long long ldbt, int kofs, int cus, const Batch &bt) {
     if (c1 <= c0 || wb <= 0) return EMFA_OK;
-    EMFA_REQUIRE(wb <= kInvB, EMFA_E_INVALID, "U rows of a block of %d", wb);
+    EMFA_REQUIRE(wb <= kURows, EMFA_E_INVALID, "U rows of a block of %d", wb);
     const int nc = c1 - c0;
-    // Wider strips read L^-1 fewer times, narrower ones have the shorter chain:
-    // 8 columns while they fill the chip at most twice over (1920 unknowns: 15.6
-    // us per launch, 16 columns 22.5)
+    // A strip's time is its chain's (8, 16, 32 columns 21, 29, 42 us alone), and a
+    // CU holds one workgroup: the narrowest strips that run in one round.  In
+    // factorisations of 1920 / 8321 / 30720 unknowns all strips of 8 columns take
+    // 2.20 / 19.2 / 388 ms, of 16 2.26 / 19.0 / 382, of 32 2.28 / 18.9 / 381.
     const long long cols = (long long)nc * bt.count;
     auto go = [&](auto kernel, int strip) {
-        kernel<<<dim3((nc + strip - 1) / strip, 1, bt.count), 512, 0, s>>>(A, lda, r0, wb, c0, c1, Li, Bt, ldbt, kofs,
+        kernel<<<dim3((nc + strip - 1) / strip, 1, bt.count), 512, 0, s>>>(A, lda, r0, wb, c0, c1, linv, Bt, ldbt, kofs,
                                                                           bt);
     };
-    if (cols >= 16384)
+    if (cols > 16LL * cus)
         go(k_nopiv_urows<4>, 32);
-    else if (cols >= 4096)
+    else if (cols > 8LL * cus)
         go(k_nopiv_urows<2>, 16);
     else
         go(k_nopiv_urows<1>, 8);
@@ -596,8 +724,8 @@ emfa_status nopiv_urows_launch(hipStream_t s, cf *A, long long lda, int r0, int 
 
 emfa_status dinv_f32_launch(hipStream_t s, const cf *F, int N, cf *Dinv, int nblk, const Batch &bf, const Batch &bd) {
     k_inv_diag<<<dim3(nblk * 4, 2, bf.count), kDiagThreads, 0, s>>>(F, N, Dinv, nblk, bf, bd);
-    k_inv_join<64><<<dim3(nblk * 16, 2, bf.count), 256, 0, s>>>(F, N, N, Dinv, nblk, 0, bf, bd);
-    k_inv_join<128><<<dim3(nblk * 16, 2, bf.count), 256, 0, s>>>(F, N, N, Dinv, nblk, 0, bf, bd);
+    k_inv_join<64><<<dim3(nblk * 16, 2, bf.count), 256, 0, s>>>(F, N, N, Dinv, nblk, bf, bd);
+    k_inv_join<128><<<dim3(nblk * 16, 2, bf.count), 256, 0, s>>>(F, N, N, Dinv, nblk, bf, bd);
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
 }

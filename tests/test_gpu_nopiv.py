@@ -1,7 +1,9 @@
 """FP32 factorisations without interchanges (nopiv.hip): the diagonal block, the
-panel's rows and the diagonal-block inverses at ragged sizes."""
+panel's rows and the diagonal-block inverses at ragged sizes, and factors with
+multipliers well above one."""
 import numpy as np
 import pytest
+from scipy.linalg import solve_triangular
 
 from emfa_amd import hip
 
@@ -67,3 +69,91 @@ def test_zero_pivot_and_growth_fall_back_to_interchanges(ctx, n, at):
     assert lu.singular == (at + 1 == n)
     lu.close()
     Z.close()
+
+
+def _lu32(A):
+    """LU without interchanges in complex64, 64 columns at a time: U's rows by
+    substitution, the rows below through U^-1 of the panel"""
+    A = A.astype(np.complex64)
+    n = A.shape[0]
+    for j in range(0, n, 64):
+        e = min(n, j + 64)
+        for k in range(j, e):
+            A[k + 1:e, k] /= A[k, k]
+            A[k + 1:e, k + 1:e] -= np.outer(A[k + 1:e, k], A[k, k + 1:e])
+        if e < n:
+            A[e:, j:e] = A[e:, j:e] @ solve_triangular(A[j:e, j:e], np.eye(e - j, dtype=np.complex64))
+            A[j:e, e:] = solve_triangular(A[j:e, j:e], A[j:e, e:], lower=True, unit_diagonal=True)
+            A[e:, e:] -= A[e:, j:e] @ A[j:e, e:]
+    return A.astype(np.complex128)
+
+
+def _solution_error(F, B, want):
+    X = solve_triangular(F, solve_triangular(F, B, lower=True, unit_diagonal=True))
+    return np.linalg.norm(X - want) / np.linalg.norm(want)
+
+
+# Small shifts leave multipliers of 10 to 100.  One outer block with U rows
+# beside it, a ragged second 256-block of an outer block, several outer blocks;
+# FP32 and bf16-split updates.
+@pytest.mark.parametrize("n,nb,split,shift", [(300, 256, 0, 1.0), (400, 300, 0, 1.0), (790, 320, 1, 1.0),
+                                              (1100, 256, 0, 1.0), (1100, 256, 0, 0.5), (1100, 512, 0, 1.0)])
+def test_large_multipliers_cost_no_more_than_substitution(n, nb, split, shift):
+    ctx = hip.Context(0)
+    ctx.lu_params(nb, 0, 2)
+    ctx.lu_update_mode(split)
+    logs = []
+    for seed in range(12):
+        rng = np.random.default_rng(7 * seed + n)
+        A = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n)) + shift * np.sqrt(n) * np.eye(n)
+        A = A.astype(np.complex64).astype(np.complex128)
+        B = rng.standard_normal((n, 3)) + 1j * rng.standard_normal((n, 3))
+        Z = hip.Mat.from_numpy(ctx, A, hip.F32)
+        lu = hip.LU(ctx, Z, hip.F32)
+        if lu.pivoting() == (0, 0):
+            F, want = lu.factor().numpy(), np.linalg.solve(A, B)
+            assert np.abs(np.tril(F, -1)).max() <= 100
+            if not split:
+                logs.append(np.log(_solution_error(F, B, want) / _solution_error(_lu32(A), B, want)))
+            dB, X = hip.Mat.from_numpy(ctx, B), hip.Mat(ctx, n, 3)
+            rep, ok = hip.refine(ctx, Z, lu, dB, X, 1e-10, 30)
+            assert ok and np.linalg.norm(X.numpy() - want) <= 1e-10 * np.linalg.cond(A) * np.linalg.norm(want)
+            for x in (dB, X):
+                x.close()
+        lu.close()
+        Z.close()
+        if len(logs) == 8:
+            break
+    if not split:
+        assert len(logs) >= 4
+        # The mean ratio of the two errors: at most sqrt(2) from the matrix cores'
+        # two roundings per complex step, and three deviations of a mean of
+        # single ratios that spread by a factor of e^0.6
+        assert np.mean(logs) <= 0.5 * np.log(2) + 3 * 0.6 / np.sqrt(len(logs))
+    ctx.close()
+
+
+# runs of one and two multipliers of 5 to 90: inverses of L hold their products
+@pytest.mark.parametrize("n,t,run", [(300, 90, 1), (515, 10, 2), (1100, 90, 1)])
+def test_runs_of_large_multipliers_refine(ctx, n, t, run):
+    rng = np.random.default_rng(n + t)
+    L = np.eye(n, dtype=np.complex128) + np.tril(rng.standard_normal((n, n)), -1) / n
+    for k in range(n - 1):
+        if k % (run + 1) != run:
+            L[k + 1, k] = rng.uniform(5, t) * np.exp(2j * np.pi * rng.random())
+    U = np.triu(rng.standard_normal((n, n)), 1) / np.sqrt(n) + np.diag(1 + rng.random(n))
+    A = (L @ U).astype(np.complex64).astype(np.complex128)
+    B = rng.standard_normal((n, 2)) + 1j * rng.standard_normal((n, 2))
+    Z = hip.Mat.from_numpy(ctx, A, hip.F32)
+    lu = hip.LU(ctx, Z, hip.F32)
+    assert lu.pivoting() == (0, 0)
+    want = np.linalg.solve(A, B)
+    mine, plain = _solution_error(lu.factor().numpy(), B, want), _solution_error(_lu32(A), B, want)
+    assert mine <= 4 * plain
+    dB, X = hip.Mat.from_numpy(ctx, B), hip.Mat(ctx, n, 2)
+    # FP64 rounds the residual at 2^-53 |A| |X|, far above 1e-12 |B| for some of these
+    floor = 8 * 2.0 ** -53 * np.linalg.norm(A) * np.linalg.norm(want) / np.linalg.norm(B, axis=0).min()
+    rep, ok = hip.refine(ctx, Z, lu, dB, X, max(1e-12, floor), 6)
+    assert ok
+    for x in (lu, Z, dB, X):
+        x.close()
