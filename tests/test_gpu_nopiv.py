@@ -93,6 +93,25 @@ def _solution_error(F, B, want):
     return np.linalg.norm(X - want) / np.linalg.norm(want)
 
 
+# one diagonal block with multipliers below one, where every rounding counts alike
+@pytest.mark.parametrize("n", [20, 32, 64])
+def test_diagonal_block_rounds_once_per_product(ctx, n):
+    logs = []
+    for seed in range(16):
+        rng = np.random.default_rng(seed + n)
+        A = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n)) + 2 * np.sqrt(n) * np.eye(n)
+        A = A.astype(np.complex64).astype(np.complex128)
+        Z = hip.Mat.from_numpy(ctx, A, hip.F32)
+        lu = hip.LU(ctx, Z, hip.F32)
+        ref = _lu(A)
+        logs.append(np.log(np.linalg.norm(lu.factor().numpy() - ref) / np.linalg.norm(_lu32(A) - ref)))
+        lu.close()
+        Z.close()
+    # the same roundings as complex64's; a second one per product at the size of
+    # the entry makes this sqrt(2)
+    assert np.mean(logs) <= np.log(1.2)
+
+
 # Small shifts leave multipliers of 10 to 100.  One outer block with U rows
 # beside it, a ragged second 256-block of an outer block, several outer blocks;
 # FP32 and bf16-split updates.
