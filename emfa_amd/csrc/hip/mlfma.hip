@@ -37,6 +37,7 @@
 
 #include "em_device.h"
 #include "internal.h"
+#include "parts.h"
 
 namespace emfa {
 
@@ -1108,20 +1109,6 @@ static emfa_status ml_alloc(emfa_mlfma *M, T **dst, size_t count) {
     M->bytes += b;
     *dst = (T *)p;
     return EMFA_OK;
-}
-
-// work(0) .. work(parts - 1), one host thread each where the system grants it
-static void run_parts(int parts, const std::function<void(int)> &work) {
-    std::vector<std::thread> pool;
-    pool.reserve(parts);
-    int t = 1;
-    try {
-        for (; t < parts; ++t) pool.emplace_back(work, t);
-    } catch (...) {  // no more threads: the rest here
-    }
-    for (; t < parts; ++t) work(t);
-    work(0);
-    for (auto &th : pool) th.join();
 }
 
 // Rows row_of[i] of C.trans (rows x K, allocated here, cleared) for the offsets

@@ -56,6 +56,45 @@ def test_server_footprint_model():
     assert serve.unknowns(serve.PLATE, 14) == 560 and serve.unknowns(serve.ICOSPHERE, 3) == 1920
 
 
+PARTS = r"""
+#include <atomic>
+#include <cstdio>
+#include <new>
+#include <stdexcept>
+#include "parts.h"
+int main() {
+    for (int parts : {1, 2, 7, 16})
+        for (int bad = -1; bad < parts; ++bad) {
+            std::atomic<int> ran{0};
+            int caught = 0;
+            try {
+                emfa::run_parts(parts, [&](int t) {
+                    ++ran;
+                    if (t == bad) throw std::bad_alloc();
+                    if (t > bad && bad >= 0) throw std::runtime_error("a later part");
+                });
+            } catch (const std::bad_alloc &) {
+                caught = 1;
+            } catch (...) {
+                caught = 2;
+            }
+            if (ran != parts || caught != (bad >= 0)) return std::printf("%d parts, %d: %d %d", parts, bad, (int)ran, caught), 1;
+        }
+    return 0;
+}
+"""
+
+
+def test_exceptions_of_host_parts_reach_the_caller(tmp_path):
+    # a part that runs out of memory must not end the process
+    (tmp_path / "parts.cpp").write_text(PARTS)
+    exe = str(tmp_path / "parts")
+    subprocess.run(["g++", "-std=c++17", "-pthread", "-I", os.path.join(ROOT, "emfa_amd", "csrc", "hip"), "-o", exe,
+                    str(tmp_path / "parts.cpp")], check=True)
+    r = subprocess.run([exe], stdout=subprocess.PIPE, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
 def _has_gpu():
     return os.path.exists("/dev/kfd")
 
