@@ -1128,12 +1128,14 @@ static emfa_status ml_translations(emfa_mlfma *M, MlLevel &C, int rows, const st
         all.insert(all.end(), c.begin(), c.end());
         ptr[i + 1] = (int)all.size();
     }
-    // one upload: offsets, coefficients, sample directions, row starts, rows
-    const size_t b0 = D.size() * sizeof(double), b1 = all.size() * sizeof(all[0]), b2 = C.kh.size() * sizeof(double),
+    // one upload, the 16-byte coefficients first (the base is aligned for them, an
+    // odd number of offsets is not a multiple of their size): coefficients, offsets,
+    // sample directions, row starts, rows
+    const size_t b0 = all.size() * sizeof(all[0]), b1 = D.size() * sizeof(double), b2 = C.kh.size() * sizeof(double),
                  b3 = ptr.size() * sizeof(int), b4 = row_of.size() * sizeof(int);
     std::vector<char> h(b0 + b1 + b2 + b3 + b4);
     char *p = h.data();
-    const void *src[5] = {D.data(), all.data(), C.kh.data(), ptr.data(), row_of.data()};
+    const void *src[5] = {all.data(), D.data(), C.kh.data(), ptr.data(), row_of.data()};
     const size_t len[5] = {b0, b1, b2, b3, b4};
     for (int i = 0; i < 5; ++i) {
         std::memcpy(p, src[i], len[i]);
@@ -1151,8 +1153,8 @@ static emfa_status ml_translations(emfa_mlfma *M, MlLevel &C, int rows, const st
         for (int i0 = 0; i0 < m; i0 += 65535) {
             const int mi = std::min(65535, m - i0);
             k_ml_trans<<<dim3((C.K + 255) / 256, mi), 256, 0, s>>>(
-                (const double *)d + 3 * (size_t)i0, (const int *)(d + b0 + b1 + b2 + b3) + i0,
-                (const int *)(d + b0 + b1 + b2) + i0, (const double2 *)(d + b0), (const double *)(d + b0 + b1), C.K,
+                (const double *)(d + b0) + 3 * (size_t)i0, (const int *)(d + b0 + b1 + b2 + b3) + i0,
+                (const int *)(d + b0 + b1 + b2) + i0, (const double2 *)d, (const double *)(d + b0 + b1), C.K,
                 C.trans);
         }
         e = hipGetLastError();
