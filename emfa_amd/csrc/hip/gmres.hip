@@ -25,15 +25,14 @@ namespace emfa {
 // A step's share of a solve in us, one row a wave and one vector at a time
 // against this, FP32: 12288 unknowns 341 and 243 for one vector, 681 and 256 for
 // two, 1286 and 316 for four; FP64 474 and 445, 945 and 470, 1786 and 468.
-// Unrolling by four gains 4 to 8 % at most sizes and loses 4 % at 4096 unknowns
-// in FP64, where the matrix just misses the last cache.
+// Loads are issued U trips together (the sums' order is the same).
 template <int NC>
 struct GemvCols {
     const double2 *x[NC];
     double2 *y[NC];
 };
 
-template <typename TA, int R, int NC>
+template <typename TA, int R, int NC, int U>
 __global__ __launch_bounds__(256) void k_gemv(const cx<TA> *__restrict__ Z, int n, GemvCols<NC> v) {
     const int row = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
     const int lane = threadIdx.x & 63;
@@ -46,7 +45,7 @@ __global__ __launch_bounds__(256) void k_gemv(const cx<TA> *__restrict__ Z, int 
 #pragma unroll
         for (int c = 0; c < NC; ++c) sr[i][c] = si[i][c] = 0;
     }
-#pragma unroll 4
+#pragma unroll U
     for (int j = lane; j < n; j += 64) {
         cx<TA> a[R];
         double2 b[NC];
@@ -321,6 +320,13 @@ emfa_status emfa::gemv(emfa_ctx *ctx, const emfa_mat *Z, int nc, const double2 *
     const int fit = n / ((nc == 1 ? 12 : 7) * std::max(1, ctx->num_cu));
     int r = 1;
     while (r < 4 && 2 * r <= fit && r * elem_bytes(Z->prec) < sizeof(double2) * nc) r *= 2;
+    // Four trips together, but one at a time for one FP64 vector on a matrix about
+    // as large as the last cache (256 MB), where fewer streams keep more of it
+    // there.  One / four trips, us per product and step: 3072 unknowns 66.6 / 65.9,
+    // 3584 73.5 / 74.1, 4096 83.4 / 86.5, 4608 103.1 / 104, 5120 116.4 / 117.7, 6144
+    // 151.7 / 148.2, 9216 324 / 284.  More vectors or FP32: four throughout.
+    const double mb = (double)n * n * elem_bytes(Z->prec) / 1e6;
+    const bool edge = nc == 1 && Z->prec == EMFA_F64 && mb > 200 && mb < 450;
     auto go = [&](auto cols) {
         constexpr int NC = decltype(cols)::value;
         GemvCols<NC> v;
@@ -331,10 +337,17 @@ emfa_status emfa::gemv(emfa_ctx *ctx, const emfa_mat *Z, int nc, const double2 *
         auto rows = [&](auto r) {
             constexpr int R = decltype(r)::value;
             const int g = (n + 4 * R - 1) / (4 * R);
-            if (Z->prec == EMFA_F32)
-                k_gemv<float, R, NC><<<g, 256, 0, s>>>((const cx<float> *)Z->d, n, v);
-            else
-                k_gemv<double, R, NC><<<g, 256, 0, s>>>((const cx<double> *)Z->d, n, v);
+            if (Z->prec == EMFA_F32) {
+                k_gemv<float, R, NC, 4><<<g, 256, 0, s>>>((const cx<float> *)Z->d, n, v);
+                return;
+            }
+            if constexpr (R == 1 && NC == 1) {
+                if (edge) {
+                    k_gemv<double, R, NC, 1><<<g, 256, 0, s>>>((const cx<double> *)Z->d, n, v);
+                    return;
+                }
+            }
+            k_gemv<double, R, NC, 4><<<g, 256, 0, s>>>((const cx<double> *)Z->d, n, v);
         };
         if (r == 4)
             rows(std::integral_constant<int, 4>{});
