@@ -64,7 +64,10 @@ extern "C" emfa_status emfa_refine(emfa_ctx *ctx, const emfa_mat *Z, const emfa_
         emfa_status s2 = colnorms(ctx, R, dn, rn);
         if (s2) return s2;
         mx = 0;
-        for (int j = 0; j < m; ++j) mx = std::max(mx, bn[j] > 0 ? rn[j] / bn[j] : rn[j]);
+        for (int j = 0; j < m; ++j) {  // a column that is not a number makes the report so
+            const double v = bn[j] > 0 ? rn[j] / bn[j] : rn[j];
+            if (v > mx || std::isnan(v)) mx = v;
+        }
         return EMFA_OK;
     };
     if (ctx_alloc(ctx, (void **)&dn, sizeof(double) * m) != hipSuccess) {
@@ -103,7 +106,7 @@ extern "C" emfa_status emfa_refine(emfa_ctx *ctx, const emfa_mat *Z, const emfa_
         rep->relres_final = r;
     }
     if (st) return st;
-    if (r > tol) {
+    if (!(r <= tol)) {
         set_error("emfa_refine: residual %.3e above tolerance %.3e after %d steps", r, tol, it);
         return EMFA_E_NOCONV;
     }

@@ -452,6 +452,21 @@ def test_lu_singular_reports(ctx):
     assert lu.singular and lu.info() == 18
 
 
+@pytest.mark.parametrize("value", [np.nan, 1e39])
+def test_refine_reports_solutions_that_are_not_numbers(ctx, value):
+    # 1e39 overflows in the FP32 factor's solve
+    _say(f"refine {value}")
+    A = np.eye(5) * (2 + 1j)
+    B = np.ones((5, 2), dtype=np.complex128)
+    B[3, 0] = value
+    Z, dB, X = hip.Mat.from_numpy(ctx, A, hip.F32), hip.Mat.from_numpy(ctx, B), hip.Mat(ctx, 5, 2)
+    lu = hip.LU(ctx, Z, hip.F32)
+    rep, ok = hip.refine(ctx, Z, lu, dB, X, 1e-12, 3)
+    assert not ok and np.isnan(rep.relres_final)
+    for x in (lu, Z, dB, X):
+        x.close()
+
+
 def test_refine_f32_to_f64(ctx):
     _say("refine")
     xyz, tri, rwg = sphere(2, 1.0)
