@@ -1362,7 +1362,14 @@ __global__ __launch_bounds__(256) void k_dinv_apply(const cx<R> *__restrict__ Di
 // Refined FP32 factorisations, ms with the GEMM / with the skinny products
 // above 64 columns: 1920 unknowns, 181 columns 4.99 / 4.28; 8321, 181 columns
 // 36.6 / 34.8; 14981, 100 columns 88.3 / 89.4; 30720, 181 columns 436 / 462.
-constexpr int kSkinnyCols = 64, kSkinnyMaxCols = 256, kSkinnyMaxN = 12288, kResidSkinnyCols = 128;
+// Single solves with 65 / 128 / 256 columns, ms GEMM and skinny: FP32 1920 0.61
+// 0.62 0.63 and 0.23 0.25 0.33, 12001 4.41 4.94 6.61 and 2.69 3.11 4.97; FP64 1920
+// 1.87 1.88 1.91 and 0.30 0.34 0.49, 12001 12.8 13.0 14.9 and 4.50 5.34 9.12.
+// Residuals with 65 / 97 / 128 columns: FP32 matrix 9600 2.65 2.84 2.85 and 1.55
+// 1.96 1.97, 12288 3.61 3.62 3.61 and 2.55 3.28 3.31; FP64 10400 2.89 3.06 3.06 and
+// 2.15 2.82 2.78, 11200 3.27 3.29 3.29 and 2.50 3.29 3.24, 12288 3.59 3.60 3.59 and
+// 2.94 3.82 3.78: past kResidF64MaxN a fourth column tile no longer pays.
+constexpr int kSkinnyCols = 64, kSkinnyMaxCols = 256, kSkinnyMaxN = 12288, kResidSkinnyCols = 128, kResidF64MaxN = 11264;
 
 // W = P B: row i of W is row perm[i] of B
 template <typename R>
@@ -1504,10 +1511,12 @@ static emfa_status lu_impl(emfa_ctx *ctx, emfa_mat *Am, int *ipiv, int *info_out
     if (const char *s = getenv("EMFA_PANEL_G")) G_max = std::max(1, std::min(G_max, atoi(s)));
     // at least 48 rows of a panel per workgroup: every workgroup polls every
     // other's packet, so fewer of them make a column's exchange shorter until the
-    // update of more rows takes longer.  16 / 32 / 48 / 64 / 96 rows, FP64: 1920
-    // unknowns 14.8 / 14.3 / 14.5 / 14.5 / 15.0 ms, 4256 37.8 / 36.0 / 35.8 / 35.7 /
-    // 37.1, 8321 98.4 / 95.0 / 94.5 / 92.6 / 100.1; FP32 with interchanges: 1920
-    // 11.6 / 11.1 / 11.1 / 11.1 / 11.5, 8321 70.2 / 68.2 / 67.1 / 66.5 / 67.3.
+    // update of more rows takes longer.  16 / 32 / 96 rows, FP64: 1920 unknowns 14.8
+    // / 14.3 / 15.0 ms, 4256 37.8 / 36.0 / 37.1, 8321 98.4 / 95.0 / 100.1; then 48 / 64
+    // / 80, in turn: 1920 14.30 / 14.30 / 14.79, 4256 35.21 / 35.31 / 36.41, 8321 93.1
+    // / 92.1 / 93.4; FP32 with interchanges 645 4.13 / 4.15 / 4.36, 1920 11.15 / 11.10
+    // / 11.52, 8321 68.0 / 67.4 / 68.6.  64 rows gain 1 % at 8321 unknowns and lose
+    // 0.3 to 0.5 % at 645 and 4256: 48, for the sizes that are served most.
     int panel_rows_min = 48;
     if (const char *s = getenv("EMFA_PANEL_ROWS_MIN")) panel_rows_min = std::max(1, atoi(s));
     // scratch: slots + Bt workspace
@@ -2030,12 +2039,14 @@ emfa_status gemm_residual(emfa_ctx *ctx, const emfa_mat *A, const emfa_mat *X, e
         return e ? e : getenv("EMFA_SKINNY_MAX");
     }();
     const int resid_skinny_max = resid_env           ? std::min(kSkinnyMaxCols, atoi(resid_env))
-                                 : N <= kSkinnyMaxN ? kResidSkinnyCols
+                                 : N <= kSkinnyMaxN ? (A->prec == EMFA_F64 && N > kResidF64MaxN ? 96 : kResidSkinnyCols)
                                                     : kSkinnyCols;
     if (m <= resid_skinny_max) {
-        // 16-row tiles x 64-column groups x K slices (summed in slice order);
-        // enough slices that the last round of workgroups is a small part (8321
-        // unknowns, 49 columns: four workgroups per CU 20.2 ms, sixteen 19.9)
+        // K slices, summed in slice order: enough that the last round of workgroups
+        // is a small part (8321 unknowns, 49 columns: four per CU 20.2 ms, sixteen
+        // 19.9).  Columns count in 64s whatever tile the launcher takes, so that a
+        // column's slices, and with them its bits, are the same in any block of up
+        // to 64.
         const long long wgs = (long long)((N + 15) / 16) * ((m + 63) / 64);
         int S = (int)std::min<long long>(32, std::max<long long>(1, (16LL * ctx->num_cu + wgs - 1) / wgs));
         if (const char *e = getenv("EMFA_RESID_SPLIT")) S = std::max(1, std::min(64, atoi(e)));
