@@ -1,6 +1,6 @@
 // Device helpers shared by the dense fill and the MLFMA near field:
 // triangle quadrature rules, small vector algebra, the analytic potentials
-// of a triangle and the FP64 self terms.
+// of a triangle and the FP64 self terms of the near field.
 #pragma once
 #include <cmath>
 
@@ -26,9 +26,6 @@ template <int Q>
 __device__ __forceinline__ double rule(int p, int i) {
     return Q == 7 ? c_rule7[p][i] : c_rule3[p][i];
 }
-
-__device__ __forceinline__ void sincos_r(float x, float *s, float *c) { sincosf(x, s, c); }
-__device__ __forceinline__ void sincos_r(double x, double *s, double *c) { sincos(x, s, c); }
 
 template <typename R>
 __device__ __forceinline__ R dot3(const R *a, const R *b) {
@@ -158,9 +155,11 @@ __device__ inline void potentials(const d3 *t, d3 r, d3 *Is1, double *Is2) {
     *Is2 = s2;
 }
 
-template <int Q>
-__device__ void self_term(int kind, double k, double alpha, double sig_re, double sig_im, int cfie_mode, const d3 *t,
-                          double area, int a, int b, double *zr, double *zi, double *gr, double *gi) {
+// Self term (a, b) of a triangle, 3-point rule, without a surface impedance (the
+// dense fill has its own form for both rules and the impedance).
+__device__ inline void self_term(int kind, double k, double alpha, int cfie_mode, const d3 *t, double area, int a,
+                                 int b, double *zr, double *zi) {
+    constexpr int Q = 3;
     d3 pts[Q];
     double w[Q];
     for (int p = 0; p < Q; ++p) {
@@ -213,19 +212,10 @@ __device__ void self_term(int kind, double k, double alpha, double sig_re, doubl
     if (kind == EMFA_EFIE) {
         *zr = er;
         *zi = ei;
-        // Sigma term (EFIE.cpp:297-306): pi sigma / (S j k Z0) * sum w (r-vf).(r-vs),
-        // times coefE later in the gather via the caller's scale: coefE * pi/(S j k Z0) = 1/(4 S)
-        double acc = 0;
-        for (int i = 0; i < Q; ++i) acc += w[i] * dotd(pts[i] - vf, pts[i] - vs);
-        double f = acc / (4.0 * area);
-        *gr = f * sig_re;
-        *gi = f * sig_im;
     } else {
         // alpha * Ze + (1 - alpha) * Z0 * Zm / (8 area)
         *zr = alpha * er + (1.0 - alpha) * kZ0 * zmr / (8.0 * area);
         *zi = alpha * ei;
-        *gr = 0;
-        *gi = 0;
     }
 }
 

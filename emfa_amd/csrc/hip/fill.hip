@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256) void k_fill_pairs(const R *__restrict__ tg, in
 }
 
 // ---------------------------------------------------------------------------
-// K2: self terms in FP64 (the formulas of self_term in em_device.h), one lane
+// K2: self terms in FP64 (EFIE.cpp:231-542, Miscellaneous.cpp:32-77), one lane
 // per triangle and point p: a group of G lanes forms the nine (a, b) values of
 // a triangle, point by point, and adds them over its lanes.  All triangles in
 // one launch: it is a chain of logarithms and divisions, 18 us whatever the

@@ -249,7 +249,7 @@ __device__ cf pair_regular(const float *__restrict__ tg, int T, int tf, int a, i
             float r = sqrtf(dot3(u, u));
             float ir = 1.0f / r;
             float sn, cs;
-            sincos_r(k * r, &sn, &cs);
+            sincosf(k * r, &sn, &cs);
             const float w = (1.0f / 9.0f);
             float gr = w * cs * ir, gi = -w * sn * ir;
             float f = 0.25f * dot3(rf, rs) - ik2;
@@ -296,9 +296,8 @@ __global__ __launch_bounds__(256) void k_ml_near_fill(const float *__restrict__ 
                     for (int v = 0; v < 3; ++v)
                         t[v] = mk3(tg64[(size_t)(3 + 3 * v) * T + tf], tg64[(size_t)(4 + 3 * v) * T + tf],
                                    tg64[(size_t)(5 + 3 * v) * T + tf]);
-                    double sr, si, gr, gi;
-                    self_term<3>(KIND, kd, alpha, 0.0, 0.0, cfie_mode, t, tg64[(size_t)15 * T + tf], afs[i], bss[q],
-                                 &sr, &si, &gr, &gi);
+                    double sr, si;
+                    self_term(KIND, kd, alpha, cfie_mode, t, tg64[(size_t)15 * T + tf], afs[i], bss[q], &sr, &si);
                     zr += sg * (float)sr;
                     zi += sg * (float)si;
                 } else {
@@ -828,7 +827,7 @@ __device__ cf wt_line(const float *__restrict__ tg, int T, int tt, int ts, int b
                        ep[c];
             const float r = sqrtf(dot3(u, u)), ir = 1.0f / r;
             float sn, cs_;
-            sincos_r(k * r, &sn, &cs_);
+            sincosf(k * r, &sn, &cs_);
             ar += wp * cs_ * ir;
             ai -= wp * sn * ir;
         }
@@ -869,9 +868,8 @@ __global__ __launch_bounds__(256) void k_wt_near_fill(
             for (int v = 0; v < 3; ++v)
                 t[v] = mk3(tg64[(size_t)(3 + 3 * v) * T + tf], tg64[(size_t)(4 + 3 * v) * T + tf],
                            tg64[(size_t)(5 + 3 * v) * T + tf]);
-            double sr, si, gr, gi;
-            self_term<3>(KIND, kd, alpha, 0.0, 0.0, cfie_mode, t, tg64[(size_t)15 * T + tf], af, as, &sr, &si, &gr,
-                         &gi);
+            double sr, si;
+            self_term(KIND, kd, alpha, cfie_mode, t, tg64[(size_t)15 * T + tf], af, as, &sr, &si);
             zr = (float)sr;
             zi = (float)si;
             if (f == s) ip = stab * lf;
