@@ -855,7 +855,8 @@ emfa_status gemm_launch_bf3_planes(hipStream_t s, const Bf3Planes &g) {
     // 256 x 256 tiles (reals) move the fewest operand bytes, 128 x 128 ones fill
     // the chip from a quarter of the size on and come two to a CU, so that one's
     // C and first loads hide behind the other's products.  The line is at 1.5
-    // large tiles a CU: 1920 unknowns (at most 49) 2.26 ms a factorisation with
+    // large tiles a CU of 256 (also where max_wgs caps a context's workgroups; its
+    // cap counts twice for the small tiles): 1920 unknowns (at most 49) 2.26 ms a factorisation with
     // large tiles and 2.13 with small ones, 8321 (1024 at first, 400 half way)
     // 18.84 and 18.92, 18.68 with this line; 30720 372 and 399.
     const long long large = (long long)((g.Nr + 255) / 256) * ((g.M + 255) / 256) * g.bt.count;

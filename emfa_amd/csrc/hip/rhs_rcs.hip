@@ -27,10 +27,11 @@ __device__ __forceinline__ void load_tri(const double *__restrict__ tg, int T, i
 // MFIE (kind 2): 7-point rule, n x h part only (EMSolver/MFIE.cpp:289-322,
 // 435-436 without its 1/Z0, matching the Z0-scaled MFIE operator of the fill).
 //
-// Few values: one thread per (u, j), j fastest so the row-major writes coalesce.
-// A launch's latency either way (122880 x 1 columns 15 us, 10 as k_rhs with one
-// column per thread); it keeps the library's sincos and absolute points, and so
-// the bits that an iterative solver's step count can hang on.
+// Up to 2048 values per CU (524288 on 256 CUs: 8321 x 49 still): one thread per
+// (u, j), j fastest so the row-major writes coalesce.  A launch's latency mostly
+// (122880 x 1 columns 15 us, 10 as k_rhs with one column per thread); it keeps the
+// library's sincos and absolute points, and so the bits that an iterative solver's
+// step count can hang on.  A column's last bits differ from k_rhs's.
 template <typename R>
 __global__ __launch_bounds__(256) void k_rhs_few(const double *__restrict__ tg, const int *__restrict__ rtp,
                                              const int *__restrict__ rtm, const int *__restrict__ rap,

@@ -11,8 +11,9 @@
 // complex product is a real one with X's columns expanded in registers: real
 // column 2j + p takes (p ? Im : Re) against Re A and (p ? Re : -Im) against
 // Im A.  Partial tiles are added through LDS in wave order.  An entry's sum
-// depends on K and the slice only, never on m or CT, so a column has the same
-// bits in any block of right-hand sides.  A second job shares the launch
+// depends on K and the slice only, never on m or the tile, so a column has the
+// same bits in every block of right-hand sides that takes this route with the
+// same slices (a residual's are the same up to 64 columns).  A second job shares the launch
 // (workgroups from tiles0 on) when it writes other rows and reads nothing
 // that the first one writes.
 //
@@ -168,9 +169,10 @@ emfa_status launch(hipStream_t s, const SkinnyJob<TA, TC> &j0, const SkinnyJob<T
         return (long long)((j0.M + 16 * rt - 1) / (16 * rt) + (j1.M + 16 * rt - 1) / (16 * rt)) *
                ((m + 8 * ct - 1) / (8 * ct)) * slices;
     };
-    // The widest column tile that gives every CU a workgroup (A is read once
-    // per column group), then two row tiles where that leaves two per CU (X is
-    // read half as often).  Refined factorisation of 8321 unknowns, 49 columns:
+    // The widest column tile that gives each of 256 CUs a workgroup (A is read
+    // once per column group), then two row tiles where that leaves two per CU (X
+    // is read half as often).  Counted on the whole chip also for a context with a
+    // share of it: its products run in what the others leave.  Refined factorisation of 8321 unknowns, 49 columns:
     // 20.2 ms with one row tile, 19.5 with two, 21.4 with four; 64 columns per
     // tile instead of 32: 20.7.
     int ct = 1;

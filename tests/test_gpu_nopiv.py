@@ -176,3 +176,29 @@ def test_runs_of_large_multipliers_refine(ctx, n, t, run):
     assert ok
     for x in (lu, Z, dB, X):
         x.close()
+
+
+@pytest.mark.parametrize("n,nb", [(700, 300), (1100, 448)])
+def test_ragged_outer_blocks_in_a_graph_match_eager_launches(n, nb):
+    ctxs = [hip.Context(0) for _ in range(2)]
+    for c in ctxs:
+        c.lu_params(nb, 0, 2)
+        c.lu_update_mode(1)
+    ctxs[0].graphs(True)
+    for seed in range(4):
+        A = _matrix(n, seed)
+        F = []
+        for c in ctxs:
+            Z = hip.Mat.from_numpy(c, A, hip.F32)
+            lu = hip.LU(c, Z, hip.F32)
+            assert lu.pivoting() == (0, 0)
+            F.append(lu.factor().numpy())
+            lu.close()
+            Z.close()
+        assert np.array_equal(F[0], F[1])
+    assert ctxs[0].graph_stats() == (1, 4)
+    L, U = np.tril(F[0], -1) + np.eye(n), np.triu(F[0])
+    tol = (6 * 2.0 ** -18 + 4 * n ** 0.5 * 2.0 ** -23) * (np.abs(L) @ np.abs(U))
+    assert (np.abs(L @ U - A) <= tol).all()
+    for c in ctxs:
+        c.close()

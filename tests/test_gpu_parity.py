@@ -390,9 +390,11 @@ def test_inverse_block_solve_matches_blocked_substitution(ctx, monkeypatch, prec
 
 @pytest.mark.parametrize("n,m", [(1100, 65), (2600, 181)])
 def test_mfma_block_apply_matches_valu_apply(ctx, monkeypatch, n, m):
-    # more than 64 FP32 right-hand sides: the diagonal-block applies run as
-    # MFMA products of the expanded blocks; k_dinv_apply (EMFA_APPLY_MFMA=0)
-    # gives the same solution to FP32 accuracy on the same factor
+    # more than 64 FP32 right-hand sides on the expanded-operand route (here below
+    # the size where it is the default): the diagonal-block applies run as MFMA
+    # products of the expanded blocks; k_dinv_apply (EMFA_APPLY_MFMA=0) gives the
+    # same solution to FP32 accuracy on the same factor
+    monkeypatch.setenv("EMFA_SKINNY_MAX", "64")
     _say(f"mfma block apply n={n} m={m}")
     rng = np.random.default_rng(n + 7 * m)
     A = rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n)) + 4 * np.sqrt(n) * np.eye(n)
@@ -412,9 +414,9 @@ def test_mfma_block_apply_matches_valu_apply(ctx, monkeypatch, n, m):
 
 @pytest.mark.parametrize("m", [40, 64, 20])
 def test_shared_context_solve_matches_skinny_products(monkeypatch, m):
-    # a context with a CU share (as the solve server's workers) solves 32-64
-    # columns with the expanded-operand MFMA GEMM instead of k_smallmm; 20
-    # columns stay on k_smallmm.  Same factor, same answer to FP32 accuracy.
+    # a context with a CU share (as the solve server's workers) solves few columns
+    # with the skinny products; the expanded-operand MFMA GEMM on the same factor
+    # gives the same answer to FP32 accuracy
     _say(f"shared-context solve m={m}")
     n = 2600
     rng = np.random.default_rng(77 + m)
@@ -429,7 +431,7 @@ def test_shared_context_solve_matches_skinny_products(monkeypatch, m):
         d1 = hip.Mat.from_numpy(c, B, hip.F32)
         mats += [Z, lu, d1]
         lu.solve(d1)
-        monkeypatch.setenv("EMFA_SKINNY_MAX", "64")
+        monkeypatch.setenv("EMFA_SKINNY_MAX", "0")
         d0 = hip.Mat.from_numpy(c, B, hip.F32)
         mats.append(d0)
         lu.solve(d0)
