@@ -170,8 +170,9 @@ __device__ __forceinline__ void inv8(Tri64 &T, const cf *dinv, int lane) {
 // 32 x 32 quadrant of X across the diagonal, which the caller ignores; the
 // rest of X across the diagonal must be zero.  One rolled loop: the kernel
 // runs once per launch, and every 64 bytes of code are a cold fetch.
-// tris: 3 both, 1 L only, 2 U only.  All waves call it (it synchronises).
-__device__ __forceinline__ void join64(Tri64 &T, int tris, int wave, int lane) {
+// tris: 3 both, 1 L only, 2 U only; L's inverse as far as blocks of lmax.  All
+// waves call it (it synchronises).
+__device__ __forceinline__ void join64(Tri64 &T, int tris, int lmax, int wave, int lane) {
     cf *M = &T.m[0][0][0];
     const int l16 = lane & 15, g = lane >> 4;
     const bool odd = l16 & 1;
@@ -182,7 +183,7 @@ __device__ __forceinline__ void join64(Tri64 &T, int tris, int wave, int lane) {
         const int p = lb == 3 ? j : lb == 4 ? j >> 1 : 0;  // pair
         const int r = lb == 5 ? 16 * (j >> 2) : 0, c = lb == 3 ? 0 : 8 * (lb == 4 ? j & 1 : j & 3);
         const int s0 = 2 * b * p, s1 = s0 + b, m = 32 + b * p;
-        const bool act = (wave >> lt) < 2 && ((tris >> up) & 1);
+        const bool act = (wave >> lt) < 2 && ((tris >> up) & 1) && (up || 2 * b <= lmax);
         cf *X = M + (up ? 2 : 1) * kMat;
         // the middle factor, then the block: offsets of A's rows, B's rows and the result
 #pragma nounroll
@@ -351,7 +352,7 @@ __global__ __launch_bounds__(kDiagThreads) void k_nopiv_diag(cf *__restrict__ A,
         }
     }
     __syncthreads();
-    join64(T, 3, v, lane);
+    join64(T, 3, 16, v, lane);
     for (int r = v; r < 64; r += 16) {
         uinv[(size_t)r * kNoPivW + lane] = lane >= r ? T.m[2][r][lane] : cf{0.f, 0.f};
         linv[(size_t)r * kNoPivW + lane] = lane < r ? T.m[1][r][lane] : cf{0.f, 0.f};
@@ -360,19 +361,19 @@ __global__ __launch_bounds__(kDiagThreads) void k_nopiv_diag(cf *__restrict__ A,
 }
 
 // ---------------------------------------------------------------------------
-// What follows the diagonal block, in one launch: workgroups [0, nl) form 16 rows
-// of L21 = A21 U^-1 (a wave two of the eight column tiles, K = 64: 64 MFMAs
-// behind one round of loads), the others 32 columns of U12 by substitution with
-// L (a wave 8 columns).  In place: a workgroup's (U12: a wave's) loads are done
-// before its first store, and they touch disjoint parts of A.  8.1 us per launch
-// at 1920 unknowns (6.4 with U12 = L^-1 A12 by an explicit inverse, 17 as a VALU
-// product and substitution through LDS).
+// What follows the diagonal block, in one launch: workgroups [0, nu), whose chain
+// is the longer one, form 32 columns of U12 by substitution with L (a wave 8
+// columns), the others 16 rows of L21 = A21 U^-1 (a wave two of the eight column
+// tiles, K = 64: 64 MFMAs behind one round of loads).  In place: a workgroup's
+// (U12: a wave's) loads are done before its first store, and they touch disjoint
+// parts of A.  8.0 us per launch at 1920 unknowns (6.4 with U12 = L^-1 A12 by an
+// explicit inverse, 17 as a VALU product and substitution through LDS).
 // ---------------------------------------------------------------------------
 constexpr int kSubLd = 10;  // sixteen lanes' rows four apart on different banks
 
 __global__ __launch_bounds__(256) void k_nopiv_rows(cf *__restrict__ A, long long lda, int js, int w, int N,
                                                     const cf *__restrict__ uinv, const cf *__restrict__ linv,
-                                                    int *flags, float tau2, int nl, int c0, int c1,
+                                                    int *flags, float tau2, int nu, int c0, int c1,
                                                     float *__restrict__ Bt, long long ldbt, Batch bt) {
     __shared__ cf Xs[4][64 * kSubLd];
     A = batch_mat(bt, A);
@@ -382,8 +383,8 @@ __global__ __launch_bounds__(256) void k_nopiv_rows(cf *__restrict__ A, long lon
     Bt = batch_scr(bt, Bt);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
     const bool odd = l16 & 1;
-    if ((int)blockIdx.x >= nl) {
-        const int cb = c0 + 32 * ((int)blockIdx.x - nl) + 8 * wave, j = cb + (l16 >> 1);
+    if ((int)blockIdx.x < nu) {
+        const int cb = c0 + 32 * (int)blockIdx.x + 8 * wave, j = cb + (l16 >> 1);
         if (cb >= c1) return;
         Sub64 op;
         op.load(A + (size_t)js * lda + js, lda, linv, w, lane);
@@ -411,7 +412,7 @@ __global__ __launch_bounds__(256) void k_nopiv_rows(cf *__restrict__ A, long lon
             }
         return;
     }
-    const int r0 = js + w + 16 * (int)blockIdx.x;
+    const int r0 = js + w + 16 * ((int)blockIdx.x - nu);
     const cf *Ar = A + (size_t)min(r0 + l16, N - 1) * lda + js;
     f4 a[8];
     if (w == 64) {
@@ -490,7 +491,7 @@ __global__ __launch_bounds__(kDiagThreads) void k_inv_diag(const cf *__restrict_
             inv8<false>(T, dinv, lane);
     }
     __syncthreads();
-    join64(T, up ? 2 : 1, v, lane);
+    join64(T, up ? 2 : 1, 64, v, lane);
     cf *X = Dinv + (up ? (size_t)nblk * kInvB * kInvB : 0) + (size_t)blk * kInvB * kInvB + (size_t)64 * i * kInvB;
     for (int r = v; r < 64; r += 16) {
         X[(size_t)r * kInvB + 64 * i + lane] =
@@ -579,16 +580,21 @@ __global__ __launch_bounds__(256) void k_inv_join(const cf *__restrict__ F, long
 // workgroup, in place (the columns in LDS): per 64 rows a wave and column tile
 // substitutes (Sub64) while the other waves take the last 64 rows' part off the
 // tiles below.  Wave v owns the 16-row tiles v and 15 - v, so the triangle's
-// work is even.  L's tiles and the substitution's operands are loaded a block ahead.
+// work is even.
 // A chain of four substitutions: 21 us per launch at 1920 unknowns, where the
 // product with L's explicit inverse took 15 and that inverse 20 more per block,
-// and blocked substitution in launches of 64 rows 176 us per 512 rows.
+// and blocked substitution in launches of 64 rows 176 us per 512 rows.  Strips of
+// up to 16 columns run in one round, one workgroup a CU: L's tiles and the
+// substitution's operands are loaded a block ahead.  Strips of 32, in several
+// rounds, take half the registers instead and come two to a CU: 30720 unknowns 121
+// -> 105 us per launch, 8321 44 -> 48.
 // ---------------------------------------------------------------------------
 template <int CT>
-__global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long long lda, int r0, int wb, int c0,
+__global__ __launch_bounds__(512, CT == 4 ? 4 : 2) void k_nopiv_urows(cf *__restrict__ A, long long lda, int r0, int wb, int c0,
                                                      int c1, const cf *__restrict__ linv, float *__restrict__ Bt,
                                                      long long ldbt, int kofs, Batch bt) {
     constexpr int S = 8 * CT, LD = S + 2;
+    constexpr bool kAhead = CT < 4;
     __shared__ cf Xs[kURows * LD];
     A = batch_mat(bt, A);
     linv = batch_scr(bt, linv);
@@ -600,13 +606,13 @@ __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long lo
     const cf *L = A + (size_t)r0 * lda + r0;
     const int tile[2] = {wave, 15 - wave}, solver = wave - (8 - CT);  // column tile that the wave substitutes
     const int nst = (wb + 63) / 64;
-    f4 l[2][8];
+    f4 l[kAhead ? 2 : 1][8];
     Sub64 op;
     // L's tile in block column s
     auto load_l = [&](int h, int s) {
         const cf *Lr = L + (size_t)min(16 * tile[h] + l16, wb - 1) * lda + 64 * s + 2 * g;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) l[h][q] = *(const f4_a8 *)(Lr + 8 * q);
+        for (int q = 0; q < 8; ++q) l[kAhead ? h : 0][q] = *(const f4_a8 *)(Lr + 8 * q);
     };
     auto load_op = [&](int s) {
         op.load(L + (size_t)64 * s * lda + 64 * s, lda, linv + (size_t)s * kNoPivW * kNoPivW,
@@ -615,16 +621,17 @@ __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long lo
     // the tile's columns less L's tile times the rows of block s
     auto update = [&](int h, int s) {
         const cf *X = Xs + (64 * s + 2 * g) * LD + (l16 >> 1);
+        if (!kAhead) load_l(h, s);
 #pragma unroll
         for (int t = 0; t < CT; ++t) {
             f4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int q = 0; q < 8; ++q) mac2(p, l[h][q], X[8 * q * LD + 8 * t], X[(8 * q + 1) * LD + 8 * t], odd);
+            for (int q = 0; q < 8; ++q) mac2(p, l[kAhead ? h : 0][q], X[8 * q * LD + 8 * t], X[(8 * q + 1) * LD + 8 * t], odd);
 #pragma unroll
             for (int i = 0; i < 4; ++i) ((float *)(Xs + (16 * tile[h] + 4 * g + i) * LD + 8 * t))[l16] -= p[i];
         }
     };
-    if (solver >= 0) load_op(0);
+    if (kAhead && solver >= 0) load_op(0);
     {
         cf x[kURows * S / 512];
 #pragma unroll
@@ -640,7 +647,7 @@ __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long lo
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-        if (tile[h] >= 4 && 16 * tile[h] < wb) load_l(h, 0);
+        if (kAhead && tile[h] >= 4 && 16 * tile[h] < wb) load_l(h, 0);
     __syncthreads();
     for (int s = 0; s < nst; ++s) {
         if (s) {
@@ -650,6 +657,7 @@ __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long lo
             __syncthreads();
         }
         if (solver >= 0) {
+            if (!kAhead) load_op(s);
             cf *X = Xs + 64 * s * LD + 8 * solver;
             f4 v[4];
 #pragma unroll
@@ -657,7 +665,7 @@ __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long lo
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[i][r] = ((const float *)(X + (16 * i + 4 * g + r) * LD))[l16];
             op.solve(v, X, LD, lane);
-            if (s + 1 < nst) load_op(s + 1);
+            if (kAhead && s + 1 < nst) load_op(s + 1);
         }
         // beside it, the tiles of later blocks
         if (s) {
@@ -665,7 +673,7 @@ __global__ __launch_bounds__(512) void k_nopiv_urows(cf *__restrict__ A, long lo
             for (int h = 0; h < 2; ++h)
                 if (tile[h] >> 2 > s && 16 * tile[h] < wb) {
                     update(h, s - 1);
-                    load_l(h, s);
+                    if (kAhead) load_l(h, s);
                 }
         }
         __syncthreads();
@@ -699,7 +707,7 @@ emfa_status nopiv_rows_launch(hipStream_t s, cf *A, long long lda, int js, int w
                               const Batch &bt) {
     const int nl = (N - js - w + 15) / 16, nu = std::max(0, (c1 - c0 + 31) / 32);
     if (nl + nu <= 0) return EMFA_OK;
-    k_nopiv_rows<<<dim3(nl + nu, 1, bt.count), 256, 0, s>>>(A, lda, js, w, N, uinv, linv, flags, tau2, nl, c0, c1, Bt,
+    k_nopiv_rows<<<dim3(nl + nu, 1, bt.count), 256, 0, s>>>(A, lda, js, w, N, uinv, linv, flags, tau2, nu, c0, c1, Bt,
                                                             ldbt, bt);
     EMFA_HIP_CHECK(hipGetLastError());
     return EMFA_OK;
