@@ -718,9 +718,9 @@ emfa_status nopiv_urows_launch(hipStream_t s, cf *A, long long lda, int r0, int 
     if (c1 <= c0 || wb <= 0) return EMFA_OK;
     EMFA_REQUIRE(wb <= kURows, EMFA_E_INVALID, "U rows of a block of %d", wb);
     const int nc = c1 - c0;
-    // A strip's time is its chain's (8, 16, 32 columns 21, 29, 42 us alone), and a
-    // CU holds one workgroup: the narrowest strips that run in one round.  In
-    // factorisations of 1920 / 8321 / 30720 unknowns all strips of 8 columns take
+    // A strip's time is its chain's (8, 16, 32 columns 21, 29, 48 us alone), and a
+    // CU holds one workgroup (two of the widest): the narrowest strips that run in
+    // one round.  In factorisations of 1920 / 8321 / 30720 unknowns all strips of 8 columns take
     // 2.20 / 19.2 / 388 ms, of 16 2.26 / 19.0 / 382, of 32 2.28 / 18.9 / 381.
     const long long cols = (long long)nc * bt.count;
     auto go = [&](auto kernel, int strip) {

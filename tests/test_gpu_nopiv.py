@@ -202,3 +202,27 @@ def test_ragged_outer_blocks_in_a_graph_match_eager_launches(n, nb):
     assert (np.abs(L @ U - A) <= tol).all()
     for c in ctxs:
         c.close()
+
+
+# U rows in strips of 8, 16 and 32 columns: the CUs to fill decide, an entry's
+# sums do not depend on it; ragged blocks of rows and ragged last strips
+@pytest.mark.parametrize("n,nb", [(301, 64), (523, 100), (700, 300), (777, 512)])
+def test_strips_of_every_width_give_the_same_factor(n, nb):
+    A = _matrix(n, nb)
+    F = []
+    for share in (0, (n - nb) // 12, 2):  # one round of 8, of 16, none
+        c = hip.Context(0)
+        c.lu_params(nb, 0, 2)
+        if share:
+            c.set_cu_share(share)
+        Z = hip.Mat.from_numpy(c, A, hip.F32)
+        lu = hip.LU(c, Z, hip.F32)
+        assert lu.pivoting() == (0, 0)
+        F.append(lu.factor().numpy())
+        lu.close()
+        Z.close()
+        c.close()
+    ref = _lu(A)
+    tol = 8 * np.sqrt(n) * 2.0 ** -23 * np.abs(ref).max() + 1e-6
+    assert np.abs(F[0] - ref).max() <= tol
+    assert np.array_equal(F[0], F[1]) and np.array_equal(F[0], F[2])
